@@ -688,8 +688,10 @@ struct hm_plan {
 
     // The nested far field's tables from the builder's interval trees; nest
     // stays false (the per-level far field is used) unless every half is
-    // exactly half of its parent's interval (to 1e-12), every column leaf
-    // fits one upward task and every row chunk lies in one row leaf.
+    // half of its parent's interval to the rounding of the interval ends,
+    // every column leaf fits one upward task and every row chunk lies in one
+    // row leaf. (To a fixed 1e-12, the log kernel's 2^22 random points fell
+    // back to the per-level form by their deepest intervals' rounding.)
     template <class TN>
     void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt, bool tok) {
         nest = false;
@@ -716,8 +718,13 @@ struct hm_plan {
                 if (d.parent < 0) continue;
                 const DTNode &P = o[d.parent];
                 const double alpha = P.cy / d.cy, beta = (d.cx - P.cx) * P.cy;
-                if (!(std::fabs(alpha - 0.5) <= 1e-12) ||
-                    !(std::fabs(beta - (d.half ? 0.5 : -0.5)) <= 1e-12))
+                // interval ends and centers are rounded to eps |end|, which
+                // is eps |end| / halfwidth in the node's variable (7e-12 at
+                // depth 14 of [0, 1]; the mapped nodes behind F carry the same)
+                const double end = std::max(std::fabs(t[k].lo), std::fabs(t[k].hi));
+                const double tol = std::max(1e-12, std::min(1e-10, 4.0 * 0x1p-52 * end * std::fabs(d.cy)));
+                if (!(std::fabs(alpha - 0.5) <= tol) ||
+                    !(std::fabs(beta - (d.half ? 0.5 : -0.5)) <= tol))
                     return false;
             }
             return true;
