@@ -121,9 +121,11 @@ hipError_t hmx_launch_grad(const DevPlan &p, const MvArgs &a, bool transpose, do
 // entries: kind[t] = 0 none, 1 dense (id), 2 far (id); rows/cols 0-based
 hipError_t hmx_launch_entries(const DevPlan &p, int64_t n, const int64_t *i, const int64_t *j,
                               const int32_t *kind, const int32_t *id, double *out, hipStream_t s);
-// number of non-finite values among generated factors (after compression)
-hipError_t hmx_launch_count_nonfinite(const double *v, int64_t n, unsigned long long *count,
-                                      hipStream_t s);
+// non-finite values of the generated factors (after compression): the arrays
+// v[q] of n[q] values, HM_COUNT_BLOCKS partial counts each
+#define HM_COUNT_BLOCKS 256
+hipError_t hmx_launch_count_nonfinite(const double *const v[4], const int64_t n[4],
+                                      unsigned long long *count, hipStream_t s);
 
 // in-place diagonal scaling of stored dense blocks and bases (plans built
 // from blocks): side 0 scales columns (A and V rows), 1 rows (A and U rows);
@@ -166,5 +168,5 @@ hipError_t hmx_launch_grad(const DevPlanF &p, const MvArgsF &a, bool transpose, 
                            int64_t incy2, const float *s, int64_t incs, hipStream_t stream);
 hipError_t hmx_launch_entries(const DevPlanF &p, int64_t n, const int64_t *i, const int64_t *j,
                               const int32_t *kind, const int32_t *id, float *out, hipStream_t s);
-hipError_t hmx_launch_count_nonfinite(const float *v, int64_t n, unsigned long long *count,
-                                      hipStream_t s);
+hipError_t hmx_launch_count_nonfinite(const float *const v[4], const int64_t n[4],
+                                      unsigned long long *count, hipStream_t s);

@@ -9,6 +9,8 @@ hipError_t hmx_launch_compress(const DevPlan &p, hipStream_t s) {
     const bool gen = p.kid != HM_USER;
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<double><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<double><<<p.nfar, hmxk::WG, 0, s>>>(p);
+    if (p.U && p.V && p.nrc + p.ncc > 0)
+        hmxk::k_pad_basis<double><<<p.nrc + p.ncc, hmxk::WAVE, 0, s>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || (!p.U && !p.V)) return err;
     if (p.r <= 8) return hmx_gen_basis_r8(p, s);
@@ -47,13 +49,14 @@ hipError_t hmx_launch_entries(const DevPlan &p, int64_t n, const int64_t *i, con
     return hipGetLastError();
 }
 
-hipError_t hmx_launch_count_nonfinite(const double *v, int64_t n, unsigned long long *blockcount,
-                                      hipStream_t s) {
-    // caller provides 1024 slots
-    if (n <= 0) return hipSuccess;
-    int64_t nb = (n + hmxk::WG - 1) / hmxk::WG;
-    if (nb > 1024) nb = 1024;
-    hmxk::k_count_nonfinite<double><<<(int)nb, hmxk::WG, 0, s>>>(v, n, blockcount);
+hipError_t hmx_launch_count_nonfinite(const double *const v[4], const int64_t n[4],
+                                      unsigned long long *blockcount, hipStream_t s) {
+    hmxk::CountArgs<double> a;
+    for (int q = 0; q < 4; ++q) {
+        a.v[q] = v[q];
+        a.n[q] = v[q] ? n[q] : 0;
+    }
+    hmxk::k_count_nonfinite<double><<<dim3(HM_COUNT_BLOCKS, 4), hmxk::WG, 0, s>>>(a, blockcount);
     return hipGetLastError();
 }
 
@@ -73,6 +76,8 @@ hipError_t hmx_launch_compress(const DevPlanF &p, hipStream_t s) {
     const bool gen = p.kid != HM_USER;
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<float><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<float><<<p.nfar, hmxk::WG, 0, s>>>(p);
+    if (p.U && p.V && p.nrc + p.ncc > 0)
+        hmxk::k_pad_basis<float><<<p.nrc + p.ncc, hmxk::WAVE, 0, s>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || (!p.U && !p.V)) return err;
     if (p.r <= 8) return hmx_gen_basis_f32_r8(p, s);
@@ -104,12 +109,14 @@ hipError_t hmx_launch_entries(const DevPlanF &p, int64_t n, const int64_t *i, co
     return hipGetLastError();
 }
 
-hipError_t hmx_launch_count_nonfinite(const float *v, int64_t n, unsigned long long *blockcount,
-                                      hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    int64_t nb = (n + hmxk::WG - 1) / hmxk::WG;
-    if (nb > 1024) nb = 1024;
-    hmxk::k_count_nonfinite<float><<<(int)nb, hmxk::WG, 0, s>>>(v, n, blockcount);
+hipError_t hmx_launch_count_nonfinite(const float *const v[4], const int64_t n[4],
+                                      unsigned long long *blockcount, hipStream_t s) {
+    hmxk::CountArgs<float> a;
+    for (int q = 0; q < 4; ++q) {
+        a.v[q] = v[q];
+        a.n[q] = v[q] ? n[q] : 0;
+    }
+    hmxk::k_count_nonfinite<float><<<dim3(HM_COUNT_BLOCKS, 4), hmxk::WG, 0, s>>>(a, blockcount);
     return hipGetLastError();
 }
 

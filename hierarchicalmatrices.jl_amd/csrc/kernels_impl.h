@@ -216,14 +216,36 @@ struct HalveShape<P, 0, OMIN> {
 
 // ------------------------------------------------------------- compression
 
+// One dense block per workgroup, tile by tile: a wavefront writes a column's 64
+// rows of a tile (one contiguous run), the rows past the block's last as
+// zeros, so the padding needs no pass of its own (every array was cleared
+// whole before; n = 10000: four launches, 37 us).
 template <class T>
 __global__ __launch_bounds__(WG) void k_gen_dense(DevPlanT<T> p) {
     const DDense D = p.dense[blockIdx.x];
-    const int32_t tot = D.m * D.n;
-    for (int32_t e = threadIdx.x; e < tot; e += WG) {
-        int32_t j = e / D.m, i = e - j * D.m;
-        p.A[D.aoff + tile_index(i, j, D.n)] = kern_exact<T>(p.kid, p.x[D.row0 + i], p.y[D.col0 + j]);
+    const int lane = threadIdx.x % WAVE;
+    for (int32_t i0 = 0; i0 < D.m; i0 += HM_TILE) {
+        const bool ok = i0 + lane < D.m;
+        const T xi = p.x[D.row0 + (ok ? i0 + lane : 0)];
+        T *a = p.A + D.aoff + tile_index(i0, 0, D.n) + lane;
+        for (int32_t j = threadIdx.x / WAVE; j < D.n; j += WPB) {
+            const T v = kern_exact<T>(p.kid, xi, p.y[D.col0 + j]);
+            a[(int64_t)j * HM_TILE] = ok ? v : T(0);
+        }
     }
+}
+
+// The bases' tile padding: the rows past each cluster's last, as zeros. One
+// workgroup per cluster, the row clusters first.
+template <class T>
+__global__ __launch_bounds__(WAVE) void k_pad_basis(DevPlanT<T> p) {
+    const int b = blockIdx.x;
+    const DCluster C = b < p.nrc ? p.rcl[b] : p.ccl[b - p.nrc];
+    T *B = b < p.nrc ? p.U : p.V;
+    const int i = C.len / HM_TILE * HM_TILE + (int)threadIdx.x;
+    if (C.len % HM_TILE == 0 || i < C.len) return;
+    T *o = B + C.boff + tile_index(i, 0, p.r);
+    for (int k = 0; k < p.r; ++k) o[k * HM_TILE] = T(0);
 }
 
 // update! (src/BarycentricMatrix.jl:256-287): one lane per point of a chunk,
@@ -272,10 +294,19 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
     }
 }
 
+// Non-finite values of up to four arrays, one count per workgroup (gridDim.x of
+// them) and array (blockIdx.y)
 template <class T>
-__global__ __launch_bounds__(WG) void k_count_nonfinite(const T *v, int64_t n,
+struct CountArgs {
+    const T *v[4];
+    int64_t n[4];
+};
+template <class T>
+__global__ __launch_bounds__(WG) void k_count_nonfinite(CountArgs<T> a,
                                                         unsigned long long *blockcount) {
     __shared__ unsigned int sh[WG];
+    const T *v = a.v[blockIdx.y];
+    const int64_t n = a.n[blockIdx.y];
     unsigned int cnt = 0;
     for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG)
         cnt += isfinite(v[i]) ? 0u : 1u;
@@ -285,7 +316,7 @@ __global__ __launch_bounds__(WG) void k_count_nonfinite(const T *v, int64_t n,
         if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) blockcount[blockIdx.x] = sh[0];
+    if (threadIdx.x == 0) blockcount[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
 }
 
 // ------------------------------------------------------------------ product

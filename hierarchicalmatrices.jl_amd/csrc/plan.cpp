@@ -12,7 +12,9 @@
 #include <memory>
 #include <string>
 #include <type_traits>
-#include <unordered_map>
+#include <exception>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -100,20 +102,20 @@ struct Builder {
     bool f32 = false;  // Float32 plan: points and intervals are floats, midpoints rounded to float
     std::vector<Leaf> leaves;
     std::vector<HCluster> rcl, ccl;
-    std::unordered_map<uint64_t, int32_t> rmap, cmap;
     std::vector<DFarBlk> far;
-    std::vector<int> far_depth;
     std::vector<DDense> dense;
-    // every indsplit of the tree (row and column side): the tree stays the
-    // same for other points exactly when each split falls at the same index
+    // the indsplits of the tree (row and column side), each range's once: the
+    // tree stays the same for other points exactly when each split falls at
+    // the same index
     std::vector<DSplit> xsplits, ysplits;
     int64_t nd = 0, nk1 = 0, nk2 = 0, far_rows = 0, far_cols = 0, dense_entries = 0;
     int maxdepth = 0;
     int err = 0;
     std::string msg;
     // the interval trees of both sides (every range node() splits, with its
-    // two halves); tok turns false if a lookup meets an inconsistent node, and
-    // the plan then keeps the per-level far field
+    // two halves). A side's ranges at one depth follow from the splits above
+    // them alone, so a range is met as the same half of the same node from
+    // every block, and a node's non-empty range is one cluster
     struct TNode {
         int depth;
         int64_t first, len;
@@ -122,42 +124,17 @@ struct Builder {
         int32_t cl;  // the row / column cluster with this range, or -1
     };
     std::vector<TNode> xt, yt;
-    std::unordered_map<uint64_t, int32_t> xtm, ytm;
-    bool tok = true;
 
-    static uint64_t tkey(int depth, double lo, double hi) {
-        uint64_t a, b;
-        std::memcpy(&a, &lo, 8);
-        std::memcpy(&b, &hi, 8);
-        uint64_t h = a * 0x9E3779B97F4A7C15ull ^ (b + 0x632BE59BD9B4E019ull + (h_mix(a) << 6));
-        return h_mix(h ^ (uint64_t)depth * 0xD1B54A32D192ED03ull);
-    }
-    static uint64_t h_mix(uint64_t v) {
-        v ^= v >> 30; v *= 0xBF58476D1CE4E5B9ull;
-        v ^= v >> 27; v *= 0x94D049BB133111EBull;
-        return v ^ (v >> 31);
-    }
-    int32_t tfind(const std::vector<TNode> &t, const std::unordered_map<uint64_t, int32_t> &m,
-                  int depth, double lo, double hi) const {
-        auto it = m.find(tkey(depth, lo, hi));
-        if (it == m.end()) return -1;
-        const TNode &q = t[it->second];
-        return (q.depth == depth && q.lo == lo && q.hi == hi) ? it->second : -2;
-    }
-    // the node (depth, interval), made on first sight as half `half` of parent
-    void tadd(std::vector<TNode> &t, std::unordered_map<uint64_t, int32_t> &m, int depth,
-              int64_t first, int64_t len, double lo, double hi, int32_t parent, int half) {
-        const int32_t f = tfind(t, m, depth, lo, hi);
-        if (f == -2) { tok = false; return; }
-        if (f >= 0) {
-            const TNode &q = t[f];
-            if (q.first != first || q.len != len || q.parent != parent) tok = false;
-            return;
+    // half h of node p of one side's tree (the range [first, first + len) and
+    // its interval), made on first sight
+    static int32_t half_of(std::vector<TNode> &t, int32_t p, int h, int64_t first, int64_t len,
+                           double lo, double hi) {
+        if (t[p].child[h] < 0) {
+            const int32_t id = (int32_t)t.size();
+            t.push_back({t[p].depth + 1, first, len, lo, hi, p, {-1, -1}, h, -1});
+            t[p].child[h] = id;
         }
-        const int32_t id = (int32_t)t.size();
-        t.push_back({depth, first, len, lo, hi, parent, {-1, -1}, half, -1});
-        m.emplace(tkey(depth, lo, hi), id);
-        if (parent >= 0) t[parent].child[half] = id;
+        return t[p].child[h];
     }
 
     // indsplit (src/BarycentricMatrix.jl:299-307) on a validated non-increasing
@@ -188,22 +165,13 @@ struct Builder {
         return (int64_t)(it - lo);
     }
 
-    int32_t cluster(std::vector<HCluster> &cl, std::unordered_map<uint64_t, int32_t> &mp, int depth,
-                    int64_t first, int64_t len, double lo, double hi) {
-        const uint64_t key = ((uint64_t)depth << 42) | (uint64_t)first;
-        auto it = mp.find(key);
-        if (it != mp.end()) {
-            const HCluster &h = cl[it->second];
-            if (h.len != len || h.lo != lo || h.hi != hi) {
-                err = HM_ERR_INVALID;
-                msg = "internal: inconsistent cluster";
-            }
-            return it->second;
+    // the cluster of a tree node, made on first sight
+    static int32_t cluster(std::vector<HCluster> &cl, TNode &q) {
+        if (q.cl < 0) {
+            q.cl = (int32_t)cl.size();
+            cl.push_back({q.depth, q.first, q.len, q.lo, q.hi});
         }
-        const int32_t id = (int32_t)cl.size();
-        cl.push_back({depth, first, len, lo, hi});
-        mp.emplace(key, id);
-        return id;
+        return q.cl;
     }
 
     void put_dense(int depth, int64_t i0, int64_t m, int64_t j0, int64_t n) {
@@ -213,31 +181,24 @@ struct Builder {
     }
 
     // BarycentricMatrix2D(T, f, a, b, c, d, x, y, ir, jr), src/BarycentricMatrix.jl:236
-    void put_far(int depth, double a, double b, double c, double d, int64_t i0, int64_t m,
-                 int64_t j0, int64_t n) {
-        leaves.push_back({2, depth, i0, m, j0, n, a, b, c, d});
-        far_rows += m;
-        far_cols += n;
-        if (m > 0 && n > 0) {
-            const int32_t rc = cluster(rcl, rmap, depth, i0, m, a, b);
-            const int32_t cc = cluster(ccl, cmap, depth, j0, n, c, d);
+    void put_far(int32_t qx, int32_t qy) {
+        TNode &X = xt[qx], &Y = yt[qy];
+        leaves.push_back({2, X.depth, X.first, X.len, Y.first, Y.len, X.lo, X.hi, Y.lo, Y.hi});
+        far_rows += X.len;
+        far_cols += Y.len;
+        if (X.len > 0 && Y.len > 0) {
+            const int32_t rc = cluster(rcl, X);
+            const int32_t cc = cluster(ccl, Y);
             far.push_back({rc, cc, 0});
-            if (tok) {
-                const int32_t xn = tfind(xt, xtm, depth, a, b), yn = tfind(yt, ytm, depth, c, d);
-                if (xn < 0 || yn < 0) {
-                    tok = false;
-                } else {
-                    xt[xn].cl = rc;
-                    yt[yn].cl = cc;
-                }
-            }
-            far_depth.push_back(depth);
         }
     }
 
-    void node(int type, int depth, int64_t i0, int64_t ni, int64_t j0, int64_t nj, double a,
-              double b, double c, double d) {
+    // the block of tree nodes px (rows) and py (columns)
+    void node(int type, int32_t px, int32_t py) {
         if (err) return;
+        const int depth = xt[px].depth;
+        const int64_t i0 = xt[px].first, ni = xt[px].len, j0 = yt[py].first, nj = yt[py].len;
+        const double a = xt[px].lo, b = xt[px].hi, c = yt[py].lo, d = yt[py].hi;
         maxdepth = std::max(maxdepth, depth);
         if (depth > 200) {
             err = HM_ERR_DEGENERATE;
@@ -245,24 +206,17 @@ struct Builder {
             return;
         }
         if (type == 0) ++nd; else if (type == 1) ++nk1; else ++nk2;
-        const int64_t ni1 = split(x, nx, i0, ni, a, b), ni2 = ni - ni1;
-        const int64_t nj1 = split(y, ny, j0, nj, c, d), nj2 = nj - nj1;
+        // a range is split once; the blocks that meet it again find its halves
+        const bool newx = xt[px].child[0] < 0, newy = yt[py].child[0] < 0;
+        const int64_t ni1 = newx ? split(x, nx, i0, ni, a, b) : xt[xt[px].child[0]].len, ni2 = ni - ni1;
+        const int64_t nj1 = newy ? split(y, ny, j0, nj, c, d) : yt[yt[py].child[0]].len, nj2 = nj - nj1;
         if (err) return;
-        xsplits.push_back({i0, ni, i0 + ni1, mid(a, b)});
-        ysplits.push_back({j0, nj, j0 + nj1, mid(c, d)});
-        const int64_t i2 = i0 + ni1, j2 = j0 + nj1;
         const double ab2 = mid(a, b), cd2 = mid(c, d);
-        if (tok) {  // this node's ranges and their halves in the interval trees
-            const int32_t px = tfind(xt, xtm, depth, a, b), py = tfind(yt, ytm, depth, c, d);
-            if (px < 0 || py < 0) {
-                tok = false;
-            } else {
-                tadd(xt, xtm, depth + 1, i0, ni1, a, ab2, px, 0);
-                tadd(xt, xtm, depth + 1, i2, ni2, ab2, b, px, 1);
-                tadd(yt, ytm, depth + 1, j0, nj1, c, cd2, py, 0);
-                tadd(yt, ytm, depth + 1, j2, nj2, cd2, d, py, 1);
-            }
-        }
+        if (newx) xsplits.push_back({i0, ni, i0 + ni1, ab2});
+        if (newy) ysplits.push_back({j0, nj, j0 + nj1, cd2});
+        const int64_t i2 = i0 + ni1, j2 = j0 + nj1;
+        const int32_t x1 = half_of(xt, px, 0, i0, ni1, a, ab2), x2 = half_of(xt, px, 1, i2, ni2, ab2, b);
+        const int32_t y1 = half_of(yt, py, 0, j0, nj1, c, cd2), y2 = half_of(yt, py, 1, j2, nj2, cd2, d);
         const bool leaf = ni1 < bs && ni2 < bs && nj1 < bs && nj2 < bs;
         const int cd_ = depth + 1;
         if (type == 0) {  // KernelMatrix, src/KernelMatrix.jl:49-70
@@ -272,23 +226,23 @@ struct Builder {
                 put_dense(cd_, i2, ni2, j0, nj1);
                 put_dense(cd_, i2, ni2, j2, nj2);
             } else {
-                node(0, cd_, i0, ni1, j0, nj1, a, ab2, c, cd2);
-                node(1, cd_, i0, ni1, j2, nj2, a, ab2, cd2, d);
-                node(2, cd_, i2, ni2, j0, nj1, ab2, b, c, cd2);
-                node(0, cd_, i2, ni2, j2, nj2, ab2, b, cd2, d);
+                node(0, x1, y1);
+                node(1, x1, y2);
+                node(2, x2, y1);
+                node(0, x2, y2);
             }
         } else if (type == 1) {  // KernelMatrix1, src/KernelMatrix.jl:72-93
-            put_far(cd_, a, ab2, c, cd2, i0, ni1, j0, nj1);
-            put_far(cd_, a, ab2, cd2, d, i0, ni1, j2, nj2);
+            put_far(x1, y1);
+            put_far(x1, y2);
             if (leaf) put_dense(cd_, i2, ni2, j0, nj1);
-            else node(1, cd_, i2, ni2, j0, nj1, ab2, b, c, cd2);
-            put_far(cd_, ab2, b, cd2, d, i2, ni2, j2, nj2);
+            else node(1, x2, y1);
+            put_far(x2, y2);
         } else {  // KernelMatrix2, src/KernelMatrix.jl:95-116
-            put_far(cd_, a, ab2, c, cd2, i0, ni1, j0, nj1);
+            put_far(x1, y1);
             if (leaf) put_dense(cd_, i0, ni1, j2, nj2);
-            else node(2, cd_, i0, ni1, j2, nj2, a, ab2, cd2, d);
-            put_far(cd_, ab2, b, c, cd2, i2, ni2, j0, nj1);
-            put_far(cd_, ab2, b, cd2, d, i2, ni2, j2, nj2);
+            else node(2, x1, y2);
+            put_far(x2, y1);
+            put_far(x2, y2);
         }
     }
 };
@@ -451,6 +405,40 @@ void build_side(int64_t n, const std::vector<DDense> &dense, bool rows,
     }
 }
 
+// f and g, which do not depend on each other: a thread for g where the points
+// make them take longer than starting one (some 20 us); what g throws is thrown
+// again here.
+template <class F, class G>
+void both_sides(int64_t points, F f, G g) {
+    std::exception_ptr thrown;
+    std::thread other;
+    if (points > 1 << 15) {
+        try {
+            other = std::thread([&] {
+                try {
+                    g();
+                } catch (...) {
+                    thrown = std::current_exception();
+                }
+            });
+        } catch (const std::system_error &) {  // no thread to be had
+        }
+    }
+    struct Join {
+        std::thread &t;
+        ~Join() {
+            if (t.joinable()) t.join();
+        }
+    };
+    const bool threaded = other.joinable();
+    {
+        Join join{other};
+        f();
+        if (!threaded) g();
+    }
+    if (thrown) std::rethrow_exception(thrown);
+}
+
 template <class T>
 int upload(T **dst, const std::vector<T> &src) {
     *dst = nullptr;
@@ -554,12 +542,15 @@ struct PlanBufs {
     // matrices, moments per column node, coefficients per row node
     T *nestM = nullptr, *my = nullptr, *mx = nullptr;
     // x .. chebA and the workspace partial .. xt live in this one allocation
-    // (Staging); A, U, V and F are allocated on their own
-    void *arena = nullptr;
+    // (Staging); A, U, V and F are one allocation (factors) in plans from
+    // points, and allocated on their own in plans from blocks
+    void *arena = nullptr, *factors = nullptr;
+    unsigned long long *cnt = nullptr;  // the count of non-finite factors
     DevPlanT<T> dp{};
 
     void release() {
-        void *b[] = {arena, A, U, V, F};
+        void *b[] = {arena, factors ? factors : A, factors ? nullptr : U, factors ? nullptr : V,
+                     factors ? nullptr : F};
         for (void *q : b)
             if (q) (void)hipFree(q);
     }
@@ -693,9 +684,9 @@ struct hm_plan {
     // row leaf. (To a fixed 1e-12, the log kernel's 2^22 random points fell
     // back to the per-level form by their deepest intervals' rounding.)
     template <class TN>
-    void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt, bool tok) {
+    void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt) {
         nest = false;
-        if (!tok || f32 || xt.empty() || yt.empty()) return;
+        if (f32 || xt.empty() || yt.empty()) return;
         auto conv = [](const std::vector<TN> &t, std::vector<DTNode> &o) {
             o.resize(t.size());
             for (size_t k = 0; k < t.size(); ++k) {
@@ -992,6 +983,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (std::is_same_v<T, double>) st.reserve(&b.xt, P->ny * HM_WS_RHS);
         if ((flags & HM_PLAN_MATRIX_FREE) || (std::is_same_v<T, float> && (flags & HM_PLAN_HYBRID)))
             st.reserve(&b.yt, std::max(P->nx, P->ny));
+        if (!(flags & HM_PLAN_MATRIX_FREE)) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS);
         HM_TRY_T(st.commit(&b.arena));
     }
     if (b.my) {  // the moments of empty column nodes are read as zero
@@ -1002,12 +994,14 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     const bool stored = !(flags & HM_PLAN_MATRIX_FREE);
     const bool hybrid = (flags & HM_PLAN_HYBRID) != 0;
     if (stored) {
-        HM_TRY_T(dalloc(&b.A, nA));
-        HM_TRY_T(dalloc(&b.F, nF));
+        Staging st;
+        st.reserve(&b.A, nA);
+        st.reserve(&b.F, nF);
         if (!hybrid) {
-            HM_TRY_T(dalloc(&b.U, nU));
-            HM_TRY_T(dalloc(&b.V, nV));
+            st.reserve(&b.U, nU);
+            st.reserve(&b.V, nV);
         }
+        HM_TRY_T(st.commit(&b.factors));
     }
 #undef HM_TRY_T
     DevPlanT<T> &dp = b.dp;
@@ -1019,16 +1013,11 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
 
     if (stored) {
-        // tile padding (rows beyond a block's or cluster's length) is zeroed
-        bool padded = false;
-        for (const DDense &D : P->dense) padded |= (D.m % HM_TILE) != 0;
-        for (const DCluster &C : P->rcl) padded |= (C.len % HM_TILE) != 0;
-        for (const DCluster &C : P->ccl) padded |= (C.len % HM_TILE) != 0;
         const bool user = P->kid == HM_USER;  // A and F come from hm_plan_set_leaf_data
-        if (padded || user) {
-            T *arrs[] = {b.A, b.U, b.V, user ? b.F : nullptr};
-            const int64_t lens[] = {nA, nU, nV, nF};
-            for (int q = 0; q < 4; ++q)
+        if (user) {
+            T *arrs[] = {b.A, b.F};
+            const int64_t lens[] = {nA, nF};
+            for (int q = 0; q < 2; ++q)
                 if (lens[q] > 0 && arrs[q]) {
                     hipError_t e0 = hipMemsetAsync((void *)arrs[q], 0, sizeof(T) * lens[q], s);
                     if (e0 != hipSuccess) return fail(HM_ERR_HIP, "memset: %s", hipGetErrorString(e0));
@@ -1037,25 +1026,17 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         hipError_t e = hmx_launch_compress(dp, s);
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression launch: %s", hipGetErrorString(e));
         // count non-finite factors (coincident points give Inf, as in the reference)
-        unsigned long long *d_cnt = nullptr;
-        e = hipMalloc((void **)&d_cnt, 1024 * sizeof(unsigned long long));
-        if (e == hipSuccess) {
-            std::vector<unsigned long long> h(1024);
-            int64_t total = 0;
-            const T *arrs[] = {user ? nullptr : b.A, b.U, b.V, user ? nullptr : b.F};
-            const int64_t lens[] = {nA, nU, nV, nF};
-            for (int q = 0; q < 4 && e == hipSuccess; ++q) {
-                if (lens[q] <= 0 || !arrs[q]) continue;
-                e = hipMemsetAsync(d_cnt, 0, 1024 * sizeof(unsigned long long), s);
-                if (e == hipSuccess) e = hmx_launch_count_nonfinite(arrs[q], lens[q], d_cnt, s);
-                if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d_cnt, 1024 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-                if (e == hipSuccess) e = hipStreamSynchronize(s);
-                for (auto v : h) total += (int64_t)v;
-            }
-            (void)hipFree(d_cnt);
-            P->nonfinite = total;
-            P->nonfinite_basis = total;
-        }
+        const T *arrs[] = {user ? nullptr : b.A, b.U, b.V, user ? nullptr : b.F};
+        const int64_t lens[] = {nA, nU, nV, nF};
+        std::vector<unsigned long long> h(4 * HM_COUNT_BLOCKS, 0);
+        e = hmx_launch_count_nonfinite(arrs, lens, b.cnt, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(h.data(), b.cnt, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        int64_t total = 0;
+        for (auto v : h) total += (int64_t)v;
+        P->nonfinite = total;
+        P->nonfinite_basis = total;
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression: %s", hipGetErrorString(e));
     }
     hipError_t e = hipStreamSynchronize(s);
@@ -1126,16 +1107,17 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
             const size_t q = (size_t)(std::max(I.nx, I.ny) / std::max(blocksize, 1)) + 16;
             Bt.leaves.reserve(20 * q);
             Bt.far.reserve(14 * q);
-            Bt.far_depth.reserve(14 * q);
             Bt.dense.reserve(8 * q);
             Bt.rcl.reserve(5 * q);
             Bt.ccl.reserve(5 * q);
-            Bt.rmap.reserve(5 * q);
-            Bt.cmap.reserve(5 * q);
+            Bt.xt.reserve(6 * q);
+            Bt.yt.reserve(6 * q);
+            Bt.xsplits.reserve(3 * q);
+            Bt.ysplits.reserve(3 * q);
         }
-        Bt.tadd(Bt.xt, Bt.xtm, 0, 0, I.nx, I.a, I.b, -1, 0);
-        Bt.tadd(Bt.yt, Bt.ytm, 0, 0, I.ny, I.c, I.d, -1, 0);
-        Bt.node(0, 0, 0, I.nx, 0, I.ny, I.a, I.b, I.c, I.d);
+        Bt.xt.push_back({0, 0, I.nx, I.a, I.b, -1, {-1, -1}, 0, -1});
+        Bt.yt.push_back({0, 0, I.ny, I.c, I.d, -1, {-1, -1}, 0, -1});
+        Bt.node(0, 0, 0);
         if (Bt.err) {
             return count == 1 ? fail(Bt.err, "%s", Bt.msg.c_str())
                               : fail(Bt.err, "instance %lld: %s", (long long)t, Bt.msg.c_str());
@@ -1170,7 +1152,6 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
             };
             merge(B.xt, Bt.xt, ro, rb);
             merge(B.yt, Bt.yt, co, cb);
-            B.tok = B.tok && Bt.tok;
         }
         B.nd += Bt.nd; B.nk1 += Bt.nk1; B.nk2 += Bt.nk2;
         B.far_rows += Bt.far_rows; B.far_cols += Bt.far_cols; B.dense_entries += Bt.dense_entries;
@@ -1231,10 +1212,10 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
         C.far_end = (int32_t)k + 1;
     }
 
-    build_side(nx, P->dense, true, P->rcl, P->rows);
-    build_side(ny, P->dense, false, P->ccl, P->cols);
+    both_sides(nx + ny, [&] { build_side(nx, P->dense, true, P->rcl, P->rows); },
+               [&] { build_side(ny, P->dense, false, P->ccl, P->cols); });
     P->list_multi();
-    P->build_nest(B.xt, B.yt, B.tok);
+    P->build_nest(B.xt, B.yt);
     // the cluster maps the Float64 MFMA upward pass reads from its task
     // record: (a+b)/2 and 1/((b-a)/2) as the Float64 cluster maps form them
     if (!f32) {
