@@ -8,6 +8,29 @@ template <class T> struct Real2;
 template <> struct Real2<double> { using type = double2; };
 template <> struct Real2<float> { using type = float2; };
 
+// Where a single-right-hand-side product takes its near-field entries and F
+// from (nested1.h)
+enum { N1_FREE, N1_EXACT, N1_READ };
+
+// One side of the single-right-hand-side passes over the interval trees
+struct N1Side {
+    const N1Sub *sub;
+    const N1Node *node;
+    const int32_t *lev;
+    const N1Leaf *leaf;
+    const N1Path *path;
+    const N1Chunk *ch;
+    const N1Run *run;    // of the chunks (nunit = 0)
+    const N1Unit *unit;
+    const N1UnitRun *urun;
+    // as output side: the translation records in far_by_* order (a source
+    // above the subtrees with its slots, another with nslots = 0), and the
+    // clusters, those with a source above the subtrees first
+    const DTrRec *tr;
+    const N1Target *target;
+    int32_t nsub, nch, ncl, nheavy, nunit;
+};
+
 // Device-side view of a plan (all pointers are device pointers). T is the
 // element type of the plan: double (Float64) or float (Float32).
 template <class T>
@@ -43,6 +66,7 @@ struct DevPlanT {
     int32_t nrtask, nctask;
     int64_t nslots_r, nslots_c;
     T *A, *U, *V, *F;          // stored factors (null when matrix-free)
+    int32_t *uv_bad;           // set to 1 when a formed value of U or V is not finite
     // the row / column clusters with more than one upward task (the others'
     // tasks write w themselves)
     const int32_t *multi_r, *multi_c;
@@ -66,6 +90,11 @@ struct DevPlanT {
     int32_t nyleaf;
     const T *nestM;
     T *my, *mx;
+    // one right-hand side over the interval trees (n1 is 0 when the trees or
+    // the rank do not allow it), and its padded r x r matrices (N1Mat)
+    int n1;
+    N1Side n1x, n1y;
+    const T *n1m;
 };
 
 template <class T>
@@ -113,6 +142,13 @@ hipError_t hmx_launch_matvec(const DevPlan &p, const MvArgs &a, bool transpose, 
 // dense blocks, 2 regenerates them.
 hipError_t hmx_launch_matvec_m(const DevPlan &p, const MvArgs &a, int mode, int prec, int nq,
                                hipStream_t s);
+// one product of one right-hand side over the interval trees (p.n1, r <= 32);
+// src: N1_FREE, N1_EXACT or N1_READ. Pass events as hmx_launch_matvec's (no
+// reduce).
+hipError_t hmx_launch_matvec_n1(const DevPlan &p, const MvArgs &a, bool transpose, int src,
+                                hipStream_t s, const hipEvent_t *ev);
+hipError_t hmx_launch_matvec_n1(const DevPlanF &p, const MvArgsF &a, bool transpose, int src,
+                                hipStream_t s, const hipEvent_t *ev);
 // gradients (matrix-free near field, Chebyshev-form far field):
 //   forward (tr = false): y = beta*y + s .* (d/dx_i of (H x)_i)
 //   transpose (tr = true): y = beta*y + H^T x, y2 = beta*y2 + s .* (d/dy_j of (H^T x)_j)

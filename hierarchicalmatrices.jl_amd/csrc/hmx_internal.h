@@ -130,3 +130,74 @@ struct DSplit {
     int64_t first, len, at;
     double mid;
 };
+
+// Single right-hand sides over the interval trees: each side's tree is cut
+// into subtrees of at most N1_NODES nodes and a few chunks, each walked by one
+// workgroup (nested1.h). Node numbers inside a subtree are local: breadth
+// first from its root 0, so a depth's nodes are consecutive and every node
+// precedes its halves.
+#define N1_NODES 63          // nodes per subtree (LDS: one rank vector each)
+#define N1_PATH 16           // path nodes staged together
+#define N1_SPLIT_CHUNKS 4096 // a downward workgroup per chunk up to this many chunks
+
+struct N1Sub {
+    int32_t node, nnode;  // first node record, nodes
+    int32_t lev, nlev;    // first depth offset (nlev + 1 of them), depths
+    int32_t leaf, nleaf;  // first leaf record, non-empty leaves
+    int32_t path, npath;  // the nodes above the root, the tree's root first
+    int32_t ch, nch;      // the chunks of its points
+    int32_t unit, nunit;  // their units (none where a workgroup takes a chunk)
+};
+
+struct N1Node {
+    int32_t cl;    // the cluster with this range, or -1
+    int32_t c[2];  // halves (local), -1: none or empty
+};
+
+struct N1Leaf {
+    int64_t first;
+    int32_t len, loc;  // points, local node
+    double cx, cy;     // (center, 1/halfwidth)
+};
+
+// A node above a subtree: its cluster (or -1), the half of it that holds the
+// subtree, and the subtree's partial-sum slot of that cluster (-1: no cluster)
+struct N1Path {
+    int64_t slot;
+    int32_t cl, half;
+};
+
+struct N1Chunk {
+    int64_t p0;         // first point
+    int32_t np, leaf;   // points; local node of the leaf holding them
+    int32_t run, nrun;  // the near field's column runs
+    int32_t sub, pad;
+    double cx, cy;      // the leaf's (center, 1/halfwidth)
+};
+
+// A cluster of the output side and its translation records
+struct N1Target {
+    int32_t id, beg, end;
+};
+
+// A dense block as a chunk reads it: the columns q0 .. q0 + n - 1 of the other
+// side, the chunk's rows from row off of the block on, and the stored entries
+// (aoff; cols = the block's columns as stored). The output side's columns take
+// the block's rows and columns exchanged.
+struct N1Run {
+    int64_t q0, aoff;
+    int32_t n, off, cols, pad;
+};
+
+// Two consecutive chunks of a subtree (or its last one), a wavefront's work
+struct N1Unit {
+    int32_t ch, nch;
+    int32_t run, nrun;
+};
+
+// A run of consecutive columns of a unit's dense blocks: mask 1 those of its
+// first chunk, 2 of the second, 3 of both
+struct N1UnitRun {
+    int64_t q0;
+    int32_t n, mask;
+};

@@ -1,5 +1,5 @@
 // inst_f32_r16.hip -- kernels of FP32 plans for ranks in bucket 16 (r <= 16).
-#include "kernels_impl.h"
+#include "nested1.h"
 
 hipError_t hmx_matvec_f32_r16(const DevPlanF &p, const MvArgsF &a, bool tr, int mode, int kb,
                               hipStream_t s, const hipEvent_t *ev) {
@@ -13,4 +13,8 @@ hipError_t hmx_grad_f32_r16(const DevPlanF &p, const MvArgsF &a, bool tr, float 
 
 hipError_t hmx_gen_basis_f32_r16(const DevPlanF &p, hipStream_t s) {
     return hmxk::gen_basis_r<float, 16>(p, s);
+}
+
+hipError_t hmx_matvec_n1_f32_r16(const DevPlanF &p, const MvArgsF &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
+    return hmxk::matvec_n1<float, 16>(p, a, tr, src, s, ev);
 }

@@ -1,5 +1,5 @@
 // inst_r24.hip -- kernels for ranks in bucket 24 (r <= 24).
-#include "kernels_impl.h"
+#include "nested1.h"
 
 hipError_t hmx_matvec_r24(const DevPlan &p, const MvArgs &a, bool tr, int mode, int kb,
                           hipStream_t s, const hipEvent_t *ev) {
@@ -16,4 +16,8 @@ hipError_t hmx_gen_basis_r24(const DevPlan &p, hipStream_t s) { return hmxk::gen
 hipError_t hmx_matvec_m_r24(const DevPlan &p, const MvArgs &a, int mode, int prec, int nq,
                             hipStream_t s) {
     return hmxk::matvec_m_r<32>(p, a, mode, prec, nq, s);
+}
+
+hipError_t hmx_matvec_n1_r24(const DevPlan &p, const MvArgs &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
+    return hmxk::matvec_n1<double, 24>(p, a, tr, src, s, ev);
 }

@@ -249,12 +249,12 @@ __global__ __launch_bounds__(WAVE) void k_pad_basis(DevPlanT<T> p) {
 }
 
 // update! (src/BarycentricMatrix.jl:256-287): one lane per point of a chunk,
-// for every cluster covering the chunk.
+// for every cluster covering the chunk. *bad = 1 where a value is not finite.
 template <class T, int RMAX>
 __global__ __launch_bounds__(WG) void k_gen_basis(const DChunk *ch, int nch, const DFar *fl,
                                                  const DCluster *cl, const T *nodes,
                                                  const T *lam, const T *pts,
-                                                 T *B, int r) {
+                                                 T *B, int r, int32_t *bad) {
 #pragma clang fp contract(off)
     const int wid = wave_id();
     const int lane = threadIdx.x % WAVE;
@@ -275,9 +275,15 @@ __global__ __launch_bounds__(WG) void k_gen_basis(const DChunk *ch, int nch, con
         for (int k = 0; k < RMAX; ++k)
             if (k < r) s += row[k];
         T *out = B + C.boff + tile_index(f.off + lane, 0, r);
+        bool fin = true;
 #pragma unroll
         for (int k = 0; k < RMAX; ++k)
-            if (k < r) out[k * HM_TILE] = row[k] / s;
+            if (k < r) {
+                const T v = row[k] / s;
+                out[k * HM_TILE] = v;
+                fin = fin && isfinite(v);
+            }
+        if (!fin) *bad = 1;
     }
 }
 
@@ -294,8 +300,9 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
     }
 }
 
-// Non-finite values of up to four arrays, one count per workgroup (gridDim.x of
-// them) and array (blockIdx.y)
+// Per workgroup (gridDim.x of them) and array (blockIdx.y, up to four): the
+// non-finite values (low half of the word) and the finite ones within 10^8
+// (10^2 for float) of the largest number (high half, one per thread at most)
 template <class T>
 struct CountArgs {
     const T *v[4];
@@ -304,12 +311,17 @@ struct CountArgs {
 template <class T>
 __global__ __launch_bounds__(WG) void k_count_nonfinite(CountArgs<T> a,
                                                         unsigned long long *blockcount) {
-    __shared__ unsigned int sh[WG];
+    __shared__ unsigned long long sh[WG];
     const T *v = a.v[blockIdx.y];
     const int64_t n = a.n[blockIdx.y];
-    unsigned int cnt = 0;
-    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG)
-        cnt += isfinite(v[i]) ? 0u : 1u;
+    const T lim = sizeof(T) == 8 ? (T)1e300 : (T)1e36;
+    unsigned int low = 0, high = 0;
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
+        const T q = v[i];
+        low += isfinite(q) ? 0u : 1u;
+        high |= isfinite(q) && fabsT(q) > lim ? 1u : 0u;
+    }
+    const unsigned long long cnt = (unsigned long long)low | ((unsigned long long)high << 32);
     sh[threadIdx.x] = cnt;
     __syncthreads();
     for (int o = WG / 2; o > 0; o /= 2) {
@@ -1039,14 +1051,17 @@ inline int64_t tr_waves(int64_t ncl, int r, int kb) {
     return (ncl + G - 1) / G;
 }
 
+__global__ void k_clear_word(int32_t *w) { *w = 0; }
+
 template <class T, int RMAX>
 hipError_t gen_basis_r(const DevPlanT<T> &p, hipStream_t s) {
+    k_clear_word<<<1, 1, 0, s>>>(p.uv_bad);
     if (p.ncch > 0 && p.V)
         k_gen_basis<T, RMAX><<<nblk(p.ncch), WG, 0, s>>>(p.cch, p.ncch, p.cfar, p.ccl, p.cnodes, p.lam,
-                                                     p.y, p.V, p.r);
+                                                     p.y, p.V, p.r, p.uv_bad);
     if (p.nrch > 0 && p.U)
         k_gen_basis<T, RMAX><<<nblk(p.nrch), WG, 0, s>>>(p.rch, p.nrch, p.rfar, p.rcl, p.rnodes, p.lam,
-                                                     p.x, p.U, p.r);
+                                                     p.x, p.U, p.r, p.uv_bad);
     return hipGetLastError();
 }
 
@@ -2469,11 +2484,14 @@ hipError_t matvec_r(const DevPlanT<T> &p, const MvArgsT<T> &a, bool tr, int mode
     hipError_t hmx_gen_basis_r##R(const DevPlan &p, hipStream_t s);                              \
     hipError_t hmx_matvec_m_r##R(const DevPlan &p, const MvArgs &a, int mode, int prec, int nq,  \
                                  hipStream_t s);
+#define HMX_DECLARE_BUCKET_N1(R)                                                                \
+    hipError_t hmx_matvec_n1_r##R(const DevPlan &p, const MvArgs &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev);
 #define HMX_DECLARE_BUCKET_F32(R)                                                               \
     hipError_t hmx_matvec_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, int mode,      \
                                    int kb, hipStream_t s, const hipEvent_t *ev);                \
     hipError_t hmx_grad_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, float *y2,       \
                                  int64_t incy2, const float *sv, int64_t incs, hipStream_t s);  \
+    hipError_t hmx_matvec_n1_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev);          \
     hipError_t hmx_gen_basis_f32_r##R(const DevPlanF &p, hipStream_t s);
 HMX_DECLARE_BUCKET(8)
 HMX_DECLARE_BUCKET(16)
@@ -2481,6 +2499,10 @@ HMX_DECLARE_BUCKET(24)
 HMX_DECLARE_BUCKET(32)
 HMX_DECLARE_BUCKET(48)
 HMX_DECLARE_BUCKET(64)
+HMX_DECLARE_BUCKET_N1(8)
+HMX_DECLARE_BUCKET_N1(16)
+HMX_DECLARE_BUCKET_N1(24)
+HMX_DECLARE_BUCKET_N1(32)
 HMX_DECLARE_BUCKET_F32(8)
 HMX_DECLARE_BUCKET_F32(16)
 HMX_DECLARE_BUCKET_F32(32)

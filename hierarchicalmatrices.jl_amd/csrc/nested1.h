@@ -1,0 +1,881 @@
+// nested1.h -- gfx950 passes of one right-hand side with a nested far field
+// (templates; instantiated per rank bucket, ranks up to 32, by inst_r*.hip).
+//
+// Per level, every point enters the moments of each cluster above it and every
+// row evaluates each covering cluster's series (12 levels at n = 2^20). Here a
+// point enters its tree leaf's moments alone and a row evaluates its leaf's
+// series alone; the interval trees carry the rest by the two fixed
+// re-expansion matrices of a half (T_k(s/2 -+ 1/2) = sum_m M[k][m] T_m(s)).
+// Each side's tree is cut at plan time into subtrees of a few chunks (N1Sub);
+// one workgroup walks a subtree in LDS, and the part of the tree above it as a
+// path of single nodes, so a product is three launches:
+//   up         per subtree: its leaves' moments, mu_P = M_0 mu_0 + M_1 mu_1 up
+//              to its root, w = A mu of the clusters in it; then the root's
+//              moments re-expanded up the path, one slot per cluster met
+//   translate  per cluster of the output side: z = sum_b F_b w_b; a source above
+//              the subtrees is summed from its slots (in slot order);
+//              coefficients c = A^T z
+//   down       per subtree: coefficients down the path and the subtree by one
+//              wavefront, then one series per row, added onto y
+// The near field, y = beta*y + near, needs nothing of the chain and fills the
+// first two launches, which wait on latencies. No atomics; the order of every
+// sum is fixed by the plan.
+//
+// Few chunks: a near workgroup takes one, its columns (read by scalar loads)
+// split over the wavefronts. Many: a wavefront takes two chunks, a row of each
+// per lane, and its columns through LDS. (By scalar loads throughout, n = 2^20
+// took 127 us, waiting on the scalar caches: 1.7 M 64-byte requests, four of
+// five misses.)
+//
+// Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 182 us
+// a product, matrix-free 233 -> 128 us, where the vector instructions alone
+// take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
+// rank 20: 427 -> 60 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
+// n = 1000: 27.0 -> 23.4 us.
+#pragma once
+#include "kernels_impl.h"
+
+#include <algorithm>
+
+namespace hmxk {
+namespace {
+
+// Where the near field's entries and F come from:
+// (N1_FREE, N1_EXACT and N1_READ of hmx_device.h)
+//   N1_FREE   formed from the points and nodes, several terms of 1/d^m on one
+//             reciprocal (matrix-free products)
+//   N1_EXACT  formed term by term, as the stored entries are rounded, and summed
+//             in the order of N1_READ: a stored or hybrid plan of 1/d^m, whose
+//             values it saves reading
+//   N1_READ   the stored entries (the log kernel, a caller's f, entries that
+//             are not all finite)
+
+// ----------------------------------------------------- wave-uniform loads
+template <class T> struct Vec8;
+template <> struct Vec8<double> { typedef double type __attribute__((ext_vector_type(8), aligned(8))); };
+template <> struct Vec8<float> { typedef float type __attribute__((ext_vector_type(8), aligned(4))); };
+#define HMX_CONST_AS __attribute__((address_space(4)))
+
+// o = p[0 .. 7] by scalar loads (p wave-uniform, not written by this kernel)
+template <class T>
+__device__ __forceinline__ void sload8(const T *p, T (&o)[8]) {
+    using V = typename Vec8<T>::type;
+    const V v = *(const HMX_CONST_AS V *)(p);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) o[u] = v[u];
+}
+template <class T>
+__device__ __forceinline__ T sload1(const T *p) {
+    return *(const HMX_CONST_AS T *)(p);
+}
+
+// a table record (a multiple of 4 bytes) by scalar loads
+template <class S>
+__device__ __forceinline__ S sload_struct(const S *p) {
+    constexpr int N = sizeof(S) / 4;
+    int32_t w[N];
+    const HMX_CONST_AS int32_t *q = (const HMX_CONST_AS int32_t *)(const void *)p;
+#pragma unroll
+    for (int k = 0; k < N; ++k) w[k] = q[k];
+    S o;
+    __builtin_memcpy(&o, w, sizeof(S));
+    return o;
+}
+
+// ------------------------------------------------------------- near field
+// zero, denormal, infinity or NaN
+__device__ __forceinline__ bool odd_class(double v) { return __builtin_amdgcn_class(v, 0x2F7); }
+__device__ __forceinline__ bool odd_class(float v) { return __builtin_amdgcn_classf(v, 0x2F7); }
+__device__ __forceinline__ double rcp_raw(double v) { return __builtin_amdgcn_rcp(v); }
+__device__ __forceinline__ float rcp_raw(float v) { return __builtin_amdgcn_rcpf(v); }
+__device__ __forceinline__ double rcp_refine(double d, double r) {
+    double e = __builtin_fma(-d, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-d, r, 1.0);
+    return __builtin_fma(r, e, r);
+}
+__device__ __forceinline__ float rcp_refine(float d, float r) {
+    const float e = __builtin_fmaf(-d, r, 1.0f);
+    return __builtin_fmaf(r, e, r);
+}
+
+// acc_i + sum_{u < N} f(p_i, q_u) v_u for NR rows (f(q_u, p_i) when TR).
+// 1/d^m: the terms of four columns over one common denominator, v0/d0 + v1/d1
+// = (v0 d1 + v1 d0) / (d0 d1) twice over. If a denominator leaves the normal
+// range (its reciprocal is zero, denormal, infinite or NaN) the lane forms its
+// terms one by one; one test for all of the denominators, so that their chains
+// run side by side (a branch each: n = 2^20 spent 45 us more). FP32 holds four
+// factors of 1/d only; its other powers share a reciprocal between two.
+// EXACT: term by term. The refined reciprocal is 1/d^m rounded as a division
+// rounds it: before its last step it is within 2^-48, and that step's own
+// error is the final rounding.
+template <class T, int KID, bool TR, bool EXACT, int N, int NR>
+__device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T *acc) {
+    if constexpr (KID <= 2 && !EXACT) {
+        constexpr int S = (sizeof(T) == 8 || KID == 0) ? 4 : 2, G = N / S;
+        T num[NR][G], den[NR][G], r[NR][G];
+        bool odd = false;
+        auto dist = [&](int i, int u) {
+            const T e = TR ? q[u] - p[i] : p[i] - q[u];
+            return KID == 0 ? e : KID == 1 ? e * e : e * e * e;
+        };
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const int u = g * S;
+                const T d0 = dist(i, u), d1 = dist(i, u + 1);
+                T n = fmaT(v[u], d1, v[u + 1] * d0), d = d0 * d1;
+                if constexpr (S == 4) {
+                    const T d2 = dist(i, u + 2), d3 = dist(i, u + 3);
+                    const T n2 = fmaT(v[u + 2], d3, v[u + 3] * d2), e = d2 * d3;
+                    n = fmaT(n, e, n2 * d);
+                    d = d * e;
+                }
+                num[i][g] = n;
+                den[i][g] = d;
+                r[i][g] = rcp_raw(d);
+                odd |= odd_class(r[i][g]);
+            }
+        if (__builtin_expect(odd, 0)) {
+            for (int i = 0; i < NR; ++i)
+#pragma unroll
+                for (int u = 0; u < N; ++u) acc[i] = fmaT(rcpT(dist(i, u)), v[u], acc[i]);
+        } else {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int i = 0; i < NR; ++i)
+                    acc[i] = fmaT(num[i][g], rcp_refine(den[i][g], r[i][g]), acc[i]);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const T f = TR ? kern_fast<T, KID>(q[u], p[i]) : kern_fast<T, KID>(p[i], q[u]);
+                acc[i] = fmaT(f, v[u], acc[i]);
+            }
+    }
+}
+
+// One row's sum over a chunk's dense blocks (its runs), eight columns at a
+// time: batches b0, b0 + bs, ... of each block. A block's last batch is its last
+// eight columns, those of the batch before it at weight zero; a block narrower
+// than eight repeats its last column at weight zero. (The next batch is not
+// loaded ahead: two batches and the addresses do not fit the scalar registers,
+// and the other wavefronts cover the loads.) row: the lane's row of the chunk.
+template <class T, int KID, bool TR, int SRC>
+__device__ __forceinline__ T near_runs(const N1Run *runs, int nrun, T p, const T *pts_in,
+                                       const T *A, const T *x, int64_t incx, int row, int b0,
+                                       int bs) {
+    T acc = T(0);
+    for (int e = 0; e < nrun; ++e) {
+        const N1Run R = sload_struct(runs + e);
+        const T *qs = pts_in + R.q0, *vs = x + R.q0 * incx;
+        // stored entries: element (row, j) of the block, tiles of 64 rows
+        const int i = R.off + row;
+        const T *Ar = SRC != N1_READ ? nullptr
+                      : TR           ? A + R.aoff + (int64_t)i * HM_TILE
+                                     : A + R.aoff + tile_index(i, 0, R.cols);
+        auto entry = [&](int j) {
+            return TR ? Ar[(int64_t)(j >> 6) * HM_TILE * R.cols + (j & (HM_TILE - 1))]
+                      : Ar[j * HM_TILE];
+        };
+        for (int t = b0; 8 * t < R.n; t += bs) {
+            T q[8], v[8];
+            const int j0 = R.n >= 8 ? min(8 * t, R.n - 8) : 0;
+            if (R.n >= 8) {
+                if constexpr (SRC != N1_READ) sload8(qs + j0, q);
+                if (incx == 1) {
+                    sload8(vs + j0, v);
+                } else {
+                    const T *vj = vs + j0 * incx;
+#pragma unroll
+                    for (int u = 0; u < 8; ++u, vj += incx) v[u] = sload1(vj);
+                }
+                if (j0 < 8 * t) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = j0 + u < 8 * t ? T(0) : v[u];
+                }
+                if constexpr (SRC == N1_READ) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) q[u] = entry(j0 + u);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int j = min(u, R.n - 1);
+                    if constexpr (SRC == N1_READ) q[u] = entry(j);
+                    else q[u] = sload1(qs + j);
+                    const T xv = sload1(vs + j * incx);
+                    v[u] = u < R.n ? xv : T(0);
+                }
+            }
+            if constexpr (SRC == N1_READ) {
+                // a column at weight zero adds nothing, whatever its entry
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (j0 + u >= 8 * t && j0 + u < R.n) acc = fmaT(q[u], v[u], acc);
+            } else {
+                near_terms<T, KID, TR, SRC == N1_EXACT, 8, 1>(&p, q, v, &acc);
+            }
+        }
+    }
+    return acc;
+}
+
+// Columns in LDS, for wavefronts with two rows per lane (rows of two chunks):
+// the sums of a tile's n columns (a multiple of eight, padded at weight zero)
+// for one or both rows. A 16-byte broadcast read takes 8 LDS cycles, shared by
+// four SIMDs, where a row's four terms take 23 vector cycles a column: read
+// for one row alone, LDS would be the slower of the two.
+template <class T, int KID, bool TR, bool EXACT, int NR>
+__device__ __forceinline__ void near_tile(const V2<T> *t, int n, const T (&p)[NR], T (&acc)[NR]) {
+    constexpr int N = KID == 3 ? 2 : 8;
+    for (int j = 0; j < n; j += N) {
+        T q[N], v[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const V2<T> c = t[j + u];
+            q[u] = c.x;
+            v[u] = c.y;
+        }
+        near_terms<T, KID, TR, EXACT, N, NR>(p, q, v, acc);
+    }
+}
+
+// Near field of a unit (one or two chunks, a row of each per lane): its runs'
+// columns pass through this wavefront's LDS 64 at a time, the next tile's
+// loads in flight meanwhile. A run serves the first chunk (mask 1), the second
+// (2) or both (3).
+template <class T, int KID, bool TR, bool EXACT>
+__device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const T (&p)[2],
+                                          const T *pts_in, const T *x, int64_t incx,
+                                          V2<T> (*tile)[WAVE], int lane, T (&acc)[2]) {
+    if (nrun == 0) return;
+    N1UnitRun R = sload_struct(runs);
+    int e = 0, j = 0, b = 0;
+    auto load = [&](const N1UnitRun &Q, int j0, V2<T> &c) {
+        const int64_t at = Q.q0 + min(j0 + lane, Q.n - 1);
+        c.x = pts_in[at];
+        c.y = x[at * incx];
+    };
+    V2<T> c;
+    load(R, 0, c);
+    while (e < nrun) {
+        const int n = min(WAVE, R.n - j), mask = R.mask;
+        if (lane >= n) c.y = T(0);
+        V2<T> *t = tile[b];
+        t[lane] = c;
+        wave_sync();
+        j += WAVE;
+        if (j >= R.n) {
+            j = 0;
+            if (++e < nrun) R = sload_struct(runs + e);
+        }
+        if (e < nrun) load(R, j, c);
+        const int n8 = (n + 7) & ~7;
+        if (mask == 3) {
+            near_tile<T, KID, TR, EXACT, 2>(t, n8, p, acc);
+        } else {
+            const T p1[1] = {mask == 1 ? p[0] : p[1]};
+            T a1[1] = {mask == 1 ? acc[0] : acc[1]};
+            near_tile<T, KID, TR, EXACT, 1>(t, n8, p1, a1);
+            if (mask == 1) acc[0] = a1[0];
+            else acc[1] = a1[0];
+        }
+        b ^= 1;
+    }
+}
+
+template <class T>
+__device__ __forceinline__ void n1_write(const N1Chunk &C, const MvArgsT<T> &a, int beta, int lane,
+                                         T v) {
+    if (lane < C.np) {
+        T *yo = a.y + (C.p0 + lane) * a.incy;
+        *yo = (beta ? *yo : T(0)) + v;
+    }
+}
+
+// One workgroup of the near field, y = beta*y + near: a chunk, its columns
+// split over the wavefronts and their sums added in LDS in wavefront order, or
+// (with units) a unit per wavefront.
+template <class T>
+struct NearLds {
+    union {
+        V2<T> tile[WPB][2][WAVE];
+        T red[WPB][WAVE];
+    };
+    __device__ NearLds() {}
+};
+template <class T, int KID, bool TR, int SRC>
+__device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pts_out,
+                                           const T *pts_in, const T *A, const MvArgsT<T> &a,
+                                           NearLds<T> &s) {
+    const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
+    if (o.nunit == 0) {
+        const N1Chunk C = sload_struct(o.ch + blk);
+        const int row = min(lane, C.np - 1);
+        const T po = SRC == N1_READ ? T(0) : pts_out[C.p0 + row];
+        T acc = near_runs<T, KID, TR, SRC>(o.run + C.run, C.nrun, po, pts_in, A, a.x, a.incx, row,
+                                           wv, WPB);
+        s.red[wv][lane] = acc;
+        __syncthreads();
+        if (wv != 0) return;
+#pragma unroll
+        for (int u = 1; u < WPB; ++u) acc += s.red[u][lane];
+        n1_write(C, a, a.beta, lane, acc);
+        return;
+    }
+    if constexpr (SRC == N1_READ) return;  // stored entries in units: k_down's near part
+    const int c = blk * WPB + wv;
+    if (c >= o.nunit) return;
+    const N1Unit Un = sload_struct(o.unit + c);
+    N1Chunk C[2];
+    T po[2], acc[2] = {T(0), T(0)};
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        C[q] = sload_struct(o.ch + Un.ch + (q < Un.nch ? q : 0));
+        po[q] = pts_out[C[q].p0 + min(lane, C[q].np - 1)];
+    }
+    near_unit<T, KID, TR, SRC == N1_EXACT>(o.urun + Un.run, Un.nrun, po, pts_in, a.x, a.incx, s.tile[wv], lane, acc);
+    n1_write(C[0], a, a.beta, lane, acc[0]);
+    if (Un.nch == 2) n1_write(C[1], a, a.beta, lane, acc[1]);
+}
+
+// -------------------------------------------------------------- far field
+// A plan's r x r matrices for lanes (m, h) = (lane % 32, lane / 32), padded
+// with zeros to RMAX, one row of 64 values per step (N1Mats): M_h[m][k] and
+// M_h[k][m] for k < RMAX, A[m][16h' + j] and A[h' + j][m] for j < RMAX / 2.
+template <class T, int RMAX>
+struct N1Mat {
+    static constexpr int HALF = RMAX / 2;
+    static constexpr int MU = 0, MD = RMAX * WAVE, AU = 2 * RMAX * WAVE,
+                         AT = AU + HALF * WAVE, SIZE = AT + HALF * WAVE;
+};
+template <class T, int N>
+__device__ __forceinline__ void load_rows(const T *m, int lane, T (&row)[N]) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) row[k] = m[k * WAVE + lane];
+}
+// sum_k row[k] v[k], v in LDS (entries past r: finite, or the row's are zero)
+template <class T, int N>
+__device__ __forceinline__ T dot_row(const T (&row)[N], const T *v) {
+    T s0 = T(0), s1 = T(0);
+#pragma unroll
+    for (int k = 0; k < N; k += 2) {
+        s0 = fmaT(row[k], v[k], s0);
+        s1 = fmaT(row[k + 1], v[k + 1], s1);
+    }
+    return s0 + s1;
+}
+
+// Upward pass, one workgroup per subtree of the input side. The subtree's
+// records and the matrix rows are read before they are needed (the pass is a
+// chain of latencies: a few leaves, the depths, the path).
+template <class T, int RMAX>
+struct UpLds {
+    alignas(16) T mom[N1_NODES][RMAX];
+    alignas(16) T pv[2][RMAX];
+    N1Node nodes[N1_NODES];
+    int32_t lev[N1_NODES + 1];
+};
+template <class T, int RMAX>
+__device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const T *x, int64_t incx,
+                                            const T *mats, T *partial, T *w, int r, int blk,
+                                            UpLds<T, RMAX> &L_) {
+    using Mt = N1Mat<T, RMAX>;
+    auto &mom = L_.mom;
+    auto &pv = L_.pv;
+    auto &nodes = L_.nodes;
+    auto &lev = L_.lev;
+    const N1Sub S = sload_struct(s.sub + blk);
+    const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
+    const int m = lane & 31, h = lane >> 5;
+    if ((int)threadIdx.x < S.nnode) nodes[threadIdx.x] = s.node[S.node + threadIdx.x];
+    if ((int)threadIdx.x <= S.nlev) lev[threadIdx.x] = s.lev[S.lev + threadIdx.x];
+    // the path, its nodes' records in the lanes (the last wavefront walks it)
+    int p_half = 0;
+    int64_t p_slot = -1;
+    if (wv == WPB - 1 && lane < min(S.npath, WAVE)) {
+        const N1Path P = s.path[S.path + S.npath - 1 - lane];
+        p_half = P.half;
+        p_slot = P.slot;
+    }
+    for (int e = wv; e < S.nleaf; e += WPB) {
+        const N1Leaf L = sload_struct(s.leaf + S.leaf + e);
+        const T cx = (T)L.cx, cy = (T)L.cy;
+        T acc[RMAX];
+#pragma unroll
+        for (int k = 0; k < RMAX; ++k) acc[k] = T(0);
+        for (int i = lane; i < L.len; i += WAVE) {
+            const T xv = x[(L.first + i) * incx];
+            const T xh = (pts[L.first + i] - cx) * cy;
+            const T x2 = xh + xh;
+            T t0 = xv, t1 = xh * xv;  // T_m(xh) x by the recurrence
+            acc[0] += t0;
+            acc[1] += t1;
+#pragma unroll
+            for (int k = 2; k < RMAX; ++k) {
+                const T t2 = fmaT(x2, t1, -t0);
+                acc[k] += t2;
+                t0 = t1;
+                t1 = t2;
+            }
+        }
+        int base = 0;
+        Halve<RMAX, WAVE / 2>::run(acc, lane, base);
+        constexpr int LEFT = HalveShape<RMAX, WAVE / 2>::left;
+        constexpr int MASK = HalveShape<RMAX, WAVE / 2>::mask;
+        if ((lane & MASK) == 0) {
+#pragma unroll
+            for (int i = 0; i < LEFT; ++i) mom[L.loc][base + i] = acc[i];
+        }
+    }
+    T Mr[RMAX];
+    load_rows(mats + Mt::MU, lane, Mr);
+    __syncthreads();
+    for (int l = S.nlev - 2; l >= 0; --l) {
+        const int nb = lev[l], ne = lev[l + 1];
+        for (int n = nb + wv; n < ne; n += WPB) {
+            const N1Node N = nodes[n];
+            if (N.c[0] < 0 && N.c[1] < 0) continue;  // a leaf (wave-uniform)
+            const int c = h ? N.c[1] : N.c[0];
+            T v = dot_row(Mr, mom[c >= 0 ? c : 0]);
+            if (c < 0) v = T(0);  // an empty half
+            v += __shfl_xor(v, 32);
+            if (h == 0 && m < RMAX) mom[n][m] = v;
+        }
+        __syncthreads();
+    }
+    // w of the clusters; the last wavefront walks the path meanwhile
+    if (wv < WPB - 1 || S.npath == 0) {
+        T Ar[Mt::HALF];
+        load_rows(mats + Mt::AU, lane, Ar);
+        const int step = S.npath == 0 ? WPB : WPB - 1;
+        for (int n = wv; n < S.nnode; n += step) {
+            const int cl = nodes[n].cl;
+            if (cl < 0) continue;
+            T v = dot_row(Ar, &mom[n][h * Mt::HALF]);
+            v += __shfl_xor(v, 32);
+            if (h == 0 && m < r) w[(int64_t)cl * r + m] = v;
+        }
+        return;
+    }
+    const T *cur = mom[0];
+    for (int e = 0; e < S.npath; ++e) {  // from the root's parent up
+        if (e > 0 && e % WAVE == 0) {
+            const int at = S.npath - 1 - e - lane;
+            if (at >= 0) {
+                const N1Path P = s.path[S.path + at];
+                p_half = P.half;
+                p_slot = P.slot;
+            }
+        }
+        const int64_t slot = rl_l(p_slot, e % WAVE);
+        T v = dot_row(Mr, cur);
+        if (h != rl_i(p_half, e % WAVE)) v = T(0);
+        v += __shfl_xor(v, 32);
+        T *nx = pv[e & 1];
+        if (h == 0 && m < RMAX) nx[m] = v;
+        if (slot >= 0 && h == 0 && m < r) partial[slot * r + m] = v;
+        wave_sync();
+        cur = nx;
+    }
+}
+
+// Translation: one wavefront per cluster of the output side whose sources all
+// lie in subtrees (a wavefront takes several in turn, the matrix rows kept);
+// the clusters with a source above them ("heavy", first in the target list)
+// take a workgroup, a source per wavefront. Lane (m, h) sums its row's half h
+// of the columns l. A cluster has at most about four sources; their node
+// values and nodes are staged four at a time in LDS with one round of loads.
+// F formed from the nodes: eight or four terms of 1/d^m share a reciprocal as
+// in the near field.
+template <class T, int RMAX>
+struct TrLds {
+    alignas(16) T sw[WPB][4][RMAX], st[WPB][4][RMAX];
+    alignas(16) T zr[WPB][RMAX];
+};
+template <class T, int RMAX, bool TRANS, int SRC, int KID>
+__device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N1Side &o, int blk,
+                                                   int nblk, const T *mats, const T *partial, const T *w,
+                                                   T *z, TrLds<T, RMAX> &L_) {
+    using Mt = N1Mat<T, RMAX>;
+    constexpr bool FREE = SRC != N1_READ;
+    constexpr int HALF = Mt::HALF, NB = 4, NT = HALF % 8 == 0 ? 8 : 4;
+    auto &sw = L_.sw;
+    auto &st = L_.st;
+    auto &zr = L_.zr;
+    const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
+    const int m = lane & 31, h = lane >> 5;
+    const int r = p.r;
+    const int mm = m < r ? m : 0;
+    const T *oth = TRANS ? p.rnodes : p.cnodes;
+    T At[HALF];
+    load_rows(mats + Mt::AT, lane, At);
+    T to = T(0), acc = T(0);
+    // ws: zero past r; ts: past r repeats
+    auto apply = [&](const T *ws, const T *ts, int64_t foff) {
+        if constexpr (FREE) {
+#pragma unroll
+            for (int j = 0; j < HALF; j += NT)
+                near_terms<T, KID, TRANS, SRC == N1_EXACT, NT, 1>(&to, ts + h * HALF + j, ws + h * HALF + j, &acc);
+        } else {
+            const T *F = p.F + foff;
+            T fv[HALF];
+#pragma unroll
+            for (int j = 0; j < HALF; ++j) {
+                const int l = min(h * HALF + j, r - 1);
+                fv[j] = __builtin_nontemporal_load(TRANS ? F + (l + r * mm) : F + (mm + r * l));
+            }
+#pragma unroll
+            for (int j = 0; j < HALF; ++j) {
+                const int l = h * HALF + j;
+                acc = fmaT(fv[j], ws[l], acc);  // ws is zero past r
+            }
+        }
+    };
+    auto finish = [&](int id, const T *zs) {  // c = A^T z
+        T c = dot_row(At, zs + h * HALF);
+        c += __shfl_xor(c, 32);
+        if (h == 0 && m < r) z[(int64_t)id * r + m] = c;
+    };
+    if (blk >= o.nheavy) {
+        const int step = (nblk - o.nheavy) * WPB;
+        for (int idx = o.nheavy + (blk - o.nheavy) * WPB + wv; idx < o.ncl; idx += step) {
+            const N1Target C = sload_struct(o.target + idx);
+            if constexpr (FREE) to = (TRANS ? p.cnodes : p.rnodes)[(int64_t)C.id * r + mm];
+            acc = T(0);
+            for (int e0 = C.beg; e0 < C.end; e0 += NB) {
+                const int ne = min(NB, C.end - e0);
+                // (source, column) = (i / RMAX, i % RMAX)
+#pragma unroll
+                for (int u = 0; u < (NB * RMAX + WAVE - 1) / WAVE; ++u) {
+                    const int i = lane + u * WAVE;
+                    const int e = i / RMAX, l = i - e * RMAX;
+                    if (e < ne) {
+                        const int64_t at = (int64_t)o.tr[e0 + e].src * r + min(l, r - 1);
+                        const T wl = w[at];
+                        sw[wv][e][l] = l < r ? wl : T(0);
+                        if constexpr (FREE) st[wv][e][l] = oth[at];
+                    }
+                }
+                wave_sync();
+                for (int e = 0; e < ne; ++e) apply(sw[wv][e], st[wv][e], FREE ? 0 : o.tr[e0 + e].foff);
+                wave_sync();
+            }
+            acc += __shfl_xor(acc, 32);
+            if (h == 0 && m < RMAX) zr[wv][m] = m < r ? acc : T(0);
+            wave_sync();
+            finish(C.id, zr[wv]);
+            wave_sync();
+        }
+        return;
+    }
+    const N1Target C = sload_struct(o.target + blk);
+    if constexpr (FREE) to = (TRANS ? p.cnodes : p.rnodes)[(int64_t)C.id * r + mm];
+    T Ar[HALF];
+    load_rows(mats + Mt::AU, lane, Ar);
+    for (int e = C.beg + wv; e < C.end; e += WPB) {
+        const DTrRec R = o.tr[e];
+        if (FREE && h == 0 && m < RMAX) st[wv][0][m] = oth[(int64_t)R.src * r + (m < r ? m : r - 1)];
+        if (R.nslots > 0) {
+            // lane half h sums the slots h, h + 2, ..., sixteen loads in flight
+            const T *ps = partial + R.pbase * r + mm;
+            T s = T(0);
+            int t = h;
+            for (; t + 30 < R.nslots; t += 32) {
+                T v[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) v[u] = ps[(int64_t)(t + 2 * u) * r];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) s += v[u];
+            }
+            for (; t < R.nslots; t += 2) s += ps[(int64_t)t * r];
+            s += __shfl_xor(s, 32);
+            if (h == 0 && m < RMAX) sw[wv][0][m] = m < r ? s : T(0);
+            wave_sync();
+            T v = dot_row(Ar, &sw[wv][0][h * HALF]);  // w = A mu
+            v += __shfl_xor(v, 32);
+            wave_sync();
+            if (h == 0 && m < RMAX) sw[wv][0][m] = v;
+        } else if (h == 0 && m < RMAX) {
+            const T wl = w[(int64_t)R.src * r + mm];
+            sw[wv][0][m] = m < r ? wl : T(0);
+        }
+        wave_sync();
+        apply(sw[wv][0], st[wv][0], R.foff);
+        wave_sync();
+    }
+    acc += __shfl_xor(acc, 32);
+    if (h == 0 && m < RMAX) zr[wv][m] = m < r ? acc : T(0);
+    __syncthreads();
+    if (wv != 0) return;
+    T s = T(0);
+    if (m < RMAX)
+        for (int u = 0; u < WPB; ++u) s += zr[u][m];
+    wave_sync();
+    if (h == 0 && m < RMAX) zr[0][m] = s;
+    wave_sync();
+    finish(C.id, zr[0]);
+}
+
+// The two launches of the far-field chain before the downward pass. Each also
+// takes about half of the near field's workgroups: the chain's are few and wait on
+// latencies, and the near field does not depend on them.
+//
+// The two kinds alternate in groups of 256 workgroups, one for each CU, the
+// chain's groups spread evenly among the near field's: with all of the chain's
+// first they filled the chip alone (n = 2^20: 63 us), and alternating one by
+// one or by eights, each kind met only half of the XCDs or of their shader
+// engines, over which consecutive workgroups are dealt (84 us). Group g is the
+// chain's number c(g) = floor(g n / total) if c(g + 1) > c(g), else the near
+// field's number g - c(g); numbers past a kind's count do nothing.
+constexpr int N1_GROUP = 256;
+inline int n1_grid(int chain, int near) {
+    return N1_GROUP * ((chain + N1_GROUP - 1) / N1_GROUP + (near + N1_GROUP - 1) / N1_GROUP);
+}
+__device__ __forceinline__ bool chain_block(int n, int &at) {
+    const int g = (int)blockIdx.x / N1_GROUP, total = (int)gridDim.x / N1_GROUP;
+    const int ng = (n + N1_GROUP - 1) / N1_GROUP;
+    const int c0 = g * ng / total, c1 = (g + 1) * ng / total;
+    at = N1_GROUP * (c1 > c0 ? c0 : g - c0) + (int)blockIdx.x % N1_GROUP;
+    return c1 > c0;
+}
+
+// Five wavefronts per SIMD are asked of the register allocator where the near
+// field is formed: left alone it gives four (upward) and three (translation);
+// six cost the near field's chains their registers (85 us).
+constexpr int n1_waves(int src, int kid) { return src != N1_READ && kid < 3 ? 5 : 1; }
+
+template <class T, int RMAX, int SRC, int KID, bool TR>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID))))
+void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *A, const T *mats,
+             MvArgsT<T> a, int r, int nup, int nb0, int nb) {
+    __shared__ union Lds {
+        UpLds<T, RMAX> up;
+        NearLds<T> near;
+        __device__ Lds() {}
+    } s;
+    int at;
+    if (chain_block(nup, at)) {
+        if (at < nup) n1_up_block<T, RMAX>(in, in_pts, a.x, a.incx, mats, a.partial, a.w, r, at, s.up);
+    } else if (at < nb) {
+        near_block<T, KID, TR, SRC>(out, at + nb0, out_pts, in_pts, A, a, s.near);
+    }
+}
+
+template <class T, int RMAX, int SRC, int KID, bool TR>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID))))
+void k_n1_translate(DevPlanT<T> p, N1Side out, const T *in_pts, const T *out_pts, MvArgsT<T> a,
+                    int ntr, int nb0, int nb) {
+    __shared__ union Lds {
+        TrLds<T, RMAX> tr;
+        NearLds<T> near;
+        __device__ Lds() {}
+    } s;
+    int at;
+    if (chain_block(ntr, at)) {
+        if (at < ntr)
+            n1_translate_block<T, RMAX, TR, SRC, KID>(p, out, at, ntr, p.n1m, a.partial, a.w, a.z, s.tr);
+    } else if (at < nb) {
+        near_block<T, KID, TR, SRC>(out, at + nb0, out_pts, in_pts, p.A, a, s.near);
+    }
+}
+
+// The coefficients of a subtree's nodes into cof (LDS): the path's, one node
+// after another, then each node's halves together (lane half h takes half h).
+// One wavefront; pz: its LDS, sixteen path nodes' z at a time (and the last
+// batch's final node in row N1_PATH); lane l holds local node l's record.
+template <class T, int RMAX>
+__device__ __forceinline__ void n1_coefficients(const N1Side &s, const N1Sub &S, const T *mats,
+                                                const T *z, int r, int lane, T (*cof)[RMAX],
+                                                T (*pz)[RMAX]) {
+    using Mt = N1Mat<T, RMAX>;
+    const int m = lane & 31, h = lane >> 5;
+    N1Node nd{-1, {-1, -1}};
+    N1Path P{-1, -1, 0};
+    if (lane < S.nnode) nd = s.node[S.node + lane];
+    if (lane < min(N1_PATH, S.npath)) P = s.path[S.path + lane];
+    T Mr[RMAX];
+    load_rows(mats + Mt::MD, lane, Mr);
+    // the nodes' own z
+    for (int i0 = 0; i0 < S.nnode * RMAX; i0 += WAVE) {
+        const int i = i0 + lane, n = i / RMAX, l = i - n * RMAX;
+        const int cl = __shfl(nd.cl, n < S.nnode ? n : 0);
+        if (n < S.nnode) cof[n][l] = (cl >= 0 && l < r) ? z[(int64_t)cl * r + l] : T(0);
+    }
+    int half = 0;
+    const T *cur = nullptr;
+    for (int e0 = 0; e0 < S.npath; e0 += N1_PATH) {
+        const int ne = min(N1_PATH, S.npath - e0);
+        if (cur) {
+            if (lane < ne) P = s.path[S.path + e0 + lane];
+            wave_sync();
+            if (h == 0 && m < RMAX) pz[N1_PATH][m] = cur[m];
+            cur = pz[N1_PATH];
+            wave_sync();
+        }
+#pragma unroll
+        for (int u = 0; u < N1_PATH * RMAX / WAVE; ++u) {
+            const int i = lane + u * WAVE, e = i / RMAX, l = i - e * RMAX;
+            const int cl = __shfl(P.cl, e);
+            if (e < ne) pz[e][l] = (cl >= 0 && l < r) ? z[(int64_t)cl * r + l] : T(0);
+        }
+        wave_sync();
+        for (int e = 0; e < ne; ++e) {
+            if (cur) {
+                T v = dot_row(Mr, cur);
+                if (h != half) v = T(0);
+                v += __shfl_xor(v, 32);
+                if (h == 0 && m < RMAX) pz[e][m] += v;
+                wave_sync();
+            }
+            cur = pz[e];
+            half = rl_i(P.half, e);
+        }
+    }
+    wave_sync();
+    if (cur) {
+        T v = dot_row(Mr, cur);
+        if (h != half) v = T(0);
+        v += __shfl_xor(v, 32);
+        if (h == 0 && m < RMAX) cof[0][m] += v;
+        wave_sync();
+    }
+    for (int n = 0; n < S.nnode; ++n) {
+        const int ca = rl_i(nd.c[0], n), cb = rl_i(nd.c[1], n);
+        if (ca < 0 && cb < 0) continue;  // a leaf (wave-uniform)
+        const int c = h ? cb : ca;
+        const T v = dot_row(Mr, cof[n]);
+        if (c >= 0 && m < RMAX) cof[c][m] += v;
+        wave_sync();
+    }
+}
+
+// One row of a chunk: the leaf's series by Clenshaw (coefficients in LDS, zero
+// past r)
+template <class T, int RMAX>
+__device__ __forceinline__ T n1_series(const N1Chunk &C, const T (*cof)[RMAX], T p) {
+    const T xh = (p - (T)C.cx) * (T)C.cy, x2 = xh + xh;
+    const T *ck = cof[C.leaf];
+    T b1 = T(0), b2 = T(0);
+#pragma unroll
+    for (int k = RMAX - 1; k >= 1; --k) {
+        const T b0 = fmaT(x2, b1, ck[k] - b2);
+        b2 = b1;
+        b1 = b0;
+    }
+    return fmaT(xh, b1, ck[0] - b2);
+}
+
+// Downward pass: the far field added onto y, which holds the near field. A
+// subtree per workgroup, its chunks over the wavefronts.
+template <class T, int RMAX>
+__global__ __launch_bounds__(WG) void k_n1_down(N1Side o, const T *pts_out, const T *z,
+                                               const T *mats, MvArgsT<T> a, int r) {
+    __shared__ __align__(16) T cof[N1_NODES][RMAX];
+    __shared__ __align__(16) T pz[N1_PATH + 1][RMAX];
+    const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
+    const N1Sub S = sload_struct(o.sub + blockIdx.x);
+    if (wv == WPB - 1) n1_coefficients<T, RMAX>(o, S, mats, z, r, lane, cof, pz);
+    __syncthreads();
+    for (int c = S.ch + wv; c < S.ch + S.nch; c += WPB) {
+        const N1Chunk C = sload_struct(o.ch + c);
+        const T po = pts_out[C.p0 + min(lane, C.np - 1)];
+        n1_write(C, a, 1, lane, n1_series<T, RMAX>(C, cof, po));
+    }
+}
+
+// One product y = beta*y + op(H) x of one right-hand side over the interval
+// trees. Many chunks of stored entries stream through k_down's near part, on
+// the side stream when there is one.
+template <class T, int RMAX, int SRC, int KID, bool TR>
+hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s,
+                       const hipEvent_t *ev) {
+    auto mark = [&](int q) {
+        if (ev) (void)hipEventRecord(ev[q], s);
+    };
+    const N1Side &in = TR ? p.n1x : p.n1y, &out = TR ? p.n1y : p.n1x;
+    const T *in_pts = TR ? p.x : p.y, *out_pts = TR ? p.y : p.x;
+    const bool far = p.nfar > 0;
+    const bool stream = SRC == N1_READ && out.nunit > 0;
+    const bool split = stream && a.side && !ev;
+    auto near_part = [&](hipStream_t ns) {
+        MvArgsT<T> an = a;
+        an.part = 1;
+        if constexpr (TR)
+            k_down<T, RMAX, false, 0, true, true, 1><<<nblk(p.ncch), WG, 0, ns>>>(
+                p, p.cch, p.ncch, p.cnear, p.cfar, p.ccl, p.V, p.cmap, p.y, p.x, a.z, an);
+        else
+            k_down<T, RMAX, false, 0, false, true, 1><<<nblk(p.nrch), WG, 0, ns>>>(
+                p, p.rch, p.nrch, p.rnear, p.rfar, p.rcl, p.U, p.rmap, p.x, p.y, a.z, an);
+    };
+    if (split) {
+        hipError_t e = hipEventRecord(a.fork, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(a.side, a.fork, 0);
+        if (e != hipSuccess) return e;
+        near_part(a.side);
+        e = hipEventRecord(a.join, a.side);
+        if (e != hipSuccess) return e;
+    }
+    // the near field's workgroups, five ninths with the upward pass, whose own
+    // work is the smaller (n = 2^20: 68 and 67 us at one half each)
+    const int nb = stream ? 0 : out.nunit > 0 ? (out.nunit + WPB - 1) / WPB : out.nch;
+    const int nb0 = far ? (5 * nb + 8) / 9 : nb;
+    const int nup = far ? in.nsub : 0;
+    mark(0);
+    if (nup + nb0 > 0)
+        k_n1_up<T, RMAX, SRC, KID, TR><<<n1_grid(nup, nb0), WG, 0, s>>>(
+            in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, nup, 0, nb0);
+    mark(1);
+    mark(2);
+    if (far) {
+        // light clusters: at most four wavefronts per SIMD, looping
+        const int ntr = out.nheavy + std::min((out.ncl - out.nheavy + WPB - 1) / WPB, 1024);
+        k_n1_translate<T, RMAX, SRC, KID, TR><<<n1_grid(ntr, nb - nb0), WG, 0, s>>>(
+            p, out, in_pts, out_pts, a, ntr, nb0, nb - nb0);
+    }
+    mark(3);
+    if (split) {
+        const hipError_t e = hipStreamWaitEvent(s, a.join, 0);
+        if (e != hipSuccess) return e;
+    } else if (stream) {
+        near_part(s);
+    }
+    if (far) k_n1_down<T, RMAX><<<out.nsub, WG, 0, s>>>(out, out_pts, a.z, p.n1m, a, p.r);
+    mark(4);
+    return hipGetLastError();
+}
+
+// src: N1_FREE, N1_EXACT (kernels 1/d^m) or N1_READ
+template <class T, int RMAX, bool TR>
+hipError_t matvec_n1_k(const DevPlanT<T> &p, const MvArgsT<T> &a, int src, hipStream_t s,
+                       const hipEvent_t *ev) {
+    if (src == N1_READ) return matvec_n1_t<T, RMAX, N1_READ, 0, TR>(p, a, s, ev);
+    if (src == N1_EXACT) {
+        switch (p.kid) {
+        case 0: return matvec_n1_t<T, RMAX, N1_EXACT, 0, TR>(p, a, s, ev);
+        case 1: return matvec_n1_t<T, RMAX, N1_EXACT, 1, TR>(p, a, s, ev);
+        default: return matvec_n1_t<T, RMAX, N1_EXACT, 2, TR>(p, a, s, ev);
+        }
+    }
+    switch (p.kid) {
+    case 0: return matvec_n1_t<T, RMAX, N1_FREE, 0, TR>(p, a, s, ev);
+    case 1: return matvec_n1_t<T, RMAX, N1_FREE, 1, TR>(p, a, s, ev);
+    case 2: return matvec_n1_t<T, RMAX, N1_FREE, 2, TR>(p, a, s, ev);
+    default: return matvec_n1_t<T, RMAX, N1_FREE, 3, TR>(p, a, s, ev);
+    }
+}
+
+template <class T, int RMAX>
+hipError_t matvec_n1(const DevPlanT<T> &p, const MvArgsT<T> &a, bool tr, int src, hipStream_t s,
+                     const hipEvent_t *ev) {
+    return tr ? matvec_n1_k<T, RMAX, true>(p, a, src, s, ev)
+              : matvec_n1_k<T, RMAX, false>(p, a, src, s, ev);
+}
+
+}  // namespace
+}  // namespace hmxk

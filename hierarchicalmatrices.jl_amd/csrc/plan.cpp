@@ -439,6 +439,244 @@ void both_sides(int64_t points, F f, G g) {
     if (thrown) std::rethrow_exception(thrown);
 }
 
+// One side's interval tree cut into subtrees (N1Side's tables).
+struct N1Host {
+    std::vector<N1Sub> sub;
+    std::vector<N1Node> node;
+    std::vector<int32_t> lev;
+    std::vector<N1Leaf> leaf;
+    std::vector<N1Path> path;
+    std::vector<N1Chunk> ch;
+    std::vector<N1Run> run;
+    std::vector<N1Unit> unit;
+    std::vector<N1UnitRun> urun;
+    std::vector<DTrRec> tr;
+    std::vector<N1Target> target;
+    int32_t nheavy = 0;
+    // per cluster: its first slot and slot count (0: inside a subtree)
+    std::vector<int64_t> sbase;
+    std::vector<int32_t> scount;
+    int64_t slots = 0;
+
+    // A subtree has at most N1_NODES nodes and GC chunks (or is one leaf).
+    // GC: 4 while a downward workgroup takes one chunk (its wavefronts share
+    // the path and the subtree with three others at most), else so that about
+    // 1024 to 2048 workgroups share the paths' work among their chunks.
+    bool cut(const std::vector<DTNode> &t, const Side &S, const std::vector<DDense> &dense,
+             bool rows, size_t ncl) {
+        const std::vector<DChunk> &dc = S.ch;
+        const int64_t nch = (int64_t)dc.size();
+        int32_t GC = 4;
+        if (nch > N1_SPLIT_CHUNKS)
+            while (GC < 32 && (int64_t)GC * 1024 < nch) GC *= 2;
+        const size_t nt = t.size();
+        std::vector<int32_t> nn(nt, 0), cb(nt, 0), cn(nt, 0);
+        for (size_t k = nt; k-- > 0;) {  // halves come after their parent
+            const DTNode &d = t[k];
+            if (d.len == 0) continue;
+            nn[k] = 1;
+            if (d.child[0] < 0) {
+                const size_t c = std::lower_bound(dc.begin(), dc.end(), d.first,
+                                                  [](const DChunk &a, int64_t v) { return a.p0 < v; }) -
+                                 dc.begin();
+                size_t e = c;
+                while (e < dc.size() && dc[e].p0 < d.first + d.len) {
+                    if (dc[e].p0 + dc[e].np > d.first + d.len) return false;
+                    ++e;
+                }
+                if (c == dc.size() || dc[c].p0 != d.first) return false;
+                cb[k] = (int32_t)c;
+                cn[k] = (int32_t)(e - c);
+            } else {
+                bool one = false;
+                for (int h = 0; h < 2; ++h) {
+                    const int32_t c = d.child[h];
+                    if (nn[c] == 0) continue;
+                    if (!one) cb[k] = cb[c];
+                    else if (cb[c] != cb[k] + cn[k]) return false;
+                    one = true;
+                    nn[k] += nn[c];
+                    cn[k] += cn[c];
+                }
+                if (!one) return false;
+            }
+        }
+        sbase.assign(ncl, 0);
+        scount.assign(ncl, 0);
+        ch.resize(dc.size());
+        std::vector<int32_t> pcount(nt, 0), pathnodes, queue;
+        std::vector<std::pair<int32_t, int32_t>> stack;  // (node, path length above it)
+        std::vector<int32_t> cur;                        // the path to the node at hand
+        size_t covered = 0;
+        for (size_t root = 0; root < nt; ++root) {
+            if (t[root].parent >= 0 || t[root].len == 0) continue;
+            stack.push_back({(int32_t)root, 0});
+            while (!stack.empty()) {
+                const auto [k, above] = stack.back();
+                stack.pop_back();
+                cur.resize(above);
+                const DTNode &d = t[k];
+                const bool is_leaf = d.child[0] < 0;
+                if (!(nn[k] <= N1_NODES && (cn[k] <= GC || is_leaf))) {
+                    cur.push_back(k);
+                    for (int h = 1; h >= 0; --h)
+                        if (nn[d.child[h]] > 0) stack.push_back({d.child[h], above + 1});
+                    continue;
+                }
+                N1Sub u{};
+                u.path = (int32_t)pathnodes.size();
+                u.npath = above;
+                for (int32_t q : cur) {
+                    pathnodes.push_back(q);
+                    ++pcount[q];
+                }
+                pathnodes.push_back(k);  // the node below the last path node
+                u.node = (int32_t)node.size();
+                u.lev = (int32_t)lev.size();
+                u.leaf = (int32_t)leaf.size();
+                u.ch = cb[k];
+                u.nch = cn[k];
+                queue.assign(1, k);
+                size_t at = 0, end = 1;
+                while (at < end) {  // one depth at a time
+                    lev.push_back((int32_t)at);
+                    for (; at < end; ++at) {
+                        const DTNode &q = t[queue[at]];
+                        N1Node g{q.cl, {-1, -1}};
+                        if (q.child[0] < 0) {
+                            leaf.push_back({q.first, q.len, (int32_t)at, q.cx, q.cy});
+                            for (int32_t c = cb[queue[at]]; c < cb[queue[at]] + cn[queue[at]]; ++c) {
+                                N1Chunk &w = ch[c];
+                                w.p0 = dc[c].p0;
+                                w.np = dc[c].np;
+                                w.leaf = (int32_t)at;
+                                w.sub = (int32_t)sub.size();
+                                w.cx = q.cx;
+                                w.cy = q.cy;
+                                ++covered;
+                            }
+                        } else {
+                            for (int h = 0; h < 2; ++h)
+                                if (nn[q.child[h]] > 0) {
+                                    g.c[h] = (int32_t)queue.size();
+                                    queue.push_back(q.child[h]);
+                                }
+                        }
+                        node.push_back(g);
+                    }
+                    end = queue.size();
+                }
+                lev.push_back((int32_t)end);
+                u.nnode = (int32_t)end;
+                u.nlev = (int32_t)lev.size() - 1 - u.lev;
+                u.nleaf = (int32_t)leaf.size() - u.leaf;
+                sub.push_back(u);
+            }
+        }
+        if (covered != dc.size()) return false;
+        // slots: a node's subtrees consecutive, in the order they were cut
+        std::vector<int64_t> nextslot(nt, -1);
+        for (size_t k = 0; k < nt; ++k) {
+            if (pcount[k] == 0 || t[k].cl < 0) continue;
+            nextslot[k] = slots;
+            sbase[t[k].cl] = slots;
+            scount[t[k].cl] = pcount[k];
+            slots += pcount[k];
+        }
+        path.reserve(pathnodes.size());
+        size_t pos = 0;
+        for (N1Sub &u : sub) {
+            u.path = (int32_t)path.size();
+            for (int32_t e = 0; e < u.npath; ++e) {
+                const int32_t q = pathnodes[pos + e], below = pathnodes[pos + e + 1];
+                path.push_back({nextslot[q] >= 0 ? nextslot[q]++ : -1, t[q].cl, t[below].half});
+            }
+            pos += (size_t)u.npath + 1;
+        }
+        if (nch <= N1_SPLIT_CHUNKS) {
+            for (int64_t c = 0; c < nch; ++c) {
+                ch[c].run = (int32_t)run.size();
+                ch[c].nrun = dc[c].near_end - dc[c].near_beg;
+                for (int32_t e = dc[c].near_beg; e < dc[c].near_end; ++e) {
+                    const DNear &N = S.near[e];
+                    const DDense &D = dense[N.blk];
+                    run.push_back(rows ? N1Run{D.col0, D.aoff, D.n, N.off, D.n, 0}
+                                       : N1Run{D.row0, D.aoff, D.m, N.off, D.n, 0});
+                }
+            }
+            return true;
+        }
+        // the columns of a chunk's dense blocks as runs, adjacent ones joined;
+        // its list holds them in ascending order (the tree rule visits a row's
+        // blocks from the upper interval end down, a column's likewise), the
+        // order in which k_down sums the stored entries
+        auto runs_of = [&](int64_t c, std::vector<N1UnitRun> &o) {
+            o.clear();
+            for (int32_t e = dc[c].near_beg; e < dc[c].near_end; ++e) {
+                const DDense &D = dense[S.near[e].blk];
+                const N1UnitRun q = rows ? N1UnitRun{D.col0, D.n, 0} : N1UnitRun{D.row0, D.m, 0};
+                if (!o.empty() && o.back().q0 + o.back().n > q.q0) return false;
+                if (!o.empty() && o.back().q0 + o.back().n == q.q0) o.back().n += q.n;
+                else o.push_back(q);
+            }
+            return true;
+        };
+        std::vector<N1UnitRun> ra, rb;
+        for (N1Sub &u : sub) {
+            u.unit = (int32_t)unit.size();
+            for (int32_t c = u.ch; c < u.ch + u.nch; c += 2) {
+                N1Unit w{c, std::min(2, u.ch + u.nch - c), (int32_t)urun.size(), 0};
+                rb.clear();
+                if (!runs_of(c, ra) || (w.nch == 2 && !runs_of(c + 1, rb))) return false;
+                // the union of both, cut where the set of chunks served changes
+                size_t ia = 0, ib = 0;
+                int64_t at = 0;
+                while (ia < ra.size() || ib < rb.size()) {
+                    const int64_t a0 = ia < ra.size() ? std::max(at, ra[ia].q0) : INT64_MAX;
+                    const int64_t b0 = ib < rb.size() ? std::max(at, rb[ib].q0) : INT64_MAX;
+                    const int64_t q0 = std::min(a0, b0);
+                    const int mask = (a0 == q0 ? 1 : 0) | (b0 == q0 ? 2 : 0);
+                    int64_t end = INT64_MAX;
+                    if (mask & 1) end = std::min(end, ra[ia].q0 + ra[ia].n);
+                    else end = std::min(end, a0);
+                    if (mask & 2) end = std::min(end, rb[ib].q0 + rb[ib].n);
+                    else end = std::min(end, b0);
+                    urun.push_back({q0, (int32_t)(end - q0), mask});
+                    ++w.nrun;
+                    at = end;
+                    if (ia < ra.size() && ra[ia].q0 + ra[ia].n <= at) ++ia;
+                    if (ib < rb.size() && rb[ib].q0 + rb[ib].n <= at) ++ib;
+                }
+                unit.push_back(w);
+            }
+            u.nunit = (int32_t)unit.size() - u.unit;
+        }
+        return true;
+    }
+
+    // as output side, with the other side's slots: the translation records in
+    // this side's far-list order and the clusters, those with a source above
+    // the subtrees first
+    void targets(const std::vector<DCluster> &cl, const std::vector<int32_t> &list,
+                 const std::vector<DFarBlk> &far, bool rows, const N1Host &src) {
+        tr.resize(list.size());
+        for (size_t e = 0; e < list.size(); ++e) {
+            const DFarBlk &b = far[list[e]];
+            const int32_t q = rows ? b.cc : b.rc;
+            tr[e] = DTrRec{b.foff, src.sbase[q], q, src.scount[q]};
+        }
+        for (int pass = 0; pass < 2; ++pass) {
+            for (size_t k = 0; k < cl.size(); ++k) {
+                bool heavy = false;
+                for (int32_t e = cl[k].far_beg; e < cl[k].far_end; ++e) heavy |= tr[e].nslots > 0;
+                if (heavy == (pass == 0))
+                    target.push_back({(int32_t)k, cl[k].far_beg, cl[k].far_end});
+            }
+            if (pass == 0) nheavy = (int32_t)target.size();
+        }
+    }
+};
+
 template <class T>
 int upload(T **dst, const std::vector<T> &src) {
     *dst = nullptr;
@@ -541,6 +779,7 @@ struct PlanBufs {
     // nested far field of the MFMA passes (Float64 plans): the re-expansion
     // matrices, moments per column node, coefficients per row node
     T *nestM = nullptr, *my = nullptr, *mx = nullptr;
+    T *n1m = nullptr;  // padded matrices of the single-right-hand-side tree passes
     // x .. chebA and the workspace partial .. xt live in this one allocation
     // (Staging); A, U, V and F are one allocation (factors) in plans from
     // points, and allocated on their own in plans from blocks
@@ -607,6 +846,16 @@ struct hm_plan {
     DTNode *d_xtn = nullptr, *d_ytn = nullptr;
     int32_t *d_xlev = nullptr, *d_ylev = nullptr, *d_chunk_leaf = nullptr;
     DTask *d_yleaf = nullptr;
+    // one right-hand side over the interval trees (nested1.h): both sides'
+    // tables; regen: a stored or hybrid plan's dense entries and F may be
+    // formed from the points and nodes instead of read; refit: the points were
+    // replaced after that was decided; uv_finite: U and V hold finite values
+    // alone, as far as uv_known says (the device's word after a refit);
+    // uv_replayed: a graph holds a refit, whose replays are not seen here
+    bool n1 = false, regen = false, refit = false, uv_finite = true, uv_known = true,
+         uv_replayed = false;
+    N1Host n1x, n1y;
+    N1Side d_n1x{}, d_n1y{};
     void *d_tables = nullptr;  // the one allocation holding d_rcl .. d_yleaf (Staging)
     // side stream and fork / join events of products whose near field runs
     // beside the far-field chain; made at the first such product that is not
@@ -623,6 +872,7 @@ struct hm_plan {
     std::vector<DSplit> xsplits, ysplits;
     DSplit *d_xsplits = nullptr, *d_ysplits = nullptr;
     int32_t *d_status = nullptr;  // the plan's own status word (in d_tables)
+    int32_t *d_uv_bad = nullptr;  // a value of U or V is not finite (in d_tables)
     int max_kb = HM_MAX_KB;  // right-hand sides per forward launch (1, 2, 4 or 8)
     int tuned_kb = HM_MAX_KB, tuned_mode = -1;  // hm_plan_tune's choice
     std::vector<hipEvent_t> prof_events;  // 5 per product
@@ -675,52 +925,78 @@ struct hm_plan {
         dp.nylev = ylev_off.empty() ? 0 : (int32_t)ylev_off.size() - 1;
         dp.chunk_leaf = d_chunk_leaf;
         dp.yleaf = d_yleaf; dp.nyleaf = (int32_t)yleaf.size();
+        dp.n1 = n1 ? 1 : 0;
+        dp.n1x = d_n1x;
+        dp.n1y = d_n1y;
+    }
+
+    // The interval trees as device nodes; false unless every half is half of
+    // its parent's interval to the rounding of the interval ends. Float64
+    // ends are rounded to eps |end|, which is eps |end| / halfwidth in the
+    // node's variable (7e-12 at depth 14 of [0, 1]; the mapped nodes behind F
+    // carry the same). Float32 trees nest where the midpoints are exact.
+    template <class TN>
+    bool tree_nodes(const std::vector<TN> &t, std::vector<DTNode> &o) const {
+        o.resize(t.size());
+        for (size_t k = 0; k < t.size(); ++k) {
+            const TN &q = t[k];
+            DTNode d{};
+            d.first = q.first;
+            d.len = (int32_t)q.len;
+            d.parent = q.parent;
+            d.child[0] = q.child[0];
+            d.child[1] = q.child[1];
+            d.cl = q.cl;
+            d.half = q.half;
+            d.cx = 0.5 * (q.lo + q.hi);
+            d.cy = 1.0 / (0.5 * (q.hi - q.lo));
+            o[k] = d;
+        }
+        for (size_t k = 0; k < t.size(); ++k) {
+            const DTNode &d = o[k];
+            if ((d.child[0] < 0) != (d.child[1] < 0) || !std::isfinite(d.cy)) return false;
+            if (d.parent < 0) continue;
+            const DTNode &P = o[d.parent];
+            const double alpha = P.cy / d.cy, beta = (d.cx - P.cx) * P.cy;
+            const double end = std::max(std::fabs(t[k].lo), std::fabs(t[k].hi));
+            const double tol = std::max(1e-12, std::min(1e-10, 4.0 * 0x1p-52 * end * std::fabs(d.cy)));
+            if (!(std::fabs(alpha - 0.5) <= tol) ||
+                !(std::fabs(beta - (d.half ? 0.5 : -0.5)) <= tol))
+                return false;
+        }
+        return true;
+    }
+
+    // Tables of the single-right-hand-side tree passes; n1 stays false (the
+    // per-level passes are used) where the trees do not nest, a chunk lies in
+    // several leaves, or the rank exceeds 32 (a wavefront's two halves hold a
+    // matrix row per lane).
+    template <class TN>
+    void build_n1(const std::vector<TN> &xt, const std::vector<TN> &yt,
+                  const std::vector<int32_t> &by_rc, const std::vector<int32_t> &by_cc) {
+        n1 = false;
+        if (r > 32 || xt.empty() || yt.empty()) return;
+        std::vector<DTNode> xs, ys;
+        if (!nest && (!tree_nodes(xt, xs) || !tree_nodes(yt, ys))) return;
+        bool okx = false, oky = false;
+        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, rows, dense, true, rcl.size()); },
+                   [&] { oky = n1y.cut(nest ? ytn : ys, cols, dense, false, ccl.size()); });
+        if (!okx || !oky) return;
+        n1x.targets(rcl, by_rc, far, true, n1y);
+        n1y.targets(ccl, by_cc, far, false, n1x);
+        n1 = true;
     }
 
     // The nested far field's tables from the builder's interval trees; nest
-    // stays false (the per-level far field is used) unless every half is
-    // half of its parent's interval to the rounding of the interval ends,
-    // every column leaf fits one upward task and every row chunk lies in one
-    // row leaf. (To a fixed 1e-12, the log kernel's 2^22 random points fell
-    // back to the per-level form by their deepest intervals' rounding.)
+    // stays false (the per-level far field is used) unless the trees nest
+    // (tree_nodes; to a fixed 1e-12 the log kernel's 2^22 random points fell
+    // back by their deepest intervals' rounding), every column leaf fits one
+    // upward task and every row chunk lies in one row leaf.
     template <class TN>
     void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt) {
         nest = false;
         if (f32 || xt.empty() || yt.empty()) return;
-        auto conv = [](const std::vector<TN> &t, std::vector<DTNode> &o) {
-            o.resize(t.size());
-            for (size_t k = 0; k < t.size(); ++k) {
-                const TN &q = t[k];
-                DTNode d{};
-                d.first = q.first;
-                d.len = (int32_t)q.len;
-                d.parent = q.parent;
-                d.child[0] = q.child[0];
-                d.child[1] = q.child[1];
-                d.cl = q.cl;
-                d.half = q.half;
-                d.cx = 0.5 * (q.lo + q.hi);
-                d.cy = 1.0 / (0.5 * (q.hi - q.lo));
-                o[k] = d;
-            }
-            for (size_t k = 0; k < t.size(); ++k) {
-                const DTNode &d = o[k];
-                if ((d.child[0] < 0) != (d.child[1] < 0) || !std::isfinite(d.cy)) return false;
-                if (d.parent < 0) continue;
-                const DTNode &P = o[d.parent];
-                const double alpha = P.cy / d.cy, beta = (d.cx - P.cx) * P.cy;
-                // interval ends and centers are rounded to eps |end|, which
-                // is eps |end| / halfwidth in the node's variable (7e-12 at
-                // depth 14 of [0, 1]; the mapped nodes behind F carry the same)
-                const double end = std::max(std::fabs(t[k].lo), std::fabs(t[k].hi));
-                const double tol = std::max(1e-12, std::min(1e-10, 4.0 * 0x1p-52 * end * std::fabs(d.cy)));
-                if (!(std::fabs(alpha - 0.5) <= tol) ||
-                    !(std::fabs(beta - (d.half ? 0.5 : -0.5)) <= tol))
-                    return false;
-            }
-            return true;
-        };
-        if (!conv(xt, xtn) || !conv(yt, ytn)) return;
+        if (!tree_nodes(xt, xtn) || !tree_nodes(yt, ytn)) return;
         auto by_depth = [](const std::vector<TN> &t, bool internal_only, std::vector<int32_t> &ids,
                            std::vector<int32_t> &off) {
             int maxd = 0;
@@ -912,6 +1188,33 @@ std::vector<T> nest_matrices(int r) {
 }
 }  // extern "C++"
 
+// The matrices of the single-right-hand-side tree passes, laid out for lanes
+// (m, h) = (lane % 32, lane / 32) and padded with zeros to the rank bucket
+// (N1Mat): M_h[m][k], M_h[k][m], A[m][h R/2 + j], A[h R/2 + j][m].
+extern "C++" {
+template <class T>
+std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> &A) {
+    const int R = r <= 8 ? 8 : r <= 16 ? 16 : (r <= 24 && std::is_same_v<T, double>) ? 24 : 32;
+    const int HALF = R / 2;
+    std::vector<T> out((size_t)(2 * R + 2 * HALF) * 64, T(0));
+    T *MU = out.data(), *MD = MU + (size_t)R * 64, *AU = MD + (size_t)R * 64,
+      *AT = AU + (size_t)HALF * 64;
+    for (int lane = 0; lane < 64; ++lane) {
+        const int m = lane % 32, h = lane / 32;
+        if (m >= r) continue;
+        for (int k = 0; k < r; ++k) {
+            MU[k * 64 + lane] = M[((size_t)h * r + m) * r + k];
+            MD[k * 64 + lane] = M[((size_t)h * r + k) * r + m];
+        }
+        for (int j = 0; j < HALF && h * HALF + j < r; ++j) {
+            AU[j * 64 + lane] = A[(size_t)m * r + h * HALF + j];
+            AT[j * 64 + lane] = A[(size_t)(h * HALF + j) * r + m];
+        }
+    }
+    return out;
+}
+}  // extern "C++"
+
 // The element-typed part of a plan: nodes, weights, cluster maps and the
 // Chebyshev-form matrix in T, the device arrays, the device view, and the
 // compression (dense blocks, F, U, V) for stored and hybrid plans.
@@ -956,8 +1259,9 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
                     (T)((m ? 2.0L : 1.0L) * cosl((long double)m * (2 * k - 1) * PI_L / (2.0L * r)) / r);
     }
     const std::vector<T> xv(x, x + P->nx), yv(y, y + P->ny);
-    std::vector<T> nestM;
-    if (std::is_same_v<T, double> && P->nest) nestM = nest_matrices<T>(r);
+    std::vector<T> nestM, n1m;
+    if ((std::is_same_v<T, double> && P->nest) || P->n1) nestM = nest_matrices<T>(r);
+    if (P->n1) n1m = n1_matrices<T>(r, nestM, chebA);
     int rc;
 #define HM_TRY_T(expr) do { rc = (expr); if (rc != HM_OK) return rc; } while (0)
     const int64_t nslots = std::max(P->rows.nslots, P->cols.nslots);
@@ -977,7 +1281,8 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
             st.reserve(&b.my, (int64_t)P->ytn.size() * r * HM_WS_RHS);
             st.reserve(&b.mx, (int64_t)P->xtn.size() * r * HM_WS_RHS);
         }
-        st.reserve(&b.partial, nslots * r * HM_WS_RHS);
+        if (P->n1) st.add(&b.n1m, n1m);
+        st.reserve(&b.partial, std::max(nslots * HM_WS_RHS, std::max(P->n1x.slots, P->n1y.slots)) * r);
         st.reserve(&b.w, ncl * r * HM_WS_RHS);
         st.reserve(&b.z, ncl * r * HM_WS_RHS);
         if (std::is_same_v<T, double>) st.reserve(&b.xt, P->ny * HM_WS_RHS);
@@ -1009,8 +1314,9 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     dp.x = b.x; dp.y = b.y; dp.lam = b.lam;
     dp.rnodes = b.rnodes; dp.cnodes = b.cnodes;
     dp.rmap = b.rmap; dp.cmap = b.cmap; dp.chebA = b.chebA;
-    dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx;
+    dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx; dp.n1m = b.n1m;
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
+    dp.uv_bad = P->d_uv_bad;
 
     if (stored) {
         const bool user = P->kid == HM_USER;  // A and F come from hm_plan_set_leaf_data
@@ -1033,10 +1339,29 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (e == hipSuccess)
             e = hipMemcpyAsync(h.data(), b.cnt, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
-        int64_t total = 0;
-        for (auto v : h) total += (int64_t)v;
-        P->nonfinite = total;
-        P->nonfinite_basis = total;
+        int64_t bad[4] = {0, 0, 0, 0}, big[4] = {0, 0, 0, 0};
+        for (int q = 0; q < 4; ++q)
+            for (int k = 0; k < HM_COUNT_BLOCKS; ++k) {
+                bad[q] += (int64_t)(h[q * HM_COUNT_BLOCKS + k] & 0xffffffffull);
+                big[q] += (int64_t)(h[q * HM_COUNT_BLOCKS + k] >> 32);
+            }
+        P->nonfinite = bad[0] + bad[1] + bad[2] + bad[3];
+        P->nonfinite_basis = P->nonfinite;
+        P->uv_finite = bad[1] + bad[2] == 0;
+        // A product may form the entries of 1/d^m itself: one reciprocal costs
+        // a few vector instructions where an entry costs 8 bytes of HBM (stored
+        // n = 2^20, rank 24: 402 M entries, 3.2 GB). The values are the stored
+        // ones while they and d^m stay in the normal range; the log kernel's
+        // and the caller's own entries are read.
+        double span = 0.0;
+        for (size_t t = 0; t + 1 < P->row_off.size(); ++t) {
+            const double xh = x[P->row_off[t]], xl = x[P->row_off[t + 1] - 1];
+            const double yh = y[P->col_off[t]], yl = y[P->col_off[t + 1] - 1];
+            span = std::max({span, std::fabs(xh - yl), std::fabs(yh - xl)});
+        }
+        const bool power = P->kid == HM_CAUCHY || P->kid == HM_COULOMB || P->kid == HM_COULOMB3;
+        const double top = std::is_same_v<T, double> ? 1e100 : 1e12;
+        P->regen = power && span < top && bad[0] + big[0] + bad[3] + big[3] == 0;
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression: %s", hipGetErrorString(e));
     }
     hipError_t e = hipStreamSynchronize(s);
@@ -1216,6 +1541,7 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
                [&] { build_side(ny, P->dense, false, P->ccl, P->cols); });
     P->list_multi();
     P->build_nest(B.xt, B.yt);
+    P->build_n1(B.xt, B.yt, by_rc, by_cc);
     // the cluster maps the Float64 MFMA upward pass reads from its task
     // record: (a+b)/2 and 1/((b-a)/2) as the Float64 cluster maps form them
     if (!f32) {
@@ -1270,8 +1596,37 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
         st.add(&P->d_yleaf, P->yleaf);
         st.add(&P->d_xsplits, P->xsplits);
         st.add(&P->d_ysplits, P->ysplits);
+        auto add_n1 = [&](N1Side &d, N1Host &h) {
+            st.add(const_cast<N1Sub **>(&d.sub), h.sub);
+            st.add(const_cast<N1Node **>(&d.node), h.node);
+            st.add(const_cast<int32_t **>(&d.lev), h.lev);
+            st.add(const_cast<N1Leaf **>(&d.leaf), h.leaf);
+            st.add(const_cast<N1Path **>(&d.path), h.path);
+            st.add(const_cast<N1Chunk **>(&d.ch), h.ch);
+            st.add(const_cast<N1Run **>(&d.run), h.run);
+            st.add(const_cast<N1UnitRun **>(&d.urun), h.urun);
+            st.add(const_cast<N1Unit **>(&d.unit), h.unit);
+            st.add(const_cast<DTrRec **>(&d.tr), h.tr);
+            st.add(const_cast<N1Target **>(&d.target), h.target);
+            d.nsub = (int32_t)h.sub.size();
+            d.nunit = (int32_t)h.unit.size();
+            d.nch = (int32_t)h.ch.size();
+            d.ncl = (int32_t)h.target.size();
+            d.nheavy = h.nheavy;
+        };
+        if (P->n1) {
+            add_n1(P->d_n1x, P->n1x);
+            add_n1(P->d_n1y, P->n1y);
+        }
         st.reserve(&P->d_status, 1);
+        st.reserve(&P->d_uv_bad, 1);
         HM_TRY(st.commit(&P->d_tables));
+        // the device holds these now
+        const int64_t sx = P->n1x.slots, sy = P->n1y.slots;
+        P->n1x = N1Host{};
+        P->n1y = N1Host{};
+        P->n1x.slots = sx;
+        P->n1y.slots = sy;
     }
     P->far_by_rc_h = std::move(by_rc);
     if (f32) HM_TRY(setup_typed<float>(P, x, y, B.rcl, B.ccl, flags, nA, nU, nV, nF, (hipStream_t)stream));
@@ -1467,6 +1822,7 @@ static int from_blocks_t(int64_t nrows, int64_t ncols, int64_t nleaves, const in
     DevPlanT<T> &dp = b.dp;
     P->fill_structure(dp);
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
+    dp.uv_bad = P->d_uv_bad;
     (void)stream;
     *out = P;
     return HM_OK;
@@ -1564,6 +1920,15 @@ static int update_points_t(hm_plan_t P, const T *x, const T *y, int32_t *status,
     // the factors that depend on the points (dense blocks; U and V of stored
     // plans) are formed again; F depends on the intervals alone
     if (e == hipSuccess && !(P->flags & HM_PLAN_MATRIX_FREE)) e = hmx_launch_refit(b.dp, s);
+    P->refit = true;  // whether the new factors are finite is not known here
+    if (b.U || b.V) {
+        P->uv_known = false;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            P->uv_replayed = true;
+        }
+    }
     if (e != hipSuccess) return fail(HM_ERR_HIP, "update_points launch: %s", hipGetErrorString(e));
     return HM_OK;
 }
@@ -1789,6 +2154,26 @@ static bool split_near_field(hm_plan_t P, hipStream_t s) {
     return true;
 }
 
+// Whether a stored plan's U and V are finite. After new points the device
+// knows; its word is read back once, except on a stream that is being captured
+// (no: that product then reads U and V, as any plan with such values).
+static bool basis_finite(hm_plan_t P, hipStream_t s) {
+    if (P->uv_replayed) return false;
+    if (!P->uv_known) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        int32_t bad = 1;
+        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
+            hipMemcpyAsync(&bad, P->d_uv_bad, sizeof(bad), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        P->uv_finite = bad == 0;
+        P->uv_known = true;
+    }
+    return P->uv_finite;
+}
+
 template <class T>
 static MvArgsT<T> ws_args(hm_plan_t P) {
     MvArgsT<T> a{};
@@ -1891,6 +2276,12 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
             a.fork = P->fork;
             a.join = P->join;
         }
+        // one right-hand side over the interval trees. A stored plan's U and V
+        // equal the Chebyshev form's basis up to rounding unless a node meets
+        // a point (non-finite entries then keep the stored form)
+        bool n1 = P->n1 && kb == 1;
+        if (n1 && mode == 0) n1 = basis_finite(P, s);
+        const int src = mode == 2 ? N1_FREE : P->regen && !P->refit ? N1_EXACT : N1_READ;
         const hipEvent_t *ev = nullptr;
         if (P->profile) {
             const size_t at = P->prof_events.size();
@@ -1901,7 +2292,8 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
             }
             ev = P->prof_events.data() + at;
         }
-        hipError_t e = hmx_launch_matvec(P->bufs<T>().dp, a, tr, mode, kb, s, ev);
+        hipError_t e = n1 ? hmx_launch_matvec_n1(P->bufs<T>().dp, a, tr, src, s, ev)
+                          : hmx_launch_matvec(P->bufs<T>().dp, a, tr, mode, kb, s, ev);
         if (e != hipSuccess) return fail(HM_ERR_HIP, "matvec launch: %s", hipGetErrorString(e));
         q += kb;
     }
