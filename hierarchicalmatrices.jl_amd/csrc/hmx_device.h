@@ -142,12 +142,12 @@ hipError_t hmx_launch_matvec(const DevPlan &p, const MvArgs &a, bool transpose, 
 // dense blocks, 2 regenerates them.
 hipError_t hmx_launch_matvec_m(const DevPlan &p, const MvArgs &a, int mode, int prec, int nq,
                                hipStream_t s);
-// one product of one right-hand side over the interval trees (p.n1, r <= 32);
-// src: N1_FREE, N1_EXACT or N1_READ. Pass events as hmx_launch_matvec's (no
+// one product of nq <= N1_KB right-hand sides over the interval trees (p.n1,
+// r <= 32); src: N1_FREE, N1_EXACT or N1_READ. Pass events as hmx_launch_matvec's (no
 // reduce).
-hipError_t hmx_launch_matvec_n1(const DevPlan &p, const MvArgs &a, bool transpose, int src,
+hipError_t hmx_launch_matvec_n1(const DevPlan &p, const MvArgs &a, bool transpose, int src, int nq,
                                 hipStream_t s, const hipEvent_t *ev);
-hipError_t hmx_launch_matvec_n1(const DevPlanF &p, const MvArgsF &a, bool transpose, int src,
+hipError_t hmx_launch_matvec_n1(const DevPlanF &p, const MvArgsF &a, bool transpose, int src, int nq,
                                 hipStream_t s, const hipEvent_t *ev);
 // gradients (matrix-free near field, Chebyshev-form far field):
 //   forward (tr = false): y = beta*y + s .* (d/dx_i of (H x)_i)

@@ -136,8 +136,9 @@ struct DSplit {
 // workgroup (nested1.h). Node numbers inside a subtree are local: breadth
 // first from its root 0, so a depth's nodes are consecutive and every node
 // precedes its halves.
-#define N1_NODES 63          // nodes per subtree (LDS: one rank vector each)
+#define N1_NODES 47          // nodes per subtree (LDS: a rank vector each, N1_KB of them)
 #define N1_PATH 16           // path nodes staged together
+#define N1_KB 4              // right-hand sides per launch
 #define N1_SPLIT_CHUNKS 4096 // a downward workgroup per chunk up to this many chunks
 
 struct N1Sub {

@@ -15,6 +15,7 @@ hipError_t hmx_gen_basis_f32_r8(const DevPlanF &p, hipStream_t s) {
     return hmxk::gen_basis_r<float, 8>(p, s);
 }
 
-hipError_t hmx_matvec_n1_f32_r8(const DevPlanF &p, const MvArgsF &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
-    return hmxk::matvec_n1<float, 8>(p, a, tr, src, s, ev);
+hipError_t hmx_matvec_n1_f32_r8(const DevPlanF &p, const MvArgsF &a, bool tr, int src, int nq,
+                           hipStream_t s, const hipEvent_t *ev) {
+    return hmxk::matvec_n1<float, 8>(p, a, tr, src, nq, s, ev);
 }

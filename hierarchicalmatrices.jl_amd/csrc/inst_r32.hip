@@ -18,6 +18,7 @@ hipError_t hmx_matvec_m_r32(const DevPlan &p, const MvArgs &a, int mode, int pre
     return hmxk::matvec_m_r<32>(p, a, mode, prec, nq, s);
 }
 
-hipError_t hmx_matvec_n1_r32(const DevPlan &p, const MvArgs &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
-    return hmxk::matvec_n1<double, 32>(p, a, tr, src, s, ev);
+hipError_t hmx_matvec_n1_r32(const DevPlan &p, const MvArgs &a, bool tr, int src, int nq,
+                           hipStream_t s, const hipEvent_t *ev) {
+    return hmxk::matvec_n1<double, 32>(p, a, tr, src, nq, s, ev);
 }

@@ -31,11 +31,12 @@ hipError_t hmx_launch_matvec(const DevPlan &p, const MvArgs &a, bool tr, int mod
     return hmx_matvec_r64(p, a, tr, mode, kb, s, ev);
 }
 
-hipError_t hmx_launch_matvec_n1(const DevPlan &p, const MvArgs &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
-    if (p.r <= 8) return hmx_matvec_n1_r8(p, a, tr, src, s, ev);
-    if (p.r <= 16) return hmx_matvec_n1_r16(p, a, tr, src, s, ev);
-    if (p.r <= 24) return hmx_matvec_n1_r24(p, a, tr, src, s, ev);
-    return hmx_matvec_n1_r32(p, a, tr, src, s, ev);
+hipError_t hmx_launch_matvec_n1(const DevPlan &p, const MvArgs &a, bool tr, int src, int nq,
+                                hipStream_t s, const hipEvent_t *ev) {
+    if (p.r <= 8) return hmx_matvec_n1_r8(p, a, tr, src, nq, s, ev);
+    if (p.r <= 16) return hmx_matvec_n1_r16(p, a, tr, src, nq, s, ev);
+    if (p.r <= 24) return hmx_matvec_n1_r24(p, a, tr, src, nq, s, ev);
+    return hmx_matvec_n1_r32(p, a, tr, src, nq, s, ev);
 }
 
 hipError_t hmx_launch_grad(const DevPlan &p, const MvArgs &a, bool tr, double *y2, int64_t incy2,
@@ -101,10 +102,11 @@ hipError_t hmx_launch_matvec(const DevPlanF &p, const MvArgsF &a, bool tr, int m
     return hipErrorInvalidValue;
 }
 
-hipError_t hmx_launch_matvec_n1(const DevPlanF &p, const MvArgsF &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev) {
-    if (p.r <= 8) return hmx_matvec_n1_f32_r8(p, a, tr, src, s, ev);
-    if (p.r <= 16) return hmx_matvec_n1_f32_r16(p, a, tr, src, s, ev);
-    return hmx_matvec_n1_f32_r32(p, a, tr, src, s, ev);
+hipError_t hmx_launch_matvec_n1(const DevPlanF &p, const MvArgsF &a, bool tr, int src, int nq,
+                                hipStream_t s, const hipEvent_t *ev) {
+    if (p.r <= 8) return hmx_matvec_n1_f32_r8(p, a, tr, src, nq, s, ev);
+    if (p.r <= 16) return hmx_matvec_n1_f32_r16(p, a, tr, src, nq, s, ev);
+    return hmx_matvec_n1_f32_r32(p, a, tr, src, nq, s, ev);
 }
 
 hipError_t hmx_launch_grad(const DevPlanF &p, const MvArgsF &a, bool tr, float *y2, int64_t incy2,

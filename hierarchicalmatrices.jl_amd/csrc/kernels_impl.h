@@ -2485,13 +2485,15 @@ hipError_t matvec_r(const DevPlanT<T> &p, const MvArgsT<T> &a, bool tr, int mode
     hipError_t hmx_matvec_m_r##R(const DevPlan &p, const MvArgs &a, int mode, int prec, int nq,  \
                                  hipStream_t s);
 #define HMX_DECLARE_BUCKET_N1(R)                                                                \
-    hipError_t hmx_matvec_n1_r##R(const DevPlan &p, const MvArgs &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev);
+    hipError_t hmx_matvec_n1_r##R(const DevPlan &p, const MvArgs &a, bool tr, int src, int nq,  \
+                                  hipStream_t s, const hipEvent_t *ev);
 #define HMX_DECLARE_BUCKET_F32(R)                                                               \
     hipError_t hmx_matvec_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, int mode,      \
                                    int kb, hipStream_t s, const hipEvent_t *ev);                \
     hipError_t hmx_grad_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, float *y2,       \
                                  int64_t incy2, const float *sv, int64_t incs, hipStream_t s);  \
-    hipError_t hmx_matvec_n1_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, int src, hipStream_t s, const hipEvent_t *ev);          \
+    hipError_t hmx_matvec_n1_f32_r##R(const DevPlanF &p, const MvArgsF &a, bool tr, int src,    \
+                                      int nq, hipStream_t s, const hipEvent_t *ev);             \
     hipError_t hmx_gen_basis_f32_r##R(const DevPlanF &p, hipStream_t s);
 HMX_DECLARE_BUCKET(8)
 HMX_DECLARE_BUCKET(16)

@@ -1,5 +1,5 @@
-// nested1.h -- gfx950 passes of one right-hand side with a nested far field
-// (templates; instantiated per rank bucket, ranks up to 32, by inst_r*.hip).
+// nested1.h -- gfx950 passes of up to four right-hand sides with a nested far
+// field (templates; instantiated per rank bucket, ranks up to 32, by inst_r*.hip).
 //
 // Per level, every point enters the moments of each cluster above it and every
 // row evaluates each covering cluster's series (12 levels at n = 2^20). Here a
@@ -27,11 +27,18 @@
 // took 127 us, waiting on the scalar caches: 1.7 M 64-byte requests, four of
 // five misses.)
 //
+// Two to four right-hand sides share a launch: an entry of the near field and of
+// F is formed (or read) once for them, and a wavefront per right-hand side walks
+// the tree. Single products four times over would form the entries four times;
+// the per-level passes read every level's U, V and F once for four.
+//
 // Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 182 us
 // a product, matrix-free 233 -> 128 us, where the vector instructions alone
 // take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
 // rank 20: 427 -> 60 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
-// n = 1000: 27.0 -> 23.4 us.
+// n = 1000: 27.0 -> 22.7 us. Four right-hand sides, stored log kernel, n = 2^17,
+// leaf 80, rank 20: 349 -> 155 us (the translation, whose log entries of F and
+// of the near field are read, takes 74 of them, the upward pass 53).
 #pragma once
 #include "kernels_impl.h"
 
@@ -63,6 +70,16 @@ __device__ __forceinline__ void sload8(const T *p, T (&o)[8]) {
     const V v = *(const HMX_CONST_AS V *)(p);
 #pragma unroll
     for (int u = 0; u < 8; ++u) o[u] = v[u];
+}
+template <class T> struct Vec4;
+template <> struct Vec4<double> { typedef double type __attribute__((ext_vector_type(4), aligned(8))); };
+template <> struct Vec4<float> { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
+template <class T>
+__device__ __forceinline__ void sload4(const T *p, T (&o)[4]) {
+    using V = typename Vec4<T>::type;
+    const V v = *(const HMX_CONST_AS V *)(p);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) o[u] = v[u];
 }
 template <class T>
 __device__ __forceinline__ T sload1(const T *p) {
@@ -159,17 +176,36 @@ __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T
     }
 }
 
-// One row's sum over a chunk's dense blocks (its runs), eight columns at a
-// time: batches b0, b0 + bs, ... of each block. A block's last batch is its last
-// eight columns, those of the batch before it at weight zero; a block narrower
-// than eight repeats its last column at weight zero. (The next batch is not
-// loaded ahead: two batches and the addresses do not fit the scalar registers,
-// and the other wavefronts cover the loads.) row: the lane's row of the chunk.
-template <class T, int KID, bool TR, int SRC>
-__device__ __forceinline__ T near_runs(const N1Run *runs, int nrun, T p, const T *pts_in,
-                                       const T *A, const T *x, int64_t incx, int row, int b0,
-                                       int bs) {
-    T acc = T(0);
+// acc[i][k] + sum_{u < N} f(p_i, q_u) v[u][k]: each value formed once for its KB
+// right-hand sides (term by term: a shared reciprocal's numerators would be
+// formed for each of them)
+template <class T, int KID, bool TR, int N, int NR, int KB>
+__device__ __forceinline__ void near_terms_kb(const T *p, const T *q, const T (*v)[KB],
+                                              T (*acc)[KB]) {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const T f = TR ? kern_fast<T, KID>(q[u], p[i]) : kern_fast<T, KID>(p[i], q[u]);
+#pragma unroll
+            for (int k = 0; k < KB; ++k) acc[i][k] = fmaT(f, v[u][k], acc[i][k]);
+        }
+}
+
+// One row's sums over a chunk's dense blocks (its runs), N columns at a time:
+// batches b0, b0 + bs, ... of each block. A block's last batch is its last N
+// columns, those of the batch before it at weight zero; a block narrower than N
+// repeats its last column at weight zero. (The next batch is not loaded ahead:
+// two batches and the addresses do not fit the scalar registers, and the other
+// wavefronts cover the loads.) row: the lane's row of the chunk. Of the KB
+// right-hand sides, nq are there; the others repeat the last.
+template <class T, int KID, bool TR, int SRC, int KB>
+__device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, const T *pts_in,
+                                          const T *A, const T *x, int64_t incx, int64_t ldx, int nq,
+                                          int row, int b0, int bs, T (&acc)[KB]) {
+    constexpr int N = KB == 1 ? 8 : 4;
+#pragma unroll
+    for (int k = 0; k < KB; ++k) acc[k] = T(0);
     for (int e = 0; e < nrun; ++e) {
         const N1Run R = sload_struct(runs + e);
         const T *qs = pts_in + R.q0, *vs = x + R.q0 * incx;
@@ -182,66 +218,101 @@ __device__ __forceinline__ T near_runs(const N1Run *runs, int nrun, T p, const T
             return TR ? Ar[(int64_t)(j >> 6) * HM_TILE * R.cols + (j & (HM_TILE - 1))]
                       : Ar[j * HM_TILE];
         };
-        for (int t = b0; 8 * t < R.n; t += bs) {
-            T q[8], v[8];
-            const int j0 = R.n >= 8 ? min(8 * t, R.n - 8) : 0;
-            if (R.n >= 8) {
-                if constexpr (SRC != N1_READ) sload8(qs + j0, q);
-                if (incx == 1) {
-                    sload8(vs + j0, v);
-                } else {
-                    const T *vj = vs + j0 * incx;
+        for (int t = b0; N * t < R.n; t += bs) {
+            T q[N], v[N][KB];
+            const int j0 = R.n >= N ? min(N * t, R.n - N) : 0;
+            if (KB == 1 && R.n >= N && incx == 1) {
+                if constexpr (KB == 1) {
+                    T v8[8];
+                    sload8(vs + j0, v8);
 #pragma unroll
-                    for (int u = 0; u < 8; ++u, vj += incx) v[u] = sload1(vj);
+                    for (int u = 0; u < N; ++u) v[u][0] = v8[u];
                 }
-                if (j0 < 8 * t) {
+            } else if (KB == 4 && ldx == 1 && nq == 4) {
+                if constexpr (KB == 4) {  // a row of x in one load
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) v[u] = j0 + u < 8 * t ? T(0) : v[u];
-                }
-                if constexpr (SRC == N1_READ) {
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) q[u] = entry(j0 + u);
+                    for (int u = 0; u < N; ++u) sload4(vs + min(j0 + u, R.n - 1) * incx, v[u]);
                 }
             } else {
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int j = min(u, R.n - 1);
-                    if constexpr (SRC == N1_READ) q[u] = entry(j);
-                    else q[u] = sload1(qs + j);
-                    const T xv = sload1(vs + j * incx);
-                    v[u] = u < R.n ? xv : T(0);
+                for (int u = 0; u < N; ++u) {
+                    const T *vj = vs + min(j0 + u, R.n - 1) * incx;
+#pragma unroll
+                    for (int k = 0; k < KB; ++k) v[u][k] = sload1(vj + min(k, nq - 1) * ldx);
                 }
             }
+            if (j0 < N * t || j0 + N > R.n) {
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+#pragma unroll
+                    for (int k = 0; k < KB; ++k)
+                        v[u][k] = j0 + u < N * t || j0 + u >= R.n ? T(0) : v[u][k];
+            }
             if constexpr (SRC == N1_READ) {
+#pragma unroll
+                for (int u = 0; u < N; ++u) q[u] = entry(min(j0 + u, R.n - 1));
                 // a column at weight zero adds nothing, whatever its entry
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (j0 + u >= 8 * t && j0 + u < R.n) acc = fmaT(q[u], v[u], acc);
+                for (int u = 0; u < N; ++u)
+                    if (j0 + u >= N * t && j0 + u < R.n)
+#pragma unroll
+                        for (int k = 0; k < KB; ++k) acc[k] = fmaT(q[u], v[u][k], acc[k]);
             } else {
-                near_terms<T, KID, TR, SRC == N1_EXACT, 8, 1>(&p, q, v, &acc);
+                if (KB == 1 && R.n >= N) {
+                    if constexpr (KB == 1) sload8(qs + j0, q);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < N; ++u) q[u] = sload1(qs + min(j0 + u, R.n - 1));
+                }
+                if constexpr (KB == 1) {
+                    T w[N];
+#pragma unroll
+                    for (int u = 0; u < N; ++u) w[u] = v[u][0];
+                    near_terms<T, KID, TR, SRC == N1_EXACT, N, 1>(&p, q, w, acc);
+                } else {
+                    near_terms_kb<T, KID, TR, N, 1, KB>(&p, q, v, &acc);
+                }
             }
         }
     }
-    return acc;
 }
 
 // Columns in LDS, for wavefronts with two rows per lane (rows of two chunks):
-// the sums of a tile's n columns (a multiple of eight, padded at weight zero)
-// for one or both rows. A 16-byte broadcast read takes 8 LDS cycles, shared by
-// four SIMDs, where a row's four terms take 23 vector cycles a column: read
+// a point and its KB inputs. A 16-byte broadcast read takes 8 LDS cycles, shared
+// by four SIMDs, where a row's four terms take 23 vector cycles a column: read
 // for one row alone, LDS would be the slower of the two.
-template <class T, int KID, bool TR, bool EXACT, int NR>
-__device__ __forceinline__ void near_tile(const V2<T> *t, int n, const T (&p)[NR], T (&acc)[NR]) {
-    constexpr int N = KID == 3 ? 2 : 8;
+template <class T, int KB>
+struct NearCol {
+    T q, v[KB];
+};
+
+// the sums of a tile's n columns (a multiple of eight, padded at weight zero)
+// for one or both rows
+template <class T, int KID, bool TR, bool EXACT, int NR, int KB>
+__device__ __forceinline__ void near_tile(const NearCol<T, KB> *t, int n, const T (&p)[NR],
+                                          T (&acc)[NR][KB]) {
+    constexpr int N = KID == 3 || KB > 1 ? 2 : 8;
     for (int j = 0; j < n; j += N) {
-        T q[N], v[N];
+        T q[N], v[N][KB];
 #pragma unroll
         for (int u = 0; u < N; ++u) {
-            const V2<T> c = t[j + u];
-            q[u] = c.x;
-            v[u] = c.y;
+            const NearCol<T, KB> c = t[j + u];
+            q[u] = c.q;
+#pragma unroll
+            for (int k = 0; k < KB; ++k) v[u][k] = c.v[k];
         }
-        near_terms<T, KID, TR, EXACT, N, NR>(p, q, v, acc);
+        if constexpr (KB == 1) {
+            T w[N], s[NR];
+#pragma unroll
+            for (int u = 0; u < N; ++u) w[u] = v[u][0];
+#pragma unroll
+            for (int i = 0; i < NR; ++i) s[i] = acc[i][0];
+            near_terms<T, KID, TR, EXACT, N, NR>(p, q, w, s);
+#pragma unroll
+            for (int i = 0; i < NR; ++i) acc[i][0] = s[i];
+        } else {
+            near_terms_kb<T, KID, TR, N, NR, KB>(p, q, v, acc);
+        }
     }
 }
 
@@ -249,24 +320,29 @@ __device__ __forceinline__ void near_tile(const V2<T> *t, int n, const T (&p)[NR
 // columns pass through this wavefront's LDS 64 at a time, the next tile's
 // loads in flight meanwhile. A run serves the first chunk (mask 1), the second
 // (2) or both (3).
-template <class T, int KID, bool TR, bool EXACT>
+template <class T, int KID, bool TR, bool EXACT, int KB>
 __device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const T (&p)[2],
-                                          const T *pts_in, const T *x, int64_t incx,
-                                          V2<T> (*tile)[WAVE], int lane, T (&acc)[2]) {
+                                          const T *pts_in, const T *x, int64_t incx, int64_t ldx,
+                                          int nq, NearCol<T, KB> (*tile)[WAVE], int lane,
+                                          T (&acc)[2][KB]) {
     if (nrun == 0) return;
     N1UnitRun R = sload_struct(runs);
     int e = 0, j = 0, b = 0;
-    auto load = [&](const N1UnitRun &Q, int j0, V2<T> &c) {
+    auto load = [&](const N1UnitRun &Q, int j0, NearCol<T, KB> &c) {
         const int64_t at = Q.q0 + min(j0 + lane, Q.n - 1);
-        c.x = pts_in[at];
-        c.y = x[at * incx];
+        c.q = pts_in[at];
+#pragma unroll
+        for (int k = 0; k < KB; ++k) c.v[k] = x[at * incx + min(k, nq - 1) * ldx];
     };
-    V2<T> c;
+    NearCol<T, KB> c;
     load(R, 0, c);
     while (e < nrun) {
         const int n = min(WAVE, R.n - j), mask = R.mask;
-        if (lane >= n) c.y = T(0);
-        V2<T> *t = tile[b];
+        if (lane >= n) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k) c.v[k] = T(0);
+        }
+        NearCol<T, KB> *t = tile[b];
         t[lane] = c;
         wave_sync();
         j += WAVE;
@@ -277,23 +353,28 @@ __device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const
         if (e < nrun) load(R, j, c);
         const int n8 = (n + 7) & ~7;
         if (mask == 3) {
-            near_tile<T, KID, TR, EXACT, 2>(t, n8, p, acc);
+            near_tile<T, KID, TR, EXACT, 2, KB>(t, n8, p, acc);
         } else {
             const T p1[1] = {mask == 1 ? p[0] : p[1]};
-            T a1[1] = {mask == 1 ? acc[0] : acc[1]};
-            near_tile<T, KID, TR, EXACT, 1>(t, n8, p1, a1);
-            if (mask == 1) acc[0] = a1[0];
-            else acc[1] = a1[0];
+            T a1[1][KB];
+#pragma unroll
+            for (int k = 0; k < KB; ++k) a1[0][k] = mask == 1 ? acc[0][k] : acc[1][k];
+            near_tile<T, KID, TR, EXACT, 1, KB>(t, n8, p1, a1);
+#pragma unroll
+            for (int k = 0; k < KB; ++k) {
+                if (mask == 1) acc[0][k] = a1[0][k];
+                else acc[1][k] = a1[0][k];
+            }
         }
         b ^= 1;
     }
 }
 
 template <class T>
-__device__ __forceinline__ void n1_write(const N1Chunk &C, const MvArgsT<T> &a, int beta, int lane,
-                                         T v) {
+__device__ __forceinline__ void n1_write(const N1Chunk &C, const MvArgsT<T> &a, int q, int beta,
+                                         int lane, T v) {
     if (lane < C.np) {
-        T *yo = a.y + (C.p0 + lane) * a.incy;
+        T *yo = a.y + (C.p0 + lane) * a.incy + q * a.ldy;
         *yo = (beta ? *yo : T(0)) + v;
     }
 }
@@ -301,31 +382,35 @@ __device__ __forceinline__ void n1_write(const N1Chunk &C, const MvArgsT<T> &a, 
 // One workgroup of the near field, y = beta*y + near: a chunk, its columns
 // split over the wavefronts and their sums added in LDS in wavefront order, or
 // (with units) a unit per wavefront.
-template <class T>
+template <class T, int KB>
 struct NearLds {
     union {
-        V2<T> tile[WPB][2][WAVE];
-        T red[WPB][WAVE];
+        NearCol<T, KB> tile[WPB][2][WAVE];
+        T red[WPB][KB][WAVE];
     };
     __device__ NearLds() {}
 };
-template <class T, int KID, bool TR, int SRC>
+template <class T, int KID, bool TR, int SRC, int KB>
 __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pts_out,
-                                           const T *pts_in, const T *A, const MvArgsT<T> &a,
-                                           NearLds<T> &s) {
+                                           const T *pts_in, const T *A, const MvArgsT<T> &a, int nq,
+                                           NearLds<T, KB> &s) {
     const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
     if (o.nunit == 0) {
         const N1Chunk C = sload_struct(o.ch + blk);
         const int row = min(lane, C.np - 1);
         const T po = SRC == N1_READ ? T(0) : pts_out[C.p0 + row];
-        T acc = near_runs<T, KID, TR, SRC>(o.run + C.run, C.nrun, po, pts_in, A, a.x, a.incx, row,
-                                           wv, WPB);
-        s.red[wv][lane] = acc;
-        __syncthreads();
-        if (wv != 0) return;
+        T acc[KB];
+        near_runs<T, KID, TR, SRC, KB>(o.run + C.run, C.nrun, po, pts_in, A, a.x, a.incx, a.ldx, nq,
+                                       row, wv, WPB, acc);
 #pragma unroll
-        for (int u = 1; u < WPB; ++u) acc += s.red[u][lane];
-        n1_write(C, a, a.beta, lane, acc);
+        for (int k = 0; k < KB; ++k) s.red[wv][k][lane] = acc[k];
+        __syncthreads();
+        // wavefront k adds right-hand side k's sums (KB <= WPB)
+        if (wv >= min(KB, nq)) return;
+        T v = s.red[0][wv][lane];
+#pragma unroll
+        for (int u = 1; u < WPB; ++u) v += s.red[u][wv][lane];
+        n1_write(C, a, wv, a.beta, lane, v);
         return;
     }
     if constexpr (SRC == N1_READ) return;  // stored entries in units: k_down's near part
@@ -333,15 +418,21 @@ __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pt
     if (c >= o.nunit) return;
     const N1Unit Un = sload_struct(o.unit + c);
     N1Chunk C[2];
-    T po[2], acc[2] = {T(0), T(0)};
+    T po[2], acc[2][KB];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         C[q] = sload_struct(o.ch + Un.ch + (q < Un.nch ? q : 0));
         po[q] = pts_out[C[q].p0 + min(lane, C[q].np - 1)];
+#pragma unroll
+        for (int k = 0; k < KB; ++k) acc[q][k] = T(0);
     }
-    near_unit<T, KID, TR, SRC == N1_EXACT>(o.urun + Un.run, Un.nrun, po, pts_in, a.x, a.incx, s.tile[wv], lane, acc);
-    n1_write(C[0], a, a.beta, lane, acc[0]);
-    if (Un.nch == 2) n1_write(C[1], a, a.beta, lane, acc[1]);
+    near_unit<T, KID, TR, SRC == N1_EXACT, KB>(o.urun + Un.run, Un.nrun, po, pts_in, a.x, a.incx,
+                                               a.ldx, nq, s.tile[wv], lane, acc);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int k = 0; k < KB; ++k)
+            if (q < Un.nch && k < nq) n1_write(C[q], a, k, a.beta, lane, acc[q][k]);
 }
 
 // -------------------------------------------------------------- far field
@@ -369,6 +460,51 @@ __device__ __forceinline__ T dot_row(const T (&row)[N], const T *v) {
         s1 = fmaT(row[k + 1], v[k + 1], s1);
     }
     return s0 + s1;
+}
+
+// The moments sum_j T_m(xh_j) x_j of one leaf's points (one wavefront)
+template <class T, int RMAX>
+__device__ __forceinline__ void leaf_moments(const N1Leaf &L, const T *pts, const T *x, int64_t incx,
+                                             int lane, T *out) {
+    const T cx = (T)L.cx, cy = (T)L.cy;
+    T acc[RMAX];
+#pragma unroll
+    for (int k = 0; k < RMAX; ++k) acc[k] = T(0);
+    for (int i = lane; i < L.len; i += WAVE) {
+        const T xv = x[(L.first + i) * incx];
+        const T xh = (pts[L.first + i] - cx) * cy;
+        const T x2 = xh + xh;
+        T t0 = xv, t1 = xh * xv;  // T_m(xh) x by the recurrence
+        acc[0] += t0;
+        acc[1] += t1;
+#pragma unroll
+        for (int k = 2; k < RMAX; ++k) {
+            const T t2 = fmaT(x2, t1, -t0);
+            acc[k] += t2;
+            t0 = t1;
+            t1 = t2;
+        }
+    }
+    int base = 0;
+    Halve<RMAX, WAVE / 2>::run(acc, lane, base);
+    constexpr int LEFT = HalveShape<RMAX, WAVE / 2>::left;
+    constexpr int MASK = HalveShape<RMAX, WAVE / 2>::mask;
+    if ((lane & MASK) == 0) {
+#pragma unroll
+        for (int i = 0; i < LEFT; ++i) out[base + i] = acc[i];
+    }
+}
+
+// One node's moments from its halves' (zero for an empty one)
+template <class T, int RMAX>
+__device__ __forceinline__ void node_moments(const N1Node &N, const T (&Mr)[RMAX], T (*mom)[RMAX],
+                                             int n, int m, int h) {
+    if (N.c[0] < 0 && N.c[1] < 0) return;  // a leaf (wave-uniform)
+    const int c = h ? N.c[1] : N.c[0];
+    T v = dot_row(Mr, mom[c >= 0 ? c : 0]);
+    if (c < 0) v = T(0);
+    v += __shfl_xor(v, 32);
+    if (h == 0 && m < RMAX) mom[n][m] = v;
 }
 
 // Upward pass, one workgroup per subtree of the input side. The subtree's
@@ -405,33 +541,7 @@ __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const
     }
     for (int e = wv; e < S.nleaf; e += WPB) {
         const N1Leaf L = sload_struct(s.leaf + S.leaf + e);
-        const T cx = (T)L.cx, cy = (T)L.cy;
-        T acc[RMAX];
-#pragma unroll
-        for (int k = 0; k < RMAX; ++k) acc[k] = T(0);
-        for (int i = lane; i < L.len; i += WAVE) {
-            const T xv = x[(L.first + i) * incx];
-            const T xh = (pts[L.first + i] - cx) * cy;
-            const T x2 = xh + xh;
-            T t0 = xv, t1 = xh * xv;  // T_m(xh) x by the recurrence
-            acc[0] += t0;
-            acc[1] += t1;
-#pragma unroll
-            for (int k = 2; k < RMAX; ++k) {
-                const T t2 = fmaT(x2, t1, -t0);
-                acc[k] += t2;
-                t0 = t1;
-                t1 = t2;
-            }
-        }
-        int base = 0;
-        Halve<RMAX, WAVE / 2>::run(acc, lane, base);
-        constexpr int LEFT = HalveShape<RMAX, WAVE / 2>::left;
-        constexpr int MASK = HalveShape<RMAX, WAVE / 2>::mask;
-        if ((lane & MASK) == 0) {
-#pragma unroll
-            for (int i = 0; i < LEFT; ++i) mom[L.loc][base + i] = acc[i];
-        }
+        leaf_moments<T, RMAX>(L, pts, x, incx, lane, mom[L.loc]);
     }
     T Mr[RMAX];
     load_rows(mats + Mt::MU, lane, Mr);
@@ -439,13 +549,7 @@ __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const
     for (int l = S.nlev - 2; l >= 0; --l) {
         const int nb = lev[l], ne = lev[l + 1];
         for (int n = nb + wv; n < ne; n += WPB) {
-            const N1Node N = nodes[n];
-            if (N.c[0] < 0 && N.c[1] < 0) continue;  // a leaf (wave-uniform)
-            const int c = h ? N.c[1] : N.c[0];
-            T v = dot_row(Mr, mom[c >= 0 ? c : 0]);
-            if (c < 0) v = T(0);  // an empty half
-            v += __shfl_xor(v, 32);
-            if (h == 0 && m < RMAX) mom[n][m] = v;
+            node_moments<T, RMAX>(nodes[n], Mr, mom, n, m, h);
         }
         __syncthreads();
     }
@@ -485,6 +589,75 @@ __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const
     }
 }
 
+// Upward pass of several right-hand sides: a wavefront takes one of them through
+// the whole subtree, so that the wavefronts' chains of latencies run side by
+// side without a barrier.
+template <class T, int RMAX>
+struct UpLdsKb {
+    alignas(16) T mom[N1_KB][N1_NODES][RMAX];
+    alignas(16) T pv[N1_KB][2][RMAX];
+};
+template <class T, int RMAX>
+__device__ __forceinline__ void n1_up_block_kb(const N1Side &s, const T *pts, const T *x,
+                                               int64_t incx, int64_t ldx, const T *mats, T *partial,
+                                               T *w, int r, int nq, int blk, UpLdsKb<T, RMAX> &L_) {
+    using Mt = N1Mat<T, RMAX>;
+    static_assert(N1_KB == WPB, "a wavefront per right-hand side");
+    const int lane = threadIdx.x % WAVE, q = uniform((int)(threadIdx.x / WAVE));
+    if (q >= nq) return;
+    const int m = lane & 31, h = lane >> 5;
+    auto &mom = L_.mom[q];
+    const N1Sub S = sload_struct(s.sub + blk);
+    N1Node nd{-1, {-1, -1}};
+    if (lane < S.nnode) nd = s.node[S.node + lane];
+    int p_half = 0;
+    int64_t p_slot = -1;
+    auto load_path = [&](int e) {  // the path's nodes e + lane from the root's parent up
+        const int at = S.npath - 1 - e - lane;
+        if (at >= 0) {
+            const N1Path P = s.path[S.path + at];
+            p_half = P.half;
+            p_slot = P.slot;
+        }
+    };
+    load_path(0);
+    x += q * ldx;
+    for (int e = 0; e < S.nleaf; ++e) {
+        const N1Leaf L = sload_struct(s.leaf + S.leaf + e);
+        leaf_moments<T, RMAX>(L, pts, x, incx, lane, mom[L.loc]);
+    }
+    T Mr[RMAX];
+    load_rows(mats + Mt::MU, lane, Mr);
+    wave_sync();
+    for (int n = S.nnode - 1; n >= 0; --n) {  // halves come after their node
+        const N1Node N{0, {rl_i(nd.c[0], n), rl_i(nd.c[1], n)}};
+        node_moments<T, RMAX>(N, Mr, mom, n, m, h);
+        wave_sync();
+    }
+    const T *cur = mom[0];
+    for (int e = 0; e < S.npath; ++e) {
+        if (e > 0 && e % WAVE == 0) load_path(e);
+        const int64_t slot = rl_l(p_slot, e % WAVE);
+        T v = dot_row(Mr, cur);
+        if (h != rl_i(p_half, e % WAVE)) v = T(0);
+        v += __shfl_xor(v, 32);
+        T *nx = L_.pv[q][e & 1];
+        if (h == 0 && m < RMAX) nx[m] = v;
+        if (slot >= 0 && h == 0 && m < r) partial[(slot * nq + q) * r + m] = v;
+        wave_sync();
+        cur = nx;
+    }
+    T Ar[Mt::HALF];
+    load_rows(mats + Mt::AU, lane, Ar);
+    for (int n = 0; n < S.nnode; ++n) {
+        const int cl = rl_i(nd.cl, n);
+        if (cl < 0) continue;
+        T v = dot_row(Ar, &mom[n][h * Mt::HALF]);
+        v += __shfl_xor(v, 32);
+        if (h == 0 && m < r) w[((int64_t)cl * nq + q) * r + m] = v;
+    }
+}
+
 // Translation: one wavefront per cluster of the output side whose sources all
 // lie in subtrees (a wavefront takes several in turn, the matrix rows kept);
 // the clusters with a source above them ("heavy", first in the target list)
@@ -493,15 +666,16 @@ __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const
 // values and nodes are staged four at a time in LDS with one round of loads.
 // F formed from the nodes: eight or four terms of 1/d^m share a reciprocal as
 // in the near field.
-template <class T, int RMAX>
+template <class T, int RMAX, int KB>
 struct TrLds {
-    alignas(16) T sw[WPB][4][RMAX], st[WPB][4][RMAX];
-    alignas(16) T zr[WPB][RMAX];
+    alignas(16) T sw[WPB][4][KB][RMAX], st[WPB][4][RMAX];
+    alignas(16) T zr[WPB][KB][RMAX];
 };
-template <class T, int RMAX, bool TRANS, int SRC, int KID>
-__device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N1Side &o, int blk,
-                                                   int nblk, const T *mats, const T *partial, const T *w,
-                                                   T *z, TrLds<T, RMAX> &L_) {
+template <class T, int RMAX, bool TRANS, int SRC, int KID, int KB>
+__device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N1Side &o, int nq,
+                                                   int blk, int nblk, const T *mats,
+                                                   const T *partial, const T *w, T *z,
+                                                   TrLds<T, RMAX, KB> &L_) {
     using Mt = N1Mat<T, RMAX>;
     constexpr bool FREE = SRC != N1_READ;
     constexpr int HALF = Mt::HALF, NB = 4, NT = HALF % 8 == 0 ? 8 : 4;
@@ -515,59 +689,76 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     const T *oth = TRANS ? p.rnodes : p.cnodes;
     T At[HALF];
     load_rows(mats + Mt::AT, lane, At);
-    T to = T(0), acc = T(0);
-    // ws: zero past r; ts: past r repeats
-    auto apply = [&](const T *ws, const T *ts, int64_t foff) {
-        if constexpr (FREE) {
+    T to = T(0), acc[KB];
+#pragma unroll
+    for (int k = 0; k < KB; ++k) acc[k] = T(0);
+    // ws: zero past r (and past nq); ts: past r repeats
+    auto apply = [&](const T (*ws)[RMAX], const T *ts, int64_t foff) {
+        if constexpr (FREE && KB == 1) {
 #pragma unroll
             for (int j = 0; j < HALF; j += NT)
-                near_terms<T, KID, TRANS, SRC == N1_EXACT, NT, 1>(&to, ts + h * HALF + j, ws + h * HALF + j, &acc);
+                near_terms<T, KID, TRANS, SRC == N1_EXACT, NT, 1>(&to, ts + h * HALF + j,
+                                                                  ws[0] + h * HALF + j, acc);
         } else {
             const T *F = p.F + foff;
             T fv[HALF];
 #pragma unroll
             for (int j = 0; j < HALF; ++j) {
-                const int l = min(h * HALF + j, r - 1);
-                fv[j] = __builtin_nontemporal_load(TRANS ? F + (l + r * mm) : F + (mm + r * l));
+                if constexpr (FREE) {
+                    const T t = ts[h * HALF + j];
+                    fv[j] = TRANS ? kern_fast<T, KID>(t, to) : kern_fast<T, KID>(to, t);
+                } else {
+                    const int l = min(h * HALF + j, r - 1);
+                    fv[j] = __builtin_nontemporal_load(TRANS ? F + (l + r * mm) : F + (mm + r * l));
+                }
             }
 #pragma unroll
-            for (int j = 0; j < HALF; ++j) {
-                const int l = h * HALF + j;
-                acc = fmaT(fv[j], ws[l], acc);  // ws is zero past r
-            }
+            for (int j = 0; j < HALF; ++j)
+#pragma unroll
+                for (int k = 0; k < KB; ++k) acc[k] = fmaT(fv[j], ws[k][h * HALF + j], acc[k]);
         }
     };
-    auto finish = [&](int id, const T *zs) {  // c = A^T z
-        T c = dot_row(At, zs + h * HALF);
-        c += __shfl_xor(c, 32);
-        if (h == 0 && m < r) z[(int64_t)id * r + m] = c;
+    auto put_z = [&] {  // this wavefront's sums into its zr
+#pragma unroll
+        for (int k = 0; k < KB; ++k) {
+            acc[k] += __shfl_xor(acc[k], 32);
+            if (h == 0 && m < RMAX) zr[wv][k][m] = m < r ? acc[k] : T(0);
+            acc[k] = T(0);
+        }
+    };
+    auto finish = [&](int id, const T (*zs)[RMAX]) {  // c = A^T z
+#pragma unroll 1
+        for (int k = 0; k < nq; ++k) {
+            T c = dot_row(At, zs[k] + h * HALF);
+            c += __shfl_xor(c, 32);
+            if (h == 0 && m < r) z[((int64_t)id * nq + k) * r + m] = c;
+        }
     };
     if (blk >= o.nheavy) {
         const int step = (nblk - o.nheavy) * WPB;
         for (int idx = o.nheavy + (blk - o.nheavy) * WPB + wv; idx < o.ncl; idx += step) {
             const N1Target C = sload_struct(o.target + idx);
             if constexpr (FREE) to = (TRANS ? p.cnodes : p.rnodes)[(int64_t)C.id * r + mm];
-            acc = T(0);
             for (int e0 = C.beg; e0 < C.end; e0 += NB) {
                 const int ne = min(NB, C.end - e0);
-                // (source, column) = (i / RMAX, i % RMAX)
+                // (source, right-hand side, column) = (i / KB RMAX, i / RMAX % KB, i % RMAX)
 #pragma unroll
-                for (int u = 0; u < (NB * RMAX + WAVE - 1) / WAVE; ++u) {
+                for (int u = 0; u < (NB * KB * RMAX + WAVE - 1) / WAVE; ++u) {
                     const int i = lane + u * WAVE;
-                    const int e = i / RMAX, l = i - e * RMAX;
+                    const int e = i / (KB * RMAX), k = i / RMAX % KB, l = i % RMAX;
                     if (e < ne) {
-                        const int64_t at = (int64_t)o.tr[e0 + e].src * r + min(l, r - 1);
-                        const T wl = w[at];
-                        sw[wv][e][l] = l < r ? wl : T(0);
-                        if constexpr (FREE) st[wv][e][l] = oth[at];
+                        const int64_t src = o.tr[e0 + e].src;
+                        const T wl = w[(src * nq + min(k, nq - 1)) * r + min(l, r - 1)];
+                        sw[wv][e][k][l] = l < r && k < nq ? wl : T(0);
+                        if (FREE && k == 0) st[wv][e][l] = oth[src * r + min(l, r - 1)];
                     }
                 }
                 wave_sync();
+#pragma unroll 1
                 for (int e = 0; e < ne; ++e) apply(sw[wv][e], st[wv][e], FREE ? 0 : o.tr[e0 + e].foff);
                 wave_sync();
             }
-            acc += __shfl_xor(acc, 32);
-            if (h == 0 && m < RMAX) zr[wv][m] = m < r ? acc : T(0);
+            put_z();
             wave_sync();
             finish(C.id, zr[wv]);
             wave_sync();
@@ -581,44 +772,50 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     for (int e = C.beg + wv; e < C.end; e += WPB) {
         const DTrRec R = o.tr[e];
         if (FREE && h == 0 && m < RMAX) st[wv][0][m] = oth[(int64_t)R.src * r + (m < r ? m : r - 1)];
-        if (R.nslots > 0) {
-            // lane half h sums the slots h, h + 2, ..., sixteen loads in flight
-            const T *ps = partial + R.pbase * r + mm;
-            T s = T(0);
-            int t = h;
-            for (; t + 30 < R.nslots; t += 32) {
-                T v[16];
+#pragma unroll 1
+        for (int k = 0; k < KB; ++k) {
+            const int kc = min(k, nq - 1);
+            T wl;
+            if (R.nslots > 0) {
+                // lane half h sums the slots h, h + 2, ..., sixteen loads in flight
+                const T *ps = partial + (R.pbase * nq + kc) * r + mm;
+                const int64_t ld = (int64_t)nq * r;
+                T s = T(0);
+                int t = h;
+                for (; t + 30 < R.nslots; t += 32) {
+                    T v[16];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) v[u] = ps[(int64_t)(t + 2 * u) * r];
+                    for (int u = 0; u < 16; ++u) v[u] = ps[(t + 2 * u) * ld];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) s += v[u];
+                    for (int u = 0; u < 16; ++u) s += v[u];
+                }
+                for (; t < R.nslots; t += 2) s += ps[t * ld];
+                s += __shfl_xor(s, 32);
+                if (h == 0 && m < RMAX) sw[wv][0][k][m] = m < r ? s : T(0);
+                wave_sync();
+                wl = dot_row(Ar, &sw[wv][0][k][h * HALF]);  // w = A mu
+                wl += __shfl_xor(wl, 32);
+                wave_sync();
+            } else {
+                wl = w[((int64_t)R.src * nq + kc) * r + mm];
             }
-            for (; t < R.nslots; t += 2) s += ps[(int64_t)t * r];
-            s += __shfl_xor(s, 32);
-            if (h == 0 && m < RMAX) sw[wv][0][m] = m < r ? s : T(0);
-            wave_sync();
-            T v = dot_row(Ar, &sw[wv][0][h * HALF]);  // w = A mu
-            v += __shfl_xor(v, 32);
-            wave_sync();
-            if (h == 0 && m < RMAX) sw[wv][0][m] = v;
-        } else if (h == 0 && m < RMAX) {
-            const T wl = w[(int64_t)R.src * r + mm];
-            sw[wv][0][m] = m < r ? wl : T(0);
+            if (h == 0 && m < RMAX) sw[wv][0][k][m] = m < r && k < nq ? wl : T(0);
         }
         wave_sync();
         apply(sw[wv][0], st[wv][0], R.foff);
         wave_sync();
     }
-    acc += __shfl_xor(acc, 32);
-    if (h == 0 && m < RMAX) zr[wv][m] = m < r ? acc : T(0);
+    put_z();
     __syncthreads();
     if (wv != 0) return;
-    T s = T(0);
-    if (m < RMAX)
-        for (int u = 0; u < WPB; ++u) s += zr[u][m];
-    wave_sync();
-    if (h == 0 && m < RMAX) zr[0][m] = s;
-    wave_sync();
+    for (int k = 0; k < KB; ++k) {
+        T s = T(0);
+        if (m < RMAX)
+            for (int u = 0; u < WPB; ++u) s += zr[u][k][m];
+        wave_sync();
+        if (h == 0 && m < RMAX) zr[0][k][m] = s;
+        wave_sync();
+    }
     finish(C.id, zr[0]);
 }
 
@@ -648,51 +845,63 @@ __device__ __forceinline__ bool chain_block(int n, int &at) {
 // Five wavefronts per SIMD are asked of the register allocator where the near
 // field is formed: left alone it gives four (upward) and three (translation);
 // six cost the near field's chains their registers (85 us).
-constexpr int n1_waves(int src, int kid) { return src != N1_READ && kid < 3 ? 5 : 1; }
+// Several right-hand sides: four, or three where the upward pass's LDS allows
+// no more.
+constexpr int n1_waves(int src, int kid, int rmax, int kb) {
+    if (kid == 3 || (src == N1_READ && kb == 1)) return 1;
+    return kb == 1 ? 5 : rmax > 24 || src == N1_READ ? 3 : 4;
+}
 
-template <class T, int RMAX, int SRC, int KID, bool TR>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID))))
+template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID, RMAX, KB))))
 void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *A, const T *mats,
-             MvArgsT<T> a, int r, int nup, int nb0, int nb) {
+             MvArgsT<T> a, int r, int nq, int nup, int nb0, int nb) {
     __shared__ union Lds {
-        UpLds<T, RMAX> up;
-        NearLds<T> near;
+        std::conditional_t<KB == 1, UpLds<T, RMAX>, UpLdsKb<T, RMAX>> up;
+        NearLds<T, KB> near;
         __device__ Lds() {}
     } s;
     int at;
     if (chain_block(nup, at)) {
-        if (at < nup) n1_up_block<T, RMAX>(in, in_pts, a.x, a.incx, mats, a.partial, a.w, r, at, s.up);
+        if (at >= nup) return;
+        if constexpr (KB == 1)
+            n1_up_block<T, RMAX>(in, in_pts, a.x, a.incx, mats, a.partial, a.w, r, at, s.up);
+        else
+            n1_up_block_kb<T, RMAX>(in, in_pts, a.x, a.incx, a.ldx, mats, a.partial, a.w, r, nq, at,
+                                    s.up);
     } else if (at < nb) {
-        near_block<T, KID, TR, SRC>(out, at + nb0, out_pts, in_pts, A, a, s.near);
+        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, A, a, nq, s.near);
     }
 }
 
-template <class T, int RMAX, int SRC, int KID, bool TR>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID))))
+template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID, RMAX, KB))))
 void k_n1_translate(DevPlanT<T> p, N1Side out, const T *in_pts, const T *out_pts, MvArgsT<T> a,
-                    int ntr, int nb0, int nb) {
+                    int nq, int ntr, int nb0, int nb) {
     __shared__ union Lds {
-        TrLds<T, RMAX> tr;
-        NearLds<T> near;
+        TrLds<T, RMAX, KB> tr;
+        NearLds<T, KB> near;
         __device__ Lds() {}
     } s;
     int at;
     if (chain_block(ntr, at)) {
         if (at < ntr)
-            n1_translate_block<T, RMAX, TR, SRC, KID>(p, out, at, ntr, p.n1m, a.partial, a.w, a.z, s.tr);
+            n1_translate_block<T, RMAX, TR, SRC, KID, KB>(p, out, nq, at, ntr, p.n1m, a.partial,
+                                                          a.w, a.z, s.tr);
     } else if (at < nb) {
-        near_block<T, KID, TR, SRC>(out, at + nb0, out_pts, in_pts, p.A, a, s.near);
+        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, p.A, a, nq, s.near);
     }
 }
 
 // The coefficients of a subtree's nodes into cof (LDS): the path's, one node
 // after another, then each node's halves together (lane half h takes half h).
-// One wavefront; pz: its LDS, sixteen path nodes' z at a time (and the last
-// batch's final node in row N1_PATH); lane l holds local node l's record.
+// z: ldz apart from cluster to cluster. One wavefront; pz: its LDS, sixteen path
+// nodes' z at a time (and the last batch's final node in row N1_PATH); lane l
+// holds local node l's record.
 template <class T, int RMAX>
 __device__ __forceinline__ void n1_coefficients(const N1Side &s, const N1Sub &S, const T *mats,
-                                                const T *z, int r, int lane, T (*cof)[RMAX],
-                                                T (*pz)[RMAX]) {
+                                                const T *z, int64_t ldz, int r, int lane,
+                                                T (*cof)[RMAX], T (*pz)[RMAX]) {
     using Mt = N1Mat<T, RMAX>;
     const int m = lane & 31, h = lane >> 5;
     N1Node nd{-1, {-1, -1}};
@@ -705,7 +914,7 @@ __device__ __forceinline__ void n1_coefficients(const N1Side &s, const N1Sub &S,
     for (int i0 = 0; i0 < S.nnode * RMAX; i0 += WAVE) {
         const int i = i0 + lane, n = i / RMAX, l = i - n * RMAX;
         const int cl = __shfl(nd.cl, n < S.nnode ? n : 0);
-        if (n < S.nnode) cof[n][l] = (cl >= 0 && l < r) ? z[(int64_t)cl * r + l] : T(0);
+        if (n < S.nnode) cof[n][l] = (cl >= 0 && l < r) ? z[cl * ldz + l] : T(0);
     }
     int half = 0;
     const T *cur = nullptr;
@@ -722,7 +931,7 @@ __device__ __forceinline__ void n1_coefficients(const N1Side &s, const N1Sub &S,
         for (int u = 0; u < N1_PATH * RMAX / WAVE; ++u) {
             const int i = lane + u * WAVE, e = i / RMAX, l = i - e * RMAX;
             const int cl = __shfl(P.cl, e);
-            if (e < ne) pz[e][l] = (cl >= 0 && l < r) ? z[(int64_t)cl * r + l] : T(0);
+            if (e < ne) pz[e][l] = (cl >= 0 && l < r) ? z[cl * ldz + l] : T(0);
         }
         wave_sync();
         for (int e = 0; e < ne; ++e) {
@@ -773,27 +982,32 @@ __device__ __forceinline__ T n1_series(const N1Chunk &C, const T (*cof)[RMAX], T
 
 // Downward pass: the far field added onto y, which holds the near field. A
 // subtree per workgroup, its chunks over the wavefronts.
-template <class T, int RMAX>
+// Several right-hand sides: a wavefront forms the coefficients of each.
+template <class T, int RMAX, int KB>
 __global__ __launch_bounds__(WG) void k_n1_down(N1Side o, const T *pts_out, const T *z,
-                                               const T *mats, MvArgsT<T> a, int r) {
-    __shared__ __align__(16) T cof[N1_NODES][RMAX];
-    __shared__ __align__(16) T pz[N1_PATH + 1][RMAX];
+                                                const T *mats, MvArgsT<T> a, int r, int nq) {
+    static_assert(KB <= WPB, "a wavefront per right-hand side");
+    __shared__ __align__(16) T cof[KB][N1_NODES][RMAX];
+    __shared__ __align__(16) T pz[KB][N1_PATH + 1][RMAX];
     const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
     const N1Sub S = sload_struct(o.sub + blockIdx.x);
-    if (wv == WPB - 1) n1_coefficients<T, RMAX>(o, S, mats, z, r, lane, cof, pz);
+    if (wv < nq)
+        n1_coefficients<T, RMAX>(o, S, mats, z + wv * r, (int64_t)nq * r, r, lane, cof[wv], pz[wv]);
     __syncthreads();
     for (int c = S.ch + wv; c < S.ch + S.nch; c += WPB) {
         const N1Chunk C = sload_struct(o.ch + c);
         const T po = pts_out[C.p0 + min(lane, C.np - 1)];
-        n1_write(C, a, 1, lane, n1_series<T, RMAX>(C, cof, po));
+#pragma unroll
+        for (int k = 0; k < KB; ++k)
+            if (k < nq) n1_write(C, a, k, 1, lane, n1_series<T, RMAX>(C, cof[k], po));
     }
 }
 
-// One product y = beta*y + op(H) x of one right-hand side over the interval
-// trees. Many chunks of stored entries stream through k_down's near part, on
-// the side stream when there is one.
-template <class T, int RMAX, int SRC, int KID, bool TR>
-hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s,
+// One product y = beta*y + op(H) x of nq <= KB right-hand sides over the
+// interval trees. Many chunks of stored entries stream through k_down's near part,
+// on the side stream when there is one.
+template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
+hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, int nq, hipStream_t s,
                        const hipEvent_t *ev) {
     auto mark = [&](int q) {
         if (ev) (void)hipEventRecord(ev[q], s);
@@ -806,12 +1020,27 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s,
     auto near_part = [&](hipStream_t ns) {
         MvArgsT<T> an = a;
         an.part = 1;
-        if constexpr (TR)
-            k_down<T, RMAX, false, 0, true, true, 1><<<nblk(p.ncch), WG, 0, ns>>>(
-                p, p.cch, p.ncch, p.cnear, p.cfar, p.ccl, p.V, p.cmap, p.y, p.x, a.z, an);
-        else
-            k_down<T, RMAX, false, 0, false, true, 1><<<nblk(p.nrch), WG, 0, ns>>>(
-                p, p.rch, p.nrch, p.rnear, p.rfar, p.rcl, p.U, p.rmap, p.x, p.y, a.z, an);
+        for (int q = 0; q < nq;) {
+            an.y = a.y + q * a.ldy;
+            an.x = a.x + q * a.ldx;
+            if constexpr (TR) {
+                k_down<T, RMAX, false, 0, true, true, 1><<<nblk(p.ncch), WG, 0, ns>>>(
+                    p, p.cch, p.ncch, p.cnear, p.cfar, p.ccl, p.V, p.cmap, p.y, p.x, a.z, an);
+                q += 1;
+            } else if (nq - q == 4) {
+                k_down<T, RMAX, false, 0, false, true, 4><<<nblk(p.nrch), WG, 0, ns>>>(
+                    p, p.rch, p.nrch, p.rnear, p.rfar, p.rcl, p.U, p.rmap, p.x, p.y, a.z, an);
+                q += 4;
+            } else if (nq - q >= 2) {
+                k_down<T, RMAX, false, 0, false, true, 2><<<nblk(p.nrch), WG, 0, ns>>>(
+                    p, p.rch, p.nrch, p.rnear, p.rfar, p.rcl, p.U, p.rmap, p.x, p.y, a.z, an);
+                q += 2;
+            } else {
+                k_down<T, RMAX, false, 0, false, true, 1><<<nblk(p.nrch), WG, 0, ns>>>(
+                    p, p.rch, p.nrch, p.rnear, p.rfar, p.rcl, p.U, p.rmap, p.x, p.y, a.z, an);
+                q += 1;
+            }
+        }
     };
     if (split) {
         hipError_t e = hipEventRecord(a.fork, s);
@@ -828,15 +1057,15 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s,
     const int nup = far ? in.nsub : 0;
     mark(0);
     if (nup + nb0 > 0)
-        k_n1_up<T, RMAX, SRC, KID, TR><<<n1_grid(nup, nb0), WG, 0, s>>>(
-            in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, nup, 0, nb0);
+        k_n1_up<T, RMAX, SRC, KID, TR, KB><<<n1_grid(nup, nb0), WG, 0, s>>>(
+            in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, nq, nup, 0, nb0);
     mark(1);
     mark(2);
     if (far) {
         // light clusters: at most four wavefronts per SIMD, looping
         const int ntr = out.nheavy + std::min((out.ncl - out.nheavy + WPB - 1) / WPB, 1024);
-        k_n1_translate<T, RMAX, SRC, KID, TR><<<n1_grid(ntr, nb - nb0), WG, 0, s>>>(
-            p, out, in_pts, out_pts, a, ntr, nb0, nb - nb0);
+        k_n1_translate<T, RMAX, SRC, KID, TR, KB><<<n1_grid(ntr, nb - nb0), WG, 0, s>>>(
+            p, out, in_pts, out_pts, a, nq, ntr, nb0, nb - nb0);
     }
     mark(3);
     if (split) {
@@ -845,36 +1074,44 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s,
     } else if (stream) {
         near_part(s);
     }
-    if (far) k_n1_down<T, RMAX><<<out.nsub, WG, 0, s>>>(out, out_pts, a.z, p.n1m, a, p.r);
+    if (far)
+        k_n1_down<T, RMAX, KB><<<out.nsub, WG, 0, s>>>(out, out_pts, a.z, p.n1m, a, p.r, nq);
     mark(4);
     return hipGetLastError();
 }
 
 // src: N1_FREE, N1_EXACT (kernels 1/d^m) or N1_READ
-template <class T, int RMAX, bool TR>
-hipError_t matvec_n1_k(const DevPlanT<T> &p, const MvArgsT<T> &a, int src, hipStream_t s,
+template <class T, int RMAX, bool TR, int KB>
+hipError_t matvec_n1_k(const DevPlanT<T> &p, const MvArgsT<T> &a, int src, int nq, hipStream_t s,
                        const hipEvent_t *ev) {
-    if (src == N1_READ) return matvec_n1_t<T, RMAX, N1_READ, 0, TR>(p, a, s, ev);
-    if (src == N1_EXACT) {
+    if (src == N1_READ) return matvec_n1_t<T, RMAX, N1_READ, 0, TR, KB>(p, a, nq, s, ev);
+    // several right-hand sides form term by term either way
+    if (src == N1_EXACT || (KB > 1 && p.kid <= 2)) {
         switch (p.kid) {
-        case 0: return matvec_n1_t<T, RMAX, N1_EXACT, 0, TR>(p, a, s, ev);
-        case 1: return matvec_n1_t<T, RMAX, N1_EXACT, 1, TR>(p, a, s, ev);
-        default: return matvec_n1_t<T, RMAX, N1_EXACT, 2, TR>(p, a, s, ev);
+        case 0: return matvec_n1_t<T, RMAX, N1_EXACT, 0, TR, KB>(p, a, nq, s, ev);
+        case 1: return matvec_n1_t<T, RMAX, N1_EXACT, 1, TR, KB>(p, a, nq, s, ev);
+        default: return matvec_n1_t<T, RMAX, N1_EXACT, 2, TR, KB>(p, a, nq, s, ev);
         }
     }
-    switch (p.kid) {
-    case 0: return matvec_n1_t<T, RMAX, N1_FREE, 0, TR>(p, a, s, ev);
-    case 1: return matvec_n1_t<T, RMAX, N1_FREE, 1, TR>(p, a, s, ev);
-    case 2: return matvec_n1_t<T, RMAX, N1_FREE, 2, TR>(p, a, s, ev);
-    default: return matvec_n1_t<T, RMAX, N1_FREE, 3, TR>(p, a, s, ev);
+    if constexpr (KB == 1) {
+        switch (p.kid) {
+        case 0: return matvec_n1_t<T, RMAX, N1_FREE, 0, TR, KB>(p, a, nq, s, ev);
+        case 1: return matvec_n1_t<T, RMAX, N1_FREE, 1, TR, KB>(p, a, nq, s, ev);
+        case 2: return matvec_n1_t<T, RMAX, N1_FREE, 2, TR, KB>(p, a, nq, s, ev);
+        default: break;
+        }
     }
+    return matvec_n1_t<T, RMAX, N1_FREE, 3, TR, KB>(p, a, nq, s, ev);
 }
 
 template <class T, int RMAX>
-hipError_t matvec_n1(const DevPlanT<T> &p, const MvArgsT<T> &a, bool tr, int src, hipStream_t s,
-                     const hipEvent_t *ev) {
-    return tr ? matvec_n1_k<T, RMAX, true>(p, a, src, s, ev)
-              : matvec_n1_k<T, RMAX, false>(p, a, src, s, ev);
+hipError_t matvec_n1(const DevPlanT<T> &p, const MvArgsT<T> &a, bool tr, int src, int nq,
+                     hipStream_t s, const hipEvent_t *ev) {
+    if (nq == 1)
+        return tr ? matvec_n1_k<T, RMAX, true, 1>(p, a, src, 1, s, ev)
+                  : matvec_n1_k<T, RMAX, false, 1>(p, a, src, 1, s, ev);
+    return tr ? matvec_n1_k<T, RMAX, true, N1_KB>(p, a, src, nq, s, ev)
+              : matvec_n1_k<T, RMAX, false, N1_KB>(p, a, src, nq, s, ev);
 }
 
 }  // namespace

@@ -1282,7 +1282,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
             st.reserve(&b.mx, (int64_t)P->xtn.size() * r * HM_WS_RHS);
         }
         if (P->n1) st.add(&b.n1m, n1m);
-        st.reserve(&b.partial, std::max(nslots * HM_WS_RHS, std::max(P->n1x.slots, P->n1y.slots)) * r);
+        st.reserve(&b.partial, std::max(nslots * HM_WS_RHS, std::max(P->n1x.slots, P->n1y.slots) * N1_KB) * r);
         st.reserve(&b.w, ncl * r * HM_WS_RHS);
         st.reserve(&b.z, ncl * r * HM_WS_RHS);
         if (std::is_same_v<T, double>) st.reserve(&b.xt, P->ny * HM_WS_RHS);
@@ -2258,10 +2258,16 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
     // HBM and gains nothing on a side stream; the computed ones (hybrid's
     // Clenshaw far field, matrix-free kernel values) overlap the chain
     const bool use_side = mode != 0 && split_near_field(P, s);
+    // over the interval trees, up to N1_KB right-hand sides per launch. A
+    // stored plan's U and V equal the Chebyshev form's basis up to rounding
+    // unless a node meets a point (non-finite entries then keep the stored form)
+    const bool n1 = P->n1 && (mode != 0 || basis_finite(P, s));
+    const int src = mode == 2 ? N1_FREE : P->regen && !P->refit ? N1_EXACT : N1_READ;
     for (int64_t q = 0; q < k;) {
-        // forward products take up to HM_MAX_KB right-hand sides per launch
+        // per level, forward products take up to HM_MAX_KB right-hand sides
         int kb = 1;
-        if (!tr && max_kb > 1)
+        if (n1) kb = (int)std::min<int64_t>(std::min(max_kb, N1_KB), k - q);
+        else if (!tr && max_kb > 1)
             while (kb * 2 <= max_kb && q + kb * 2 <= k) kb *= 2;
         MvArgsT<T> a = ws_args<T>(P);
         a.y = y + ioff + q * ldy;
@@ -2276,12 +2282,6 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
             a.fork = P->fork;
             a.join = P->join;
         }
-        // one right-hand side over the interval trees. A stored plan's U and V
-        // equal the Chebyshev form's basis up to rounding unless a node meets
-        // a point (non-finite entries then keep the stored form)
-        bool n1 = P->n1 && kb == 1;
-        if (n1 && mode == 0) n1 = basis_finite(P, s);
-        const int src = mode == 2 ? N1_FREE : P->regen && !P->refit ? N1_EXACT : N1_READ;
         const hipEvent_t *ev = nullptr;
         if (P->profile) {
             const size_t at = P->prof_events.size();
@@ -2292,7 +2292,7 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
             }
             ev = P->prof_events.data() + at;
         }
-        hipError_t e = n1 ? hmx_launch_matvec_n1(P->bufs<T>().dp, a, tr, src, s, ev)
+        hipError_t e = n1 ? hmx_launch_matvec_n1(P->bufs<T>().dp, a, tr, src, kb, s, ev)
                           : hmx_launch_matvec(P->bufs<T>().dp, a, tr, mode, kb, s, ev);
         if (e != hipSuccess) return fail(HM_ERR_HIP, "matvec launch: %s", hipGetErrorString(e));
         q += kb;

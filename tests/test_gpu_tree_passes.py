@@ -191,3 +191,45 @@ def test_moved_onto_a_node(cuda):
     assert torch.equal(torch.isfinite(H @ b), torch.isfinite(want))
     H.update_points(xd, yd)
     assert torch.equal(H @ b, u0)
+
+
+@pytest.mark.parametrize("kernel", ["coulombkernel", "logkernel"])
+@pytest.mark.parametrize("n,bs,r", [(50, 80, 20), (900, 40, 9), (1500, 130, 32), (2501, 80, 20)])
+@pytest.mark.parametrize("k", [2, 3, 4, 5, 7])
+def test_several_rhs(cuda, kernel, n, bs, r, k):
+    # up to four right-hand sides per launch, rows or columns contiguous, accumulating; each column
+    # within the products' 1e-12 of the oracle's mul!
+    x, y, iv = points(n, "random", n)
+    B = np.random.default_rng(k).standard_normal((n, k))
+    t = O.Tree(KID[kernel], x, y, *iv, bs, r)
+    tt = O.Tree(KID[kernel], y, x, iv[2], iv[3], iv[0], iv[1], bs, r)
+    ref = np.stack([t.matvec(np.ascontiguousarray(B[:, q])) for q in range(k)], 1)
+    reft = SIGN[kernel] * np.stack([tt.matvec(np.ascontiguousarray(B[:, q])) for q in range(k)], 1)
+    Bd = torch.from_numpy(B).to(cuda)
+    Bc = Bd.t().contiguous().t()
+    for form in ("stored", "free"):
+        H = hmx.KernelMatrix(kernel, x, y, *iv, blocksize=bs, rank=r, matrix_free=form == "free")
+        for b in (Bd, Bc):
+            u, v = (H @ b).cpu().numpy(), (H.T @ b).cpu().numpy()
+            for q in range(k):
+                assert rel(u[:, q], ref[:, q]) <= 1e-12 and rel(v[:, q], reft[:, q]) <= 1e-12, (form, q)
+        u = Bd.clone()
+        H.mul(u, Bd)
+        assert rel(u.cpu().numpy(), ref + B) <= 1e-12
+        H.close()
+
+
+@pytest.mark.parametrize("kernel", ["cauchykernel", "logkernel"])
+@pytest.mark.parametrize("form", ["stored", "free"])
+def test_several_rhs_units(cuda, kernel, form):
+    # more than 4096 chunks, against the same plan's single products (rounding
+    # of another summation order: the per-column bar of the multi-RHS passes, 1e-13)
+    n = 270001
+    x, y, iv = points(n, "random", 8)
+    H = hmx.KernelMatrix(kernel, x, y, *iv, blocksize=80, rank=16, matrix_free=form == "free")
+    B = torch.randn(n, 3, dtype=torch.float64, device=cuda)
+    u, v = H @ B, H.T @ B
+    for q in range(3):
+        b = B[:, q].contiguous()
+        assert ((u[:, q] - H @ b).norm() / u[:, q].norm()).item() <= 1e-13
+        assert ((v[:, q] - H.T @ b).norm() / v[:, q].norm()).item() <= 1e-13
