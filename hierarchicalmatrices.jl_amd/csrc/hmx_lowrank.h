@@ -37,15 +37,10 @@ struct LRItem {
     int64_t small;    // offset of the small slot
 };
 
-// LDS (doubles) available to the in-LDS factorization: M*C + 2*C*(C+1) must
-// fit (160 KB per workgroup on gfx950, less the static arrays)
-#define LR_LDS_DOUBLES 20352
-
 // op codes: the enum hm_lr_op of include/hmx.h. rank (device, count values)
 // receives each result's rank; max_rows = the largest m or n of the items;
-// lds_qr = the largest in-LDS factorization (doubles, 0: none), big_qr = some
-// factor does not fit; lds_svd = the largest Jacobi workspace (doubles);
+// lds_svd = the largest Jacobi workspace (doubles);
 // max_c = the largest factor width (cu, cv) of the items.
 hipError_t hmx_lowrank_run(int op, const LRItem *items, int64_t count, double *tall,
-                           double *small, int64_t *rank, int64_t max_rows, int64_t lds_qr,
-                           bool big_qr, int64_t lds_svd, int64_t max_c, hipStream_t s);
+                           double *small, int64_t *rank, int64_t max_rows, int64_t lds_svd,
+                           int64_t max_c, hipStream_t s);

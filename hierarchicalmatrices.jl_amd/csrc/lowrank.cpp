@@ -37,8 +37,7 @@ int hm_lowrank_op(int op, int64_t count, const int64_t *dims, const double *cons
     if (count == 0) return HM_OK;
     if (count >= (int64_t)1 << 31) return lfail(HM_ERR_INVALID, "lowrank_op: too many items");
     std::vector<LRItem> items((size_t)count);
-    int64_t tall = 0, max_rows = 0, lds_qr = 0, lds_svd = 0, max_c = 1;
-    bool big_qr = false;
+    int64_t tall = 0, max_rows = 0, lds_svd = 0, max_c = 1;
     for (int64_t t = 0; t < count; ++t) {
         const int64_t *d = dims + 5 * t;
         const int64_t m = d[0], n = d[1], k = d[2], r1 = d[3], r2 = d[4];
@@ -101,13 +100,6 @@ int hm_lowrank_op(int op, int64_t count, const int64_t *dims, const double *cons
         tall += (int64_t)it.cv * n;
         it.small = t * LR_SMALL;
         max_rows = std::max(max_rows, std::max(m, n));
-        const int64_t sides[2][2] = {{m, it.cu}, {n, it.cv}};
-        for (const auto &sd : sides) {
-            if (sd[1] == 0) continue;
-            const int64_t need = sd[0] * sd[1] + 2 * sd[1] * (sd[1] + 1);
-            if (need <= LR_LDS_DOUBLES) lds_qr = std::max(lds_qr, need);
-            else big_qr = true;
-        }
         const int64_t P = std::max(it.p, it.q), Q = std::min(it.p, it.q);
         lds_svd = std::max(lds_svd, (P + 1) * Q + (Q + 1) * Q + Q);
     }
@@ -122,8 +114,8 @@ int hm_lowrank_op(int op, int64_t count, const int64_t *dims, const double *cons
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_items, items.data(), sizeof(LRItem) * (size_t)count, hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
-        e = hmx_lowrank_run(op, d_items, count, d_tall, d_small, d_rank, max_rows, lds_qr, big_qr,
-                            lds_svd, max_c, s);
+        e = hmx_lowrank_run(op, d_items, count, d_tall, d_small, d_rank, max_rows, lds_svd,
+                            max_c, s);
     if (e == hipSuccess)
         e = hipMemcpyAsync(rank, d_rank, sizeof(int64_t) * (size_t)count, hipMemcpyDeviceToHost, s);
     hipError_t e2 = hipSuccess;

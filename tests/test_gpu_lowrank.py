@@ -154,3 +154,18 @@ def test_factors_beyond_lds_in_one_batch(cuda):
     L = rand_lr(rng, 3000, 100, 48)
     A = rng.standard_normal((2500, 3000))
     agree(DL.batch("dmul", [items_of(A=A, U2=L[0], S2=L[1], V2=L[2])])[0], LR.dmul(A, L))
+
+
+@pytest.mark.parametrize("m,n,r1,r2", [
+    (511, 513, 8, 8), (2048, 2049, 9, 7), (2600, 512, 8, 9), (1024, 513, 16, 16), (4100, 32, 20, 12),
+    (33, 700, 17, 16), (64, 511, 32, 32), (1537, 513, 40, 23), (1, 1, 1, 0), (17, 16, 15, 1)])
+def test_factor_sizes(cuda, m, n, r1, r2):
+    """Factors whose rows stay in registers, are streamed, or both, and widths on
+    either side of the 16- and 32-column forms (r2 = 0: svdtrunc of one entry)."""
+    rng = np.random.default_rng(m + 7 * n)
+    if r2 == 0:
+        agree(DL.batch("svdtrunc", [items_of(A=np.array([[-2.5]]))])[0], LR.svdtrunc(np.array([[-2.5]])))
+        return
+    L1, L2 = rand_lr(rng, m, n, r1), rand_lr(rng, m, n, r2)
+    got = DL.batch("sub", [items_of(U1=L1[0], S1=L1[1], V1=L1[2], U2=L2[0], S2=L2[1], V2=L2[2])])[0]
+    agree(got, LR.add(L1, L2, -1.0))
