@@ -51,24 +51,94 @@ __global__ __launch_bounds__(WG) void k_even_tile_F(const ELeaf *leaves, int64_t
     }
 }
 
-template <class T>
-__device__ inline T wave_xor(T v, int o) {
-    return __shfl_xor(v, o, 64);
+// Exchanges between lanes without LDS. v_permlane32_swap / v_permlane16_swap
+// exchange the halves (odd and even rows of sixteen lanes) of two registers.
+template <bool ROW>
+__device__ inline void swap32(unsigned &a, unsigned &b) {
+    if constexpr (ROW) {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    }
+}
+template <bool ROW, class T>
+__device__ inline T halve_swap(T a, T b) {
+    constexpr int W = sizeof(T) / 4;
+    unsigned x[W], y[W];
+    __builtin_memcpy(x, &a, sizeof(T));
+    __builtin_memcpy(y, &b, sizeof(T));
+#pragma unroll
+    for (int w = 0; w < W; ++w) swap32<ROW>(x[w], y[w]);
+    __builtin_memcpy(&a, x, sizeof(T));
+    __builtin_memcpy(&b, y, sizeof(T));
+    return a + b;
+}
+template <int CTRL, class T>
+__device__ inline T dpp(T v) {
+    constexpr int W = sizeof(T) / 4;
+    int x[W];
+    __builtin_memcpy(x, &v, sizeof(T));
+#pragma unroll
+    for (int w = 0; w < W; ++w) x[w] = __builtin_amdgcn_update_dpp(0, x[w], CTRL, 0xf, 0xf, true);
+    __builtin_memcpy(&v, x, sizeof(T));
+    return v;
+}
+template <int CTRL, class T>
+__device__ inline T halve_dpp(T a, T b, bool up) {
+    return (up ? b : a) + dpp<CTRL>(up ? a : b);
 }
 
-// Upward pass: one wavefront per task. Lane l takes the task's columns
-// l, l + 64, ..., so all its columns share one global parity; lanes of equal
-// parity are summed with xor shuffles 2..32, after which every even lane holds
-// the sums of one parity and every odd lane those of the other. Lane l then
-// writes k = kb + l/2 of its parity. Output e = (q*2 + par)*n + k of the
-// leaf's beta (single-task leaves) or of the task's partial slot.
+// CB (8, 16 or 32) sums over the 32 lanes of each parity. Each step halves the
+// sums a lane keeps: halves of the wavefront, rows of sixteen lanes, then within
+// a row a rotation by four lanes (each lane ends with two neighbouring groups of
+// four), by eight, and the pairs of a group of four. Returns the sum `even_col`.
+constexpr int DPP_ROR4 = 0x124, DPP_ROR8 = 0x128, DPP_XOR2 = 0x4E;  // 0x4E: quad_perm 2 3 0 1
+template <int CB, class T>
+__device__ inline T halve_sums(T (&a)[CB], int lane) {
+#pragma unroll
+    for (int u = 0; u < CB / 2; ++u) a[u] = halve_swap<false>(a[u], a[u + CB / 2]);
+#pragma unroll
+    for (int u = 0; u < CB / 4; ++u) a[u] = halve_swap<true>(a[u], a[u + CB / 4]);
+#pragma unroll
+    for (int u = 0; u < CB / 8; ++u) a[u] = halve_dpp<DPP_ROR4>(a[u], a[u + CB / 8], lane & 4);
+    if constexpr (CB >= 16) {
+#pragma unroll
+        for (int u = 0; u < CB / 16; ++u)
+            a[u] = halve_dpp<DPP_ROR8>(a[u], a[u + CB / 16], lane & 8);
+    } else {
+        a[0] += dpp<DPP_ROR8>(a[0]);
+    }
+    if constexpr (CB >= 32) a[0] = halve_dpp<DPP_XOR2>(a[0], a[1], lane & 2);
+    else a[0] += dpp<DPP_XOR2>(a[0]);
+    return a[0];
+}
+// which sum a lane ends with
+template <int CB>
+__device__ inline int even_col(int lane) {
+    const int c = (lane >> 5 & 1) * 16 | (lane >> 4 & 1) * 8 | (lane >> 2 & 1) * 4 |
+                  (lane >> 3 & 1) * 2 | (lane >> 1 & 1);
+    return c / (32 / CB);
+}
+
+// Upward pass: one workgroup per task. Thread t takes the task's columns
+// t, t + 256, ..., so a lane's columns share one global parity; a wavefront's
+// lanes of equal parity are summed, then the four wavefronts in LDS. Output
+// e = (q*2 + par)*n + k of the leaf's beta (single-task leaves) or of the task's
+// partial slot. Bound by reading F: one wavefront per task left the chip with 512
+// (n = 2^18, rank 20, eight levels: 83 us), four with 3072 (55 us, 6.1 TB/s).
 template <class T, int RB, int KB>
-__global__ __launch_bounds__(64) void k_even_up(EvenDev<T> p, const T *v, int64_t joff,
+__global__ __launch_bounds__(WG) void k_even_up(EvenDev<T> p, const T *v, int64_t joff,
                                                int64_t incv, int64_t ldv, int nq) {
+    constexpr int CB = RB <= 8 ? 8 : RB <= 16 ? 16 : 32;
+    __shared__ T part[WG / 64][2 * KB * RB];
     const EUp tk = p.up[blockIdx.x];
     const ELeaf L = p.leaves[tk.leaf];
     const int n = p.n;
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const T *F = p.F + L.foff;
     const int64_t jg = joff + L.col0;  // global column of the leaf's column 0
     T acc[KB][RB];
@@ -77,7 +147,7 @@ __global__ __launch_bounds__(64) void k_even_up(EvenDev<T> p, const T *v, int64_
 #pragma unroll
         for (int k = 0; k < RB; ++k) acc[q][k] = T(0);
     const int64_t jend = tk.j0 + tk.len;
-    for (int64_t j = tk.j0 + lane; j < jend; j += 64) {
+    for (int64_t j = tk.j0 + tid; j < jend; j += WG) {
         // all loads of the column first, then the products: each load is
         // guarded by k < n, and a guard around load and use would wait on
         // every load in turn. F is read once per product: non-temporal
@@ -93,29 +163,26 @@ __global__ __launch_bounds__(64) void k_even_up(EvenDev<T> p, const T *v, int64_
 #pragma unroll
             for (int q = 0; q < KB; ++q) acc[q][k] += f[k] * x[q];
     }
+    const int par = (int)((jg + tk.j0 + lane) & 1);
 #pragma unroll
     for (int q = 0; q < KB; ++q)
 #pragma unroll
-        for (int k = 0; k < RB; ++k)
-            if (k < n)
+        for (int kb = 0; kb < RB; kb += CB) {
+            T a[CB];
 #pragma unroll
-                for (int o = 2; o < 64; o <<= 1) acc[q][k] += wave_xor(acc[q][k], o);
-    const int par = (int)((jg + tk.j0 + lane) & 1);
+            for (int k = 0; k < CB; ++k) a[k] = kb + k < RB ? acc[q][kb + k] : T(0);
+            const T val = halve_sums<CB>(a, lane);
+            const int kk = kb + even_col<CB>(lane);
+            if (kk < n) part[wv][(q * 2 + par) * n + kk] = val;
+        }
+    __syncthreads();
     const int64_t stride = (int64_t)HM_EVEN_KB * 2 * n;
     T *out = tk.single ? p.beta + (int64_t)tk.leaf * stride : p.partial + tk.slot * stride;
+    for (int e = tid; e < 2 * KB * n; e += WG) {
+        T t = part[0][e];
 #pragma unroll
-    for (int kb = 0; kb < RB; kb += 32) {
-        const int kk = kb + (lane >> 1);
-        if (kk < n) {
-#pragma unroll
-            for (int q = 0; q < KB; ++q) {
-                T val = T(0);
-#pragma unroll
-                for (int k = kb; k < kb + 32 && k < RB; ++k)
-                    if (k == kk) val = acc[q][k];
-                out[(q * 2 + par) * n + kk] = val;
-            }
-        }
+        for (int w = 1; w < WG / 64; ++w) t += part[w][e];
+        out[e] = t;
     }
 }
 
@@ -141,7 +208,15 @@ __global__ __launch_bounds__(256) void k_even_reduce(EvenDev<T> p, int kb) {
     __shared__ T part[256];
     T s = T(0);
     if (g < G)
-        for (int t = g; t < r.ntask; t += G) s += p.partial[(r.slot0 + t) * stride + e];
+        // eight loads in flight; the sum keeps slot order
+        for (int t = g; t < r.ntask; t += 8 * G) {
+            T v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[u] = t + u * G < r.ntask ? p.partial[(r.slot0 + t + u * G) * stride + e] : T(0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
     part[threadIdx.x] = s;
     __syncthreads();
     if (threadIdx.x < E) {
@@ -224,7 +299,7 @@ hipError_t even_matvec_t(const EvenDev<T> &p, T *u, const T *v, int64_t ioff, in
         if (beta == 0 && !p.covered && p.nrows > 0)
             k_even_zero<T><<<(unsigned)((p.nrows + WG - 1) / WG), WG, 0, s>>>(uq, ioff, incu, ldu,
                                                                           p.nrows, nb);
-        if (p.nup > 0) k_even_up<T, RB, KB><<<p.nup, 64, 0, s>>>(p, vq, joff, incv, ldv, nb);
+        if (p.nup > 0) k_even_up<T, RB, KB><<<p.nup, WG, 0, s>>>(p, vq, joff, incv, ldv, nb);
         if (p.nred > 0) k_even_reduce<T><<<p.nred, 256, 0, s>>>(p, nb);
         if (p.ndown > 0) k_even_down<T, RB, KB><<<p.ndown, WG, 0, s>>>(p, uq, ioff, incu, ldu, nb,
                                                                   store);

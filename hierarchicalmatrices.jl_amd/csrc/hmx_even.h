@@ -8,7 +8,7 @@
 // accumulates every leaf:
 //
 //   up      task (leaf, <= HM_EVEN_COLS columns): beta[par][k] = sum over the
-//           task's columns J of parity par of F[j, k] v[J]; one wavefront.
+//           task's columns J of parity par of F[j, k] v[J]; one workgroup.
 //   reduce  leaves with several tasks: beta = sum of the task partials, in
 //           task order.
 //   down    segment (rows covered by the same leaves, <= 256 rows): one
@@ -18,7 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define HM_EVEN_COLS 4096  // columns per upward task (one wavefront)
+#define HM_EVEN_COLS 4096  // columns per upward task (one workgroup)
 #define HM_EVEN_ROWS 256   // rows per downward task (one thread each)
 #define HM_EVEN_KB 4       // right-hand sides the workspace holds per launch
 #define HM_EVEN_RMAX 64    // largest rank

@@ -354,3 +354,24 @@ def test_element_types_do_not_mix(cuda):
     assert b"Float32" in hmx._lib.lib.hm_last_error()
     with pytest.raises(TypeError):
         hmx.EvenBarycentricLeaves(64, 64, [(0, 0, B)], dtype=np.float64)
+
+
+@pytest.mark.parametrize("rank", [3, 8, 9, 16, 20, 32, 33, 64])
+@pytest.mark.parametrize("p", [1, 2, 63, 64, 65, 255, 257, 4097])
+def test_upward_sums(cuda, rank, p):
+    """Columns over the four wavefronts of a task and sums over the lanes of one
+    parity, every width of the exchange, one and three right-hand sides, within
+    the rounding bound of sums of p and of rank terms."""
+    m = 70
+    B = hmx.EvenBarycentricMatrix(f_osc, 1, m, 2, p + 1, rank=rank)
+    H = hmx.EvenBarycentricLeaves(m, p, [(0, 0, B)])
+    mask = (np.arange(m)[:, None] + np.arange(p)[None, :]) % 2 == 0
+    D = (np.array(B.F) @ np.array(B.W)).T * mask
+    A = (np.abs(B.F) @ np.abs(B.W)).T * mask
+    v = np.random.default_rng(p).standard_normal((p, 3))
+    want = D @ v
+    got = torch.stack([H.matvec(torch.from_numpy(np.ascontiguousarray(v[:, q])).cuda())
+                       for q in range(3)], 1).cpu().numpy()
+    both = H.matvec(torch.from_numpy(v).cuda()).cpu().numpy()
+    bar = (p + rank + 8) * 2.3e-16 * np.max(A @ np.abs(v))
+    assert np.max(np.abs(got - want)) <= bar and np.max(np.abs(both - want)) <= bar
