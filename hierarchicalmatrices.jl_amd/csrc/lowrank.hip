@@ -238,9 +238,13 @@ __device__ inline double halve_sums(double (&a)[CB], int lane) {
     for (int u = 0; u < CB / 4; ++u) a[u] = halve_swap<true>(a[u], a[u + CB / 4]);
 #pragma unroll
     for (int u = 0; u < CB / 8; ++u) a[u] = halve_dpp<DPP_ROR8>(a[u], a[u + CB / 8], lane & 8);
+    if constexpr (CB >= 16) {
 #pragma unroll
-    for (int u = 0; u < CB / 16; ++u)
-        a[u] = halve_dpp<DPP_HALF_MIRROR>(a[u], a[u + CB / 16], lane & 4);
+        for (int u = 0; u < CB / 16; ++u)
+            a[u] = halve_dpp<DPP_HALF_MIRROR>(a[u], a[u + CB / 16], lane & 4);
+    } else {
+        a[0] += dpp<DPP_HALF_MIRROR>(a[0]);
+    }
     if constexpr (CB >= 32) {
 #pragma unroll
         for (int u = 0; u < CB / 32; ++u)
@@ -258,28 +262,34 @@ __device__ inline double halve_sums(double (&a)[CB], int lane) {
 // reflectors below X's diagonal, R (upper C x C, ld LR_MAX) and tau into the
 // small slot. X's upper triangle is left as it falls: nothing reads it.
 //
-// Thread t owns rows t, t + WGR, ...; the first RR of them stay in registers
-// for the whole factorization, the rest are streamed (X is L2-resident). Every
-// row keeps its trailing columns only: x[q] is column j + q, and the update of
-// step j writes x[q - 1]. One pass per step both updates the rows and forms the
-// next step's dot products x_{j+1}[j+2:] . x_k[j+2:] (q = 0: the squared norm),
-// so a step is: halve the CB sums over the wavefront's lanes (each exchange
-// keeps half of the sums, CB + log2 exchanges in place of 6 CB), one barrier,
-// then every wavefront adds the wavefronts' sums and forms beta, tau and
-// w_k = tau (x_k[j] + v[j+1:] . x_k[j+1:]) for itself. The thread of row j + 1
-// leaves it in LDS instead of adding it to the dot products.
+// Panels of PW = 8 columns, then the columns to their right eight at a time. One
+// workgroup of 512 threads; thread t owns rows t, t + WGR, ... throughout, so the
+// passes over X need no barrier between them, only the sums over rows do.
 //
-// One workgroup of 512 threads, 256 vector registers each. Differences of 20
-// blocks of 256 to 2048 rows and 10 to 32 columns: 295 us with T, where two
-// passes per step, eight columns at a time, took 640 (779 with the factors held
-// in LDS, a launch of its own) and T another 412. What is left are the streamed
-// rows, read and written once a step at one compute unit's 64 bytes a cycle. More
-// than the register file in flight (32 columns of a streamed row) spills: 398.
-constexpr int WGR = 512, NWR = WGR / 64;
+// qr_panel: the first RR rows of a thread stay in registers for the panel's
+// steps, the rest are streamed. A row keeps its trailing columns only: x[q] is
+// column j + q, and the update of step j writes x[q - 1]. One pass per step both
+// updates the rows and forms the next step's dot products x_{j+1}[j+2:] .
+// x_k[j+2:] (q = 0: the squared norm), so a step has one barrier: the sums are
+// halved over the wavefront's lanes, then every wavefront adds the wavefronts'
+// and forms beta, tau and w_k = tau (x_k[j] + v[j+1:] . x_k[j+1:]) for itself.
+// The thread of row j + 1 leaves it in LDS instead of adding it to the sums.
+//
+// panel_sums and panel_update: S = V^T B for eight columns B (or the panel's own:
+// its Gram matrix G), one sum a lane; the eight reflectors in turn are then
+// w_j = tau_j (S_j - sum_{l<j} G_lj w_l), and B -= V w.
+//
+// Updating every trailing column in every step instead (rows in registers where
+// they fit) streams the rest of X through L2 once a step, at one compute unit's
+// 64 bytes a cycle: 295 us with T for differences of 20 blocks of 256 to 2048
+// rows and 10 to 32 columns; in panels 181. Two passes per step, eight
+// columns at a time, took 640 (779 with the factors held in LDS, a launch of its
+// own) and T another 412.
+constexpr int WGR = 512, NWR = WGR / 64, PW = 8;
+constexpr int RR = 4;  // 2048 rows in registers (six or eight: spills)
 
-template <int CB>
 struct QrLds {
-    double red[2][NWR][CB], row[2][CB];
+    double red[2][NWR][PW], row[2][PW], sums[2][NWR][PW * PW];
 };
 
 __device__ inline double lane_value(double v, int lane) {
@@ -288,54 +298,45 @@ __device__ inline double lane_value(double v, int lane) {
     return __hiloint2double(hi, lo);
 }
 
-template <int CB, int RR, int KC>
-__device__ inline void qr_steps(const TallView &T, QrLds<CB> &s) {
-    constexpr int SH = CB == 16 ? 2 : CB == 32 ? 1 : 0;  // lane >> SH: its sum's column
-    const int M = T.M, C = T.C;
+// columns p0 .. p0 + C - 1 (C <= PW), rows p0 .. M - 1
+__device__ inline void qr_panel(const TallView &T, int p0, int C, QrLds &s) {
+    const int M = T.M;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    double *const X = T.X;
-    double x[RR > 0 ? RR : 1][CB], acc[CB];
+    double *const X = T.X + (int64_t)p0 * M;
+    double x[RR][PW], acc[PW];
 #pragma unroll
-    for (int q = 0; q < CB; ++q) acc[q] = 0.0;
+    for (int q = 0; q < PW; ++q) acc[q] = 0.0;
 #pragma unroll
     for (int k = 0; k < RR; ++k) {
+        if (WGR * k >= M) break;
         const int i = tid + WGR * k;
 #pragma unroll
-        for (int q = 0; q < CB; ++q) x[k][q] = q < C && i < M ? X[(int64_t)q * M + i] : 0.0;
+        for (int q = 0; q < PW; ++q)
+            x[k][q] = q < C && i >= p0 && i < M ? X[(int64_t)q * M + i] : 0.0;
     }
 #pragma unroll
     for (int k = 0; k < RR; ++k) {
-        const double x0 = tid + WGR * k > 0 ? x[k][0] : 0.0;
+        if (WGR * k >= M) break;
+        const double x0 = tid + WGR * k > p0 ? x[k][0] : 0.0;
 #pragma unroll
-        for (int q = 0; q < CB; ++q) acc[q] += x0 * x[k][q];
-        if (tid + WGR * k == 0) {
+        for (int q = 0; q < PW; ++q) acc[q] += x0 * x[k][q];
+    }
+    if (tid == p0) {
 #pragma unroll
-            for (int q = 0; q < CB; ++q) s.row[0][q] = x[k][q];
-        }
+        for (int q = 0; q < PW; ++q) s.row[0][q] = x[0][q];
     }
     for (int i0 = WGR * RR; i0 < M; i0 += WGR) {
         const int i = min(i0 + tid, M - 1);
-        const double x0 = i0 + tid < M && i > 0 ? X[i] : 0.0;
+        const double x0 = i0 + tid < M ? X[i] : 0.0;
 #pragma unroll
-        for (int c = 0; c < CB; c += KC) {
-            if (c >= C) break;
-            double y[KC];
-#pragma unroll
-            for (int u = 0; u < KC; ++u) y[u] = c + u < C ? X[(int64_t)(c + u) * M + i] : 0.0;
-#pragma unroll
-            for (int u = 0; u < KC; ++u) acc[c + u] += x0 * y[u];
-            if (i == 0) {
-#pragma unroll
-                for (int u = 0; u < KC; ++u) s.row[0][c + u] = y[u];
-            }
-        }
+        for (int q = 0; q < PW; ++q) acc[q] += x0 * X[(int64_t)min(q, C - 1) * M + i];
     }
-    for (int j = 0; j < C; ++j) {
-        const int nk = C - j, b = j & 1;
-        const double wsum = halve_sums<CB>(acc, lane);
-        if ((lane & ((1 << SH) - 1)) == 0) s.red[b][wv][lane >> SH] = wsum;
+    for (int jl = 0; jl < C; ++jl) {
+        const int j = p0 + jl, nk = C - jl, b = jl & 1;
+        const double wsum = halve_sums<PW>(acc, lane);
+        if ((lane & 7) == 0) s.red[b][wv][lane >> 3] = wsum;
         __syncthreads();
-        const int ql = lane & (CB - 1);
+        const int ql = lane & (PW - 1);
         double sum = 0.0;
 #pragma unroll
         for (int w = 0; w < NWR; ++w) sum += s.red[b][w][ql];
@@ -352,68 +353,165 @@ __device__ inline void qr_steps(const TallView &T, QrLds<CB> &s) {
             T.R[j + LR_MAX * (j + lane)] = lane == 0 ? beta : rj - wl;
             if (lane == 0) T.tau[j] = t;
         }
+        double w[PW];
 #pragma unroll
-        for (int q = 0; q < CB; ++q) acc[q] = 0.0;
-        if constexpr (RR > 0) {
+        for (int q = 1; q < PW; ++q) w[q] = lane_value(wl, q);
+#pragma unroll
+        for (int q = 0; q < PW; ++q) acc[q] = 0.0;
+#pragma unroll
+        for (int k = 0; k < RR; ++k) {
             // rows up to j and past M go along unstored (a branch would keep
             // two copies of the row in registers)
-            double vv[RR], x0[RR];
+            if (WGR * k >= M) break;
+            const int i = tid + WGR * k;
+            const double v = x[k][0] * scal;
+            if (i > j && i < M) X[(int64_t)jl * M + i] = v;
+            const double vv = t != 0.0 && i > j ? v : 0.0;
 #pragma unroll
-            for (int k = 0; k < RR; ++k) {
-                const int i = tid + WGR * k;
-                const double v = x[k][0] * scal;
-                if (i > j && i < M) X[(int64_t)j * M + i] = v;
-                vv[k] = t != 0.0 && i > j ? v : 0.0;
-            }
+            for (int q = 1; q < PW; ++q) x[k][q - 1] = x[k][q] - w[q] * vv;
+            x[k][PW - 1] = 0.0;
+            const double x0 = i > j + 1 ? x[k][0] : 0.0;
 #pragma unroll
-            for (int u = 0; u < CB; ++u) {
-                const double wu = u + 1 < CB ? lane_value(wl, u + 1) : 0.0;
+            for (int q = 0; q < PW; ++q) acc[q] += x0 * x[k][q];
+        }
+        if (tid == j + 1) {
 #pragma unroll
-                for (int k = 0; k < RR; ++k) {
-                    x[k][u] = u + 1 < CB ? x[k][u + 1] - wu * vv[k] : 0.0;
-                    if (u == 0) x0[k] = tid + WGR * k > j + 1 ? x[k][0] : 0.0;
-                    acc[u] += x0[k] * x[k][u];
-                }
-            }
-            if (tid == j + 1) {
-#pragma unroll
-                for (int u = 0; u < CB; ++u) s.row[b ^ 1][u] = x[0][u];
-            }
+            for (int q = 0; q < PW; ++q) s.row[b ^ 1][q] = x[0][q];
         }
         for (int i0 = WGR * RR; i0 < M; i0 += WGR) {
+            // columns past the last are read as the last and not stored
             const int i = min(i0 + tid, M - 1);
-            const bool own = i0 + tid < M && i > j;
-            double *xr = X + (int64_t)j * M + i;
-            const double v = xr[0] * scal, vv = t != 0.0 ? v : 0.0;
+            const bool own = i0 + tid < M;
+            double *xr = X + (int64_t)jl * M + i;
+            double y[PW];
+#pragma unroll
+            for (int q = 0; q < PW; ++q) y[q] = xr[(int64_t)min(q, nk - 1) * M];
+            const double v = y[0] * scal, vv = t != 0.0 ? v : 0.0;
             if (own) xr[0] = v;
-            double x0 = 0.0;
 #pragma unroll
-            for (int c = 0; c < CB; c += KC) {
-                if (c + 1 >= nk) break;
-                // columns past the last are read as the last and not stored
-                int64_t o[KC];
-#pragma unroll
-                for (int u = 0; u < KC; ++u) o[u] = (int64_t)min(c + u + 1, nk - 1) * M;
-                double y[KC];
-#pragma unroll
-                for (int u = 0; u < KC; ++u) y[u] = xr[o[u]];
-#pragma unroll
-                for (int u = 0; u < KC; ++u)
-                    y[u] -= (c + u + 1 < CB ? lane_value(wl, c + u + 1) : 0.0) * vv;
-#pragma unroll
-                for (int u = 0; u < KC; ++u)
-                    if (own && c + u + 1 < nk) xr[o[u]] = y[u];
-                if (c == 0) x0 = own && i > j + 1 ? y[0] : 0.0;
-#pragma unroll
-                for (int u = 0; u < KC; ++u) acc[c + u] += x0 * y[u];
-                if (own && i == j + 1) {
-#pragma unroll
-                    for (int u = 0; u < KC; ++u) s.row[b ^ 1][c + u] = y[u];
-                }
+            for (int q = 1; q < PW; ++q) {
+                y[q] -= w[q] * vv;
+                if (own && q < nk) xr[(int64_t)q * M] = y[q];
             }
+            const double x0 = own && nk > 1 ? y[1] : 0.0;
+#pragma unroll
+            for (int q = 1; q < PW; ++q) acc[q - 1] += x0 * y[q];
         }
     }
-    for (int e = tid; e < C * C; e += WGR) {
+}
+
+// V^T B over the rows: lane 8 a + c receives v_a . B_c, for the panel's V (unit
+// lower triangular from row p0) and B = columns c0 .. of X (cn of them; those
+// past the last count as the last), or V itself (c0 == p0)
+__device__ inline double panel_sums(const TallView &T, int p0, int c0, int cn, QrLds &s, int b) {
+    const int M = T.M, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const double *V = T.X + (int64_t)p0 * M, *B = T.X + (int64_t)c0 * M;
+    double acc[PW * PW];
+#pragma unroll
+    for (int e = 0; e < PW * PW; ++e) acc[e] = 0.0;
+    for (int i0 = 0; i0 < M; i0 += WGR) {
+        const int i = min(i0 + tid, M - 1);
+        const bool own = i0 + tid < M && i >= p0;
+        double v[PW], x[PW];
+#pragma unroll
+        for (int a = 0; a < PW; ++a) v[a] = V[(int64_t)a * M + i];
+        if (c0 != p0) {
+#pragma unroll
+            for (int c = 0; c < PW; ++c) x[c] = B[(int64_t)min(c, cn - 1) * M + i];
+        }
+#pragma unroll
+        for (int a = 0; a < PW; ++a) v[a] = own && i > p0 + a ? v[a] : own && i == p0 + a ? 1.0 : 0.0;
+        if (c0 == p0) {
+#pragma unroll
+            for (int c = 0; c < PW; ++c) x[c] = v[c];
+        }
+#pragma unroll
+        for (int a = 0; a < PW; ++a)
+#pragma unroll
+            for (int c = 0; c < PW; ++c) acc[PW * a + c] += v[a] * x[c];
+    }
+    s.sums[b][wv][lane] = halve_sums<PW * PW>(acc, lane);
+    __syncthreads();
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < NWR; ++w) sum += s.sums[b][w][lane];
+    return sum;
+}
+
+// the panel's reflectors applied to columns c0 .. c0 + cn - 1; S, G as panel_sums
+// leaves them
+__device__ inline void panel_update(const TallView &T, int p0, int c0, int cn, double S, double G) {
+    const int M = T.M, tid = threadIdx.x, lane = tid & 63;
+    const int c = lane & 7, row = lane >> 3;
+    double wl = 0.0;
+#pragma unroll
+    for (int l = 0; l < PW; ++l) {
+        const double wf = __shfl(T.tau[p0 + l] * S, PW * l + c, 64);
+        const double g = __shfl(G, PW * l + row, 64);
+        if (row == l) wl = wf;
+        if (row > l) S -= g * wf;
+    }
+    double *B = T.X + (int64_t)c0 * M;
+    const double *V = T.X + (int64_t)p0 * M;
+    for (int i0 = 0; i0 < M; i0 += 2 * WGR) {
+        double v[2][PW], x[2][PW];
+        int i[2];
+        bool own[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int at = i0 + WGR * u + tid;
+            i[u] = min(at, M - 1);
+            own[u] = at < M && at >= p0;
+#pragma unroll
+            for (int a = 0; a < PW; ++a) v[u][a] = V[(int64_t)a * M + i[u]];
+#pragma unroll
+            for (int q = 0; q < PW; ++q) x[u][q] = B[(int64_t)min(q, cn - 1) * M + i[u]];
+#pragma unroll
+            for (int a = 0; a < PW; ++a)
+                v[u][a] = i[u] > p0 + a ? v[u][a] : i[u] == p0 + a ? 1.0 : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < PW; ++q) {
+#pragma unroll
+            for (int a = 0; a < PW; ++a) {
+                const double w = lane_value(wl, PW * a + q);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) x[u][q] -= v[u][a] * w;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (!own[u]) continue;
+#pragma unroll
+            for (int q = 0; q < PW; ++q)
+                if (q < cn) B[(int64_t)q * M + i[u]] = x[u][q];
+        }
+        if (i0 == 0 && tid >= p0 && tid < p0 + PW) {
+#pragma unroll
+            for (int q = 0; q < PW; ++q)
+                if (q < cn) T.R[tid + LR_MAX * (c0 + q)] = x[0][q];
+        }
+    }
+}
+
+__device__ inline void qr_steps(const TallView &T, QrLds &s) {
+    const int C = T.C;
+    int b = 0;
+    for (int p0 = 0; p0 < C; p0 += PW) {
+        qr_panel(T, p0, min(PW, C - p0), s);
+        if (p0 + PW >= C) break;
+        // tau of the panel, written by the first wavefront
+        __syncthreads();
+        const double G = panel_sums(T, p0, p0, PW, s, b);
+        b ^= 1;
+        for (int c0 = p0 + PW; c0 < C; c0 += PW) {
+            const int cn = min(PW, C - c0);
+            const double S = panel_sums(T, p0, c0, cn, s, b);
+            b ^= 1;
+            panel_update(T, p0, c0, cn, S, G);
+        }
+    }
+    for (int e = threadIdx.x; e < C * C; e += WGR) {
         const int a = e % C, c = e / C;
         if (a > c) T.R[a + LR_MAX * c] = 0.0;
     }
@@ -503,31 +601,20 @@ __device__ inline void wy_steps(const TallView &T, WyLds &s) {
     }
 }
 
-// Rows kept and columns in flight: what 256 registers hold beside the CB sums.
 __global__ __launch_bounds__(WGR) void k_lr_qr(const LRItem *items, double *tall, double *small) {
     const LRItem it = items[blockIdx.x];
     const TallView T = tall_view(it, blockIdx.y, tall, small);
     if (T.C == 0) return;
     __shared__ union Lds {
-        QrLds<16> q16;
-        QrLds<32> q32;
-        QrLds<64> q64;
+        QrLds qr;
         WyLds wy;
         __device__ Lds() {}
     } s;
-    if (T.C <= 16) {
-        qr_steps<16, 4, 16>(T, s.q16);
-        __syncthreads();
-        wy_steps<16>(T, s.wy);
-    } else if (T.C <= 32) {
-        qr_steps<32, 1, 16>(T, s.q32);
-        __syncthreads();
-        wy_steps<32>(T, s.wy);
-    } else {
-        qr_steps<64, 0, 8>(T, s.q64);
-        __syncthreads();
-        wy_steps<64>(T, s.wy);
-    }
+    qr_steps(T, s.qr);
+    __syncthreads();
+    if (T.C <= 16) wy_steps<16>(T, s.wy);
+    else if (T.C <= 32) wy_steps<32>(T, s.wy);
+    else wy_steps<64>(T, s.wy);
 }
 
 // entry (a, b) of the core whose SVD gives the result
