@@ -32,13 +32,13 @@
 // the tree. Single products four times over would form the entries four times;
 // the per-level passes read every level's U, V and F once for four.
 //
-// Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 182 us
-// a product, matrix-free 233 -> 128 us, where the vector instructions alone
+// Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 179 us
+// a product, matrix-free 233 -> 126 us, where the vector instructions alone
 // take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
-// rank 20: 427 -> 60 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
+// rank 20: 427 -> 59 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
 // n = 1000: 27.0 -> 22.7 us. Four right-hand sides, stored log kernel, n = 2^17,
-// leaf 80, rank 20: 349 -> 155 us (the translation, whose log entries of F and
-// of the near field are read, takes 74 of them, the upward pass 53).
+// leaf 80, rank 20: 349 -> 141 us (the translation, whose log entries of F and
+// of the near field are read, takes 58 of them, the upward pass 50).
 #pragma once
 #include "kernels_impl.h"
 
@@ -777,19 +777,21 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
             const int kc = min(k, nq - 1);
             T wl;
             if (R.nslots > 0) {
-                // lane half h sums the slots h, h + 2, ..., sixteen loads in flight
-                const T *ps = partial + (R.pbase * nq + kc) * r + mm;
-                const int64_t ld = (int64_t)nq * r;
+                // lane half h sums the slots h, h + 2, ..., eight loads in flight
+                // at 32-bit offsets (sixteen at 64-bit ones spilled the matrix rows)
+                const T *ps = partial + (R.pbase * nq + kc) * r;
+                const unsigned ld = 2u * nq * r;
+                unsigned at = (unsigned)h * nq * r + mm;
                 T s = T(0);
                 int t = h;
-                for (; t + 30 < R.nslots; t += 32) {
-                    T v[16];
+                for (; t + 14 < R.nslots; t += 16, at += 8 * ld) {
+                    T v[8];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) v[u] = ps[(t + 2 * u) * ld];
+                    for (int u = 0; u < 8; ++u) v[u] = ps[at + u * ld];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) s += v[u];
+                    for (int u = 0; u < 8; ++u) s += v[u];
                 }
-                for (; t < R.nslots; t += 2) s += ps[t * ld];
+                for (; t < R.nslots; t += 2, at += ld) s += ps[at];
                 s += __shfl_xor(s, 32);
                 if (h == 0 && m < RMAX) sw[wv][0][k][m] = m < r ? s : T(0);
                 wave_sync();
