@@ -6,9 +6,14 @@ Workload (one "step" = one product y = H b over the whole matrix):
   (splitmix64 seed 0). The plan (tree + compressed factors) is built and
   resident in HBM before timing; each timed step is one hm_matvec.
 
-Prints one JSON line. `value` is matvecs/s of the stored-factor product; the
-matrix-free variant is reported beside it. `roofline` describes the dominant
-kernel (the downward pass) from HIP events recorded around each pass;
+Prints one JSON line. `value` is matvecs/s of the stored-factor plan's product;
+the matrix-free variant is reported beside it. The single right-hand side's
+product forms the entries of A and F from the points and nodes (as they are
+stored, bit for bit) and never reads U and V, so it is bound by FP64 vector
+issue: `roofline` describes the dominant kernel (the upward launch, which
+carries five ninths of the near field) from HIP events recorded around each
+pass. `bytes_per_matvec` is the counted HBM traffic of a product (see
+`hbm_source`); `bytes_stored` is what the plan holds.
 `cpu_baseline` times the oracle's restatement of the reference mul! on the
 host (bounded sample, see its `sample` field).
 """
@@ -24,7 +29,6 @@ sys.path.insert(0, os.path.join(ROOT, "hierarchicalmatrices.jl_amd"))
 N = 1 << 20
 BS = 256
 RANK = 24
-HBM_PEAK_GBS = 8000.0
 # FP64 vector issue: 1024 SIMDs x 2.4 GHz, one wave64 FP64 instruction per SIMD per 4 cycles
 VALU_F64_PEAK_GINSTR = 614.4
 
@@ -94,27 +98,13 @@ def pass_times(H, fn, steps):
     return ms / max(cnt.value, 1)
 
 
-def pmc_traffic():
-    """HBM bytes per launch of the stored downward pass, from the committed
-    rocprofv3 FETCH_SIZE/WRITE_SIZE summary (scaled by a copy-kernel
-    calibration); None if the summary is absent."""
-    path = os.path.join(ROOT, "profiles", "k_down_cauchy_n2p20_pmc_traffic.md")
+def pmc_figure(name):
+    """A line `name: value` of the committed rocprofv3 counter summary of the
+    n = 2^20 Cauchy products; None if absent."""
+    path = os.path.join(ROOT, "profiles", "n2p20_passes_pmc_counters.md")
     try:
         for line in open(path):
-            if line.startswith("traffic_bytes_per_launch k_down_stored:"):
-                return int(line.split(":")[1])
-    except OSError:
-        pass
-    return None
-
-
-def pmc_valu():
-    """FP64 VALU wave instructions per product of the matrix-free downward
-    pass, from the committed rocprofv3 SQ counter summary; None if absent."""
-    path = os.path.join(ROOT, "profiles", "k_down_matrix_free_n2p20_valu_counters.md")
-    try:
-        for line in open(path):
-            if line.startswith("valu_f64_instr_per_product k_down_free:"):
+            if line.startswith(name + ":"):
                 return int(line.split(":")[1])
     except OSError:
         pass
@@ -1020,32 +1010,23 @@ def main():
         torch.cuda.empty_cache()
 
     names = ["up", "reduce", "translate", "down"]
-    r = RANK
-    bytes_down = 8 * (info["dense_entries"] + r * info["basis_rows_u"]) + 8 * (2 * N)
-    bytes_up = 8 * r * info["basis_rows_v"] + 8 * N
-    ach_down = bytes_down / (passes[3] * 1e-3) / 1e9
-    roof = dict(bound="hbm", kernel="k_down (near field + U z)", achieved=round(ach_down, 1),
-                peak=HBM_PEAK_GBS, unit="GB/s", frac=round(ach_down / HBM_PEAK_GBS, 4),
-                traffic=pmc_traffic(), algorithmic_bytes=bytes_down,
-                traffic_source="profiles/k_down_cauchy_n2p20_pmc_traffic.md (rocprofv3 --pmc)",
-                avg_ms=round(float(passes[3]), 4),
-                up_pass=dict(achieved=round(bytes_up / (passes[0] * 1e-3) / 1e9, 1),
-                             avg_ms=round(float(passes[0]), 4)))
 
-    def valu_roof(down_ms):
-        """The matrix-free downward pass against the FP64 vector-unit issue
-        rate: FP64 VALU wave instructions per product (committed PMC counts)
-        over the live pass time."""
-        instr = pmc_valu()
-        if instr is None or not down_ms:
+    def valu_roof(form, up_ms):
+        """The upward launch against the FP64 vector-unit issue rate: its FP64
+        VALU wave instructions (committed PMC counts) over the live time."""
+        instr = pmc_figure(f"valu_f64_instr_up {form}")
+        if instr is None or not up_ms:
             return None
-        ach = instr / (float(down_ms) * 1e-3) / 1e9
-        return dict(bound="valu", kernel="k_down matrix-free (near field regenerated + far field)",
+        ach = instr / (float(up_ms) * 1e-3) / 1e9
+        return dict(bound="valu", kernel="k_n1_up (moments up the trees + 5/9 of the near field)",
                     achieved=round(ach, 1), peak=VALU_F64_PEAK_GINSTR,
                     unit="G FP64 wave-instructions/s", frac=round(ach / VALU_F64_PEAK_GINSTR, 4),
-                    instructions_per_product=instr, avg_ms=round(float(down_ms), 4),
-                    source="profiles/k_down_matrix_free_n2p20_valu_counters.md (rocprofv3 --pmc)")
+                    instructions_per_launch=instr, avg_ms=round(float(up_ms), 4),
+                    source="profiles/n2p20_passes_pmc_counters.md (rocprofv3 --pmc)")
 
+    moved = pmc_figure("hbm_bytes_per_product stored")
+    # the pass events add a few us of gaps each
+    roof = valu_roof("stored", passes[0])
     workloads = None
     if not args.no_workloads:
         wsteps, wwarm = max(3, min(args.steps, 10)), max(1, min(args.warmup, 2))
@@ -1080,8 +1061,10 @@ def main():
         "config": {"workload": "cauchy_kernelmatrix_matvec", "n": N, "leaf_blocksize": BS,
                    "rank": RANK, "rhs": 1, "layout": "stored, U/V one per cluster",
                    "parallelism": "single GPU"},
-        "hbm_gbs_whole_matvec": round(info["bytes_stored"] / (ms * 1e-3) / 1e9, 1),
-        "bytes_per_matvec": info["bytes_stored"],
+        "hbm_gbs_whole_matvec": moved and round(moved / (ms * 1e-3) / 1e9, 1),
+        "bytes_per_matvec": moved,
+        "hbm_source": "profiles/n2p20_passes_pmc_counters.md (rocprofv3 --pmc)",
+        "bytes_stored": info["bytes_stored"],
         "bytes_ref_layout": info["bytes_ref_layout"],
         "pass_ms": {k: round(float(v), 4) for k, v in zip(names, passes)},
         "pass_ms_method": ("each pass timed with HIP events around its own launches, the "
@@ -1095,11 +1078,11 @@ def main():
                                      f"divides by zero there)" if v["nonfinite"] else None),
                          "unit": "matvecs/s",
                          "ms_per_step": round(v["ms"], 4),
-                         "hbm_bytes_per_matvec": v["bytes"],
+                         "bytes_stored": v["bytes"],
                          "pass_ms": {q: round(float(t), 4) for q, t in zip(names, v["passes"])},
                          "rel_diff_vs_stored": v["err"],
                          "nonfinite_factors": v["nonfinite"],
-                         **({"valu_roofline": valu_roof(v["passes"][3])}
+                         **({"valu_roofline": valu_roof("matrix_free", v["passes"][0])}
                             if k == "matrix_free" else {})} for k, v in variants.items()},
         "roofline": roof,
         "workloads": workloads,
