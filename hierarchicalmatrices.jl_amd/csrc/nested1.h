@@ -1005,6 +1005,24 @@ __global__ __launch_bounds__(WG) void k_n1_down(N1Side o, const T *pts_out, cons
     }
 }
 
+// workgroups of the translation; light clusters: at most four wavefronts per
+// SIMD, looping
+inline int n1_ntranslate(const N1Side &out) {
+    return out.nheavy + std::min((out.ncl - out.nheavy + WPB - 1) / WPB, 1024);
+}
+
+// the two launches without the near field (its workgroups: none)
+template <class T, int RMAX, int KID, bool TR>
+void n1_chain(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s) {
+    const N1Side &in = TR ? p.n1x : p.n1y, &out = TR ? p.n1y : p.n1x;
+    const T *in_pts = TR ? p.x : p.y, *out_pts = TR ? p.y : p.x;
+    const int ntr = n1_ntranslate(out);
+    k_n1_up<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(in.nsub, 0), WG, 0, s>>>(
+        in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, 1, in.nsub, 0, 0);
+    k_n1_translate<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(ntr, 0), WG, 0, s>>>(
+        p, out, in_pts, out_pts, a, 1, ntr, 0, 0);
+}
+
 // One product y = beta*y + op(H) x of nq <= KB right-hand sides over the
 // interval trees. Many chunks of stored entries stream through k_down's near part,
 // on the side stream when there is one.
@@ -1064,8 +1082,7 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, int nq, hipStr
     mark(1);
     mark(2);
     if (far) {
-        // light clusters: at most four wavefronts per SIMD, looping
-        const int ntr = out.nheavy + std::min((out.ncl - out.nheavy + WPB - 1) / WPB, 1024);
+        const int ntr = n1_ntranslate(out);
         k_n1_translate<T, RMAX, SRC, KID, TR, KB><<<n1_grid(ntr, nb - nb0), WG, 0, s>>>(
             p, out, in_pts, out_pts, a, nq, ntr, nb0, nb - nb0);
     }

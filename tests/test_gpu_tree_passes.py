@@ -233,3 +233,18 @@ def test_several_rhs_units(cuda, kernel, form):
         b = B[:, q].contiguous()
         assert ((u[:, q] - H @ b).norm() / u[:, q].norm()).item() <= 1e-13
         assert ((v[:, q] - H.T @ b).norm() / v[:, q].norm()).item() <= 1e-13
+
+
+@pytest.mark.parametrize("kernel", ["cauchykernel", "coulombkernel", "coulombprimekernel", "logkernel"])
+@pytest.mark.parametrize("n,bs,r", [(50, 80, 20), (900, 40, 9), (2501, 64, 16), (40001, 64, 32)])
+def test_gradient_chain(cuda, kernel, n, bs, r):
+    # the gradient passes' far field over the trees, both directions, against the
+    # matrix-free products (the same terms, summed in another order: 1e-13)
+    x, y, iv = points(n, "random", n)
+    H = hmx.KernelMatrix(kernel, x, y, *iv, blocksize=bs, rank=r, matrix_free=True)
+    g = torch.Generator(device=cuda).manual_seed(n)
+    b, q = (torch.randn(n, dtype=torch.float64, device=cuda, generator=g) for _ in range(2))
+    u, _ = H.matvec_grad(b)
+    gb, _ = H.tgrad(q, b)
+    for got, want in ((u, H @ b), (gb, H.T @ q)):
+        assert ((got - want).norm() / want.norm()).item() <= 1e-13
