@@ -33,7 +33,7 @@
 // the per-level passes read every level's U, V and F once for four.
 //
 // Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 179 us
-// a product, matrix-free 233 -> 126 us, where the vector instructions alone
+// a product, matrix-free 233 -> 130 us, where the vector instructions alone
 // take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
 // rank 20: 427 -> 59 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
 // n = 1000: 27.0 -> 22.7 us. Four right-hand sides, stored log kernel, n = 2^17,
@@ -117,53 +117,74 @@ __device__ __forceinline__ float rcp_refine(float d, float r) {
 }
 
 // acc_i + sum_{u < N} f(p_i, q_u) v_u for NR rows (f(q_u, p_i) when TR).
-// 1/d^m: the terms of four columns over one common denominator, v0/d0 + v1/d1
-// = (v0 d1 + v1 d0) / (d0 d1) twice over. If a denominator leaves the normal
-// range (its reciprocal is zero, denormal, infinite or NaN) the lane forms its
-// terms one by one; one test for all of the denominators, so that their chains
-// run side by side (a branch each: n = 2^20 spent 45 us more). FP32 holds four
-// factors of 1/d only; its other powers share a reciprocal between two.
-// EXACT: term by term. The refined reciprocal is 1/d^m rounded as a division
-// rounds it: before its last step it is within 2^-48, and that step's own
-// error is the final rounding.
+// 1/d^m: four columns share the reciprocal of their denominators' product, and
+// each pair's is taken out of it, 1/(d0 d1) = d2 d3 / (d0 d1 d2 d3), before it
+// meets the inputs: v0/d0 + v1/d1 = (v0 d1 + v1 d0) / (d0 d1), a numerator of
+// v d. (Over one common denominator it is v d^3, which leaves the range where
+// every term lies within it: Float32 inputs of 1e-28 at n = 2^20 lost 5 %.) FP32,
+// whose range v d leaves too, takes each term's own reciprocal, d1 / (d0 d1); its
+// d^2 and d^3 share one between two columns only. If a reciprocal (FP32: or a
+// denominator) leaves the normal range (zero, denormal, infinite or NaN) the lane
+// forms its terms one by one; one test for all of the columns, so that their
+// chains run side by side (a branch each: n = 2^20 spent 45 us more). n = 2^20,
+// leaf 256, rank 24: 130 us (common denominator 126, each term's own 144).
+// Float32, leaf 64, rank 16: 96 us (90, pairs 91).
+// EXACT: term by term. The reciprocal's last step starts within 2^-48 (FP32
+// 2^-22) of it, so the result is a division's but for rare half-way cases
+// (<= 1 ulp).
 template <class T, int KID, bool TR, bool EXACT, int N, int NR>
 __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T *acc) {
     if constexpr (KID <= 2 && !EXACT) {
         constexpr int S = (sizeof(T) == 8 || KID == 0) ? 4 : 2, G = N / S;
-        T num[NR][G], den[NR][G], r[NR][G];
+        T sum[NR];
         bool odd = false;
         auto dist = [&](int i, int u) {
             const T e = TR ? q[u] - p[i] : p[i] - q[u];
             return KID == 0 ? e : KID == 1 ? e * e : e * e * e;
         };
+        // v0/d0 + v1/d1 added on, r = 1/(d0 d1)
+        auto pair = [&](int i, int u, T r, T d0, T d1) {
+            if constexpr (sizeof(T) == 8) {
+                sum[i] = fmaT(fmaT(v[u], d1, v[u + 1] * d0), r, sum[i]);
+            } else {
+                sum[i] = fmaT(r * d1, v[u], sum[i]);
+                sum[i] = fmaT(r * d0, v[u + 1], sum[i]);
+            }
+        };
+        auto test = [&](T r, T a, T b) {
+            odd |= odd_class(r);
+            if constexpr (sizeof(T) == 4) {
+                odd |= odd_class(a);
+                odd |= odd_class(b);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NR; ++i) sum[i] = acc[i];
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
                 const int u = g * S;
-                const T d0 = dist(i, u), d1 = dist(i, u + 1);
-                T n = fmaT(v[u], d1, v[u + 1] * d0), d = d0 * d1;
+                const T d0 = dist(i, u), d1 = dist(i, u + 1), a = d0 * d1;
                 if constexpr (S == 4) {
-                    const T d2 = dist(i, u + 2), d3 = dist(i, u + 3);
-                    const T n2 = fmaT(v[u + 2], d3, v[u + 3] * d2), e = d2 * d3;
-                    n = fmaT(n, e, n2 * d);
-                    d = d * e;
+                    const T d2 = dist(i, u + 2), d3 = dist(i, u + 3), b = d2 * d3;
+                    const T r0 = rcp_raw(a * b), r = rcp_refine(a * b, r0);
+                    test(r0, a, b);
+                    pair(i, u, r * b, d0, d1);
+                    pair(i, u + 2, r * a, d2, d3);
+                } else {
+                    const T r0 = rcp_raw(a);
+                    test(r0, a, a);
+                    pair(i, u, rcp_refine(a, r0), d0, d1);
                 }
-                num[i][g] = n;
-                den[i][g] = d;
-                r[i][g] = rcp_raw(d);
-                odd |= odd_class(r[i][g]);
             }
         if (__builtin_expect(odd, 0)) {
             for (int i = 0; i < NR; ++i)
 #pragma unroll
-                for (int u = 0; u < N; ++u) acc[i] = fmaT(rcpT(dist(i, u)), v[u], acc[i]);
+                for (int u = 0; u < N; ++u) acc[i] = fmaT(T(1) / dist(i, u), v[u], acc[i]);
         } else {
 #pragma unroll
-            for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int i = 0; i < NR; ++i)
-                    acc[i] = fmaT(num[i][g], rcp_refine(den[i][g], r[i][g]), acc[i]);
+            for (int i = 0; i < NR; ++i) acc[i] = sum[i];
         }
     } else {
 #pragma unroll
