@@ -33,7 +33,7 @@
 // the per-level passes read every level's U, V and F once for four.
 //
 // Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 179 us
-// a product, matrix-free 233 -> 130 us, where the vector instructions alone
+// a product, matrix-free 233 -> 126 us, where the vector instructions alone
 // take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
 // rank 20: 427 -> 59 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
 // n = 1000: 27.0 -> 22.7 us. Four right-hand sides, stored log kernel, n = 2^17,
@@ -124,20 +124,23 @@ __device__ __forceinline__ float rcp_refine(float d, float r) {
 // every term lies within it: Float32 inputs of 1e-28 at n = 2^20 lost 5 %.) FP32,
 // whose range v d leaves too, takes each term's own reciprocal, d1 / (d0 d1); its
 // d^2 and d^3 share one between two columns only. If a reciprocal (FP32: or a
-// denominator) leaves the normal range (zero, denormal, infinite or NaN) the lane
-// forms its terms one by one; one test for all of the columns, so that their
-// chains run side by side (a branch each: n = 2^20 spent 45 us more). n = 2^20,
-// leaf 256, rank 24: 130 us (common denominator 126, each term's own 144).
-// Float32, leaf 64, rank 16: 96 us (90, pairs 91).
+// denominator) leaves the normal range (zero, denormal, infinite or NaN) it
+// returns true, and the caller forms its sum again from where it began, term by
+// term (near_single). No branch between the columns, whose chains then run side
+// by side: a branch for each four took 45 us more at n = 2^20, one for each
+// eight 4. n = 2^20, leaf 256, rank 24: Cauchy 126 us, Coulomb 147 (common
+// denominator 126 and 140); Float32, leaf 64, rank 16: 96 us (90).
 // EXACT: term by term. The reciprocal's last step starts within 2^-48 (FP32
 // 2^-22) of it, so the result is a division's but for rare half-way cases
 // (<= 1 ulp).
+// log: columns outside lo <= u < hi are padding, which adds nothing (a repeated
+// column that meets the row's point has an infinite value).
 template <class T, int KID, bool TR, bool EXACT, int N, int NR>
-__device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T *acc) {
+__device__ __forceinline__ bool near_terms(const T *p, const T *q, const T *v, T *acc, int lo,
+                                           int hi) {
+    bool odd = false;
     if constexpr (KID <= 2 && !EXACT) {
         constexpr int S = (sizeof(T) == 8 || KID == 0) ? 4 : 2, G = N / S;
-        T sum[NR];
-        bool odd = false;
         auto dist = [&](int i, int u) {
             const T e = TR ? q[u] - p[i] : p[i] - q[u];
             return KID == 0 ? e : KID == 1 ? e * e : e * e * e;
@@ -145,10 +148,10 @@ __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T
         // v0/d0 + v1/d1 added on, r = 1/(d0 d1)
         auto pair = [&](int i, int u, T r, T d0, T d1) {
             if constexpr (sizeof(T) == 8) {
-                sum[i] = fmaT(fmaT(v[u], d1, v[u + 1] * d0), r, sum[i]);
+                acc[i] = fmaT(fmaT(v[u], d1, v[u + 1] * d0), r, acc[i]);
             } else {
-                sum[i] = fmaT(r * d1, v[u], sum[i]);
-                sum[i] = fmaT(r * d0, v[u + 1], sum[i]);
+                acc[i] = fmaT(r * d1, v[u], acc[i]);
+                acc[i] = fmaT(r * d0, v[u + 1], acc[i]);
             }
         };
         auto test = [&](T r, T a, T b) {
@@ -158,8 +161,6 @@ __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T
                 odd |= odd_class(b);
             }
         };
-#pragma unroll
-        for (int i = 0; i < NR; ++i) sum[i] = acc[i];
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -178,22 +179,32 @@ __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T
                     pair(i, u, rcp_refine(a, r0), d0, d1);
                 }
             }
-        if (__builtin_expect(odd, 0)) {
-            for (int i = 0; i < NR; ++i)
-#pragma unroll
-                for (int u = 0; u < N; ++u) acc[i] = fmaT(T(1) / dist(i, u), v[u], acc[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < NR; ++i) acc[i] = sum[i];
-        }
     } else {
 #pragma unroll
         for (int u = 0; u < N; ++u)
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
                 const T f = TR ? kern_fast<T, KID>(q[u], p[i]) : kern_fast<T, KID>(p[i], q[u]);
-                acc[i] = fmaT(f, v[u], acc[i]);
+                const T t = fmaT(f, v[u], acc[i]);
+                acc[i] = KID <= 2 || (u >= lo && u < hi) ? t : acc[i];
             }
+    }
+    return odd;
+}
+
+// acc_i + sum_u f(p_i, q_u) v_u over the columns n0 <= u < n1 that col(u, q, v)
+// reads, each term a division (1/d^m) of its own
+template <class T, int KID, bool TR, int NR, class Col>
+__device__ __forceinline__ void near_single(const T *p, int n0, int n1, Col col, T *acc) {
+#pragma unroll 1
+    for (int u = n0; u < n1; ++u) {
+        T q, v;
+        col(u, q, v);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const T d = TR ? q - p[i] : p[i] - q;
+            acc[i] = fmaT(T(1) / (KID == 0 ? d : KID == 1 ? d * d : d * d * d), v, acc[i]);
+        }
     }
 }
 
@@ -202,14 +213,17 @@ __device__ __forceinline__ void near_terms(const T *p, const T *q, const T *v, T
 // formed for each of them)
 template <class T, int KID, bool TR, int N, int NR, int KB>
 __device__ __forceinline__ void near_terms_kb(const T *p, const T *q, const T (*v)[KB],
-                                              T (*acc)[KB]) {
+                                              T (*acc)[KB], int lo, int hi) {
 #pragma unroll
     for (int u = 0; u < N; ++u)
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             const T f = TR ? kern_fast<T, KID>(q[u], p[i]) : kern_fast<T, KID>(p[i], q[u]);
 #pragma unroll
-            for (int k = 0; k < KB; ++k) acc[i][k] = fmaT(f, v[u][k], acc[i][k]);
+            for (int k = 0; k < KB; ++k) {
+                const T t = fmaT(f, v[u][k], acc[i][k]);
+                acc[i][k] = KID <= 2 || (u >= lo && u < hi) ? t : acc[i][k];
+            }
         }
 }
 
@@ -239,6 +253,8 @@ __device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, cons
             return TR ? Ar[(int64_t)(j >> 6) * HM_TILE * R.cols + (j & (HM_TILE - 1))]
                       : Ar[j * HM_TILE];
         };
+        const T acc0 = acc[0];
+        bool odd = false;
         for (int t = b0; N * t < R.n; t += bs) {
             T q[N], v[N][KB];
             const int j0 = R.n >= N ? min(N * t, R.n - N) : 0;
@@ -289,10 +305,23 @@ __device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, cons
                     T w[N];
 #pragma unroll
                     for (int u = 0; u < N; ++u) w[u] = v[u][0];
-                    near_terms<T, KID, TR, SRC == N1_EXACT, N, 1>(&p, q, w, acc);
+                    odd |= near_terms<T, KID, TR, SRC == N1_EXACT, N, 1>(&p, q, w, acc, N * t - j0,
+                                                                         R.n - j0);
                 } else {
-                    near_terms_kb<T, KID, TR, N, 1, KB>(&p, q, v, &acc);
+                    near_terms_kb<T, KID, TR, N, 1, KB>(&p, q, v, &acc, N * t - j0, R.n - j0);
                 }
+            }
+        }
+        if constexpr (KB == 1 && KID <= 2 && SRC == N1_FREE) {
+            if (__builtin_expect(odd, 0)) {
+                acc[0] = acc0;
+                for (int t = b0; N * t < R.n; t += bs)
+                    near_single<T, KID, TR, 1>(&p, N * t, min(N * t + N, R.n),
+                                               [&](int u, T &qu, T &vu) {
+                                                   qu = qs[u];
+                                                   vu = vs[u * incx];
+                                               },
+                                               acc);
             }
         }
     }
@@ -307,12 +336,16 @@ struct NearCol {
     T q, v[KB];
 };
 
-// the sums of a tile's n columns (a multiple of eight, padded at weight zero)
+// the sums of a tile's n columns (padded at weight zero to a multiple of eight)
 // for one or both rows
 template <class T, int KID, bool TR, bool EXACT, int NR, int KB>
 __device__ __forceinline__ void near_tile(const NearCol<T, KB> *t, int n, const T (&p)[NR],
                                           T (&acc)[NR][KB]) {
     constexpr int N = KID == 3 || KB > 1 ? 2 : 8;
+    T acc0[NR];
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) acc0[i] = acc[i][0];
     for (int j = 0; j < n; j += N) {
         T q[N], v[N][KB];
 #pragma unroll
@@ -328,11 +361,21 @@ __device__ __forceinline__ void near_tile(const NearCol<T, KB> *t, int n, const 
             for (int u = 0; u < N; ++u) w[u] = v[u][0];
 #pragma unroll
             for (int i = 0; i < NR; ++i) s[i] = acc[i][0];
-            near_terms<T, KID, TR, EXACT, N, NR>(p, q, w, s);
+            odd |= near_terms<T, KID, TR, EXACT, N, NR>(p, q, w, s, 0, n - j);
 #pragma unroll
             for (int i = 0; i < NR; ++i) acc[i][0] = s[i];
         } else {
-            near_terms_kb<T, KID, TR, N, NR, KB>(p, q, v, acc);
+            near_terms_kb<T, KID, TR, N, NR, KB>(p, q, v, acc, 0, n - j);
+        }
+    }
+    if constexpr (KB == 1 && KID <= 2 && !EXACT) {
+        if (__builtin_expect(odd, 0)) {
+            near_single<T, KID, TR, NR>(p, 0, n, [&](int u, T &qu, T &vu) {
+                qu = t[u].q;
+                vu = t[u].v[0];
+            }, acc0);
+#pragma unroll
+            for (int i = 0; i < NR; ++i) acc[i][0] = acc0[i];
         }
     }
 }
@@ -372,15 +415,14 @@ __device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const
             if (++e < nrun) R = sload_struct(runs + e);
         }
         if (e < nrun) load(R, j, c);
-        const int n8 = (n + 7) & ~7;
         if (mask == 3) {
-            near_tile<T, KID, TR, EXACT, 2, KB>(t, n8, p, acc);
+            near_tile<T, KID, TR, EXACT, 2, KB>(t, n, p, acc);
         } else {
             const T p1[1] = {mask == 1 ? p[0] : p[1]};
             T a1[1][KB];
 #pragma unroll
             for (int k = 0; k < KB; ++k) a1[0][k] = mask == 1 ? acc[0][k] : acc[1][k];
-            near_tile<T, KID, TR, EXACT, 1, KB>(t, n8, p1, a1);
+            near_tile<T, KID, TR, EXACT, 1, KB>(t, n, p1, a1);
 #pragma unroll
             for (int k = 0; k < KB; ++k) {
                 if (mask == 1) acc[0][k] = a1[0][k];
@@ -716,10 +758,24 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     // ws: zero past r (and past nq); ts: past r repeats
     auto apply = [&](const T (*ws)[RMAX], const T *ts, int64_t foff) {
         if constexpr (FREE && KB == 1) {
+            const T acc0 = acc[0];
+            const int l0 = h * HALF;
+            bool odd = false;
 #pragma unroll
             for (int j = 0; j < HALF; j += NT)
-                near_terms<T, KID, TRANS, SRC == N1_EXACT, NT, 1>(&to, ts + h * HALF + j,
-                                                                  ws[0] + h * HALF + j, acc);
+                odd |= near_terms<T, KID, TRANS, SRC == N1_EXACT, NT, 1>(
+                    &to, ts + l0 + j, ws[0] + l0 + j, acc, 0, r - l0 - j);
+            if constexpr (KID <= 2 && SRC == N1_FREE) {
+                if (__builtin_expect(odd, 0)) {
+                    acc[0] = acc0;
+                    near_single<T, KID, TRANS, 1>(&to, l0, min(l0 + HALF, r),
+                                                  [&](int u, T &qu, T &vu) {
+                                                      qu = ts[u];
+                                                      vu = ws[0][u];
+                                                  },
+                                                  acc);
+                }
+            }
         } else {
             const T *F = p.F + foff;
             T fv[HALF];
@@ -736,7 +792,8 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
 #pragma unroll
             for (int j = 0; j < HALF; ++j)
 #pragma unroll
-                for (int k = 0; k < KB; ++k) acc[k] = fmaT(fv[j], ws[k][h * HALF + j], acc[k]);
+                for (int k = 0; k < KB; ++k)
+                    acc[k] = fmaT(h * HALF + j < r ? fv[j] : T(0), ws[k][h * HALF + j], acc[k]);
         }
     };
     auto put_z = [&] {  // this wavefront's sums into its zr
