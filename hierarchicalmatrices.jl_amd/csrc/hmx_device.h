@@ -66,7 +66,15 @@ struct DevPlanT {
     int32_t nrtask, nctask;
     int64_t nslots_r, nslots_c;
     T *A, *U, *V, *F;          // stored factors (null when matrix-free)
-    int32_t *uv_bad;           // set to 1 when a formed value of U or V is not finite
+    // Written with the factors, at construction and after new points (null when
+    // matrix-free or from blocks), read by the tree passes of one to four
+    // right-hand sides: odd[0] a value of U or V is not finite, odd[1] a dense
+    // entry and odd[2] an entry of F of 1/d^m is outside the range in which the
+    // passes form it as it is stored. Where odd[0]: bad_x, bad_y mark the points
+    // with such a value (of U, V) and bad_rc, bad_cc the clusters (null: hybrid).
+    int32_t *odd;
+    uint8_t *bad_x, *bad_y, *bad_rc, *bad_cc;
+    int64_t nodd;              // words from odd on that are cleared first
     // the row / column clusters with more than one upward task (the others'
     // tasks write w themselves)
     const int32_t *multi_r, *multi_c;
@@ -119,6 +127,7 @@ struct MvArgsT {
     // yt beside the near field first)
     hipStream_t side;
     hipEvent_t fork, join;
+    int basis;  // a stored product over the trees: values of U and V that are not finite count
 };
 
 using DevPlan = DevPlanT<double>;

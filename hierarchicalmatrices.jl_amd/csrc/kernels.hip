@@ -7,6 +7,7 @@
 hipError_t hmx_launch_compress(const DevPlan &p, hipStream_t s) {
     // HM_USER plans take A and F from the caller (hm_plan_set_leaf_data)
     const bool gen = p.kid != HM_USER;
+    hmxk::clear_odd(p, s);
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<double><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<double><<<p.nfar, hmxk::WG, 0, s>>>(p);
     if (p.U && p.V && p.nrc + p.ncc > 0)
@@ -82,6 +83,7 @@ hipError_t hmx_launch_matvec_m(const DevPlan &p, const MvArgs &a, int mode, int 
 
 hipError_t hmx_launch_compress(const DevPlanF &p, hipStream_t s) {
     const bool gen = p.kid != HM_USER;
+    hmxk::clear_odd(p, s);
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<float><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<float><<<p.nfar, hmxk::WG, 0, s>>>(p);
     if (p.U && p.V && p.nrc + p.ncc > 0)
@@ -239,6 +241,7 @@ template hipError_t hmx_launch_update_points<float>(const float *, float *, int6
                                                     hipStream_t);
 
 hipError_t hmx_launch_refit(const DevPlan &p, hipStream_t s) {
+    hmxk::clear_odd(p, s);
     if (p.kid != HM_USER && p.ndense > 0 && p.A) hmxk::k_gen_dense<double><<<p.ndense, hmxk::WG, 0, s>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || (!p.U && !p.V)) return err;
@@ -251,6 +254,7 @@ hipError_t hmx_launch_refit(const DevPlan &p, hipStream_t s) {
 }
 
 hipError_t hmx_launch_refit(const DevPlanF &p, hipStream_t s) {
+    hmxk::clear_odd(p, s);
     if (p.kid != HM_USER && p.ndense > 0 && p.A) hmxk::k_gen_dense<float><<<p.ndense, hmxk::WG, 0, s>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || (!p.U && !p.V)) return err;

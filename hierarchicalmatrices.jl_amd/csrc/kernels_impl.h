@@ -216,6 +216,15 @@ struct HalveShape<P, 0, OMIN> {
 
 // ------------------------------------------------------------- compression
 
+// The range in which the tree passes form an entry of 1/d^m as it is stored
+// (nested1.h): there d^m, its reciprocal and the reciprocal's refinement are
+// normal numbers.
+template <class T>
+__device__ __forceinline__ bool formable(T v) {
+    const T a = fabsT(v);
+    return a >= (sizeof(T) == 8 ? (T)1e-300 : (T)1e-36) && a <= (sizeof(T) == 8 ? (T)1e300 : (T)1e36);
+}
+
 // One dense block per workgroup, tile by tile: a wavefront writes a column's 64
 // rows of a tile (one contiguous run), the rows past the block's last as
 // zeros, so the padding needs no pass of its own (every array was cleared
@@ -231,6 +240,7 @@ __global__ __launch_bounds__(WG) void k_gen_dense(DevPlanT<T> p) {
         for (int32_t j = threadIdx.x / WAVE; j < D.n; j += WPB) {
             const T v = kern_exact<T>(p.kid, xi, p.y[D.col0 + j]);
             a[(int64_t)j * HM_TILE] = ok ? v : T(0);
+            if (ok && p.kid <= 2 && !formable(v)) p.odd[1] = 1;
         }
     }
 }
@@ -249,12 +259,14 @@ __global__ __launch_bounds__(WAVE) void k_pad_basis(DevPlanT<T> p) {
 }
 
 // update! (src/BarycentricMatrix.jl:256-287): one lane per point of a chunk,
-// for every cluster covering the chunk. *bad = 1 where a value is not finite.
+// for every cluster covering the chunk. A value that is not finite sets *odd
+// and marks its point and its cluster.
 template <class T, int RMAX>
 __global__ __launch_bounds__(WG) void k_gen_basis(const DChunk *ch, int nch, const DFar *fl,
                                                  const DCluster *cl, const T *nodes,
                                                  const T *lam, const T *pts,
-                                                 T *B, int r, int32_t *bad) {
+                                                 T *B, int r, int32_t *odd,
+                                                 uint8_t *bad_pt, uint8_t *bad_cl) {
 #pragma clang fp contract(off)
     const int wid = wave_id();
     const int lane = threadIdx.x % WAVE;
@@ -283,7 +295,11 @@ __global__ __launch_bounds__(WG) void k_gen_basis(const DChunk *ch, int nch, con
                 out[k * HM_TILE] = v;
                 fin = fin && isfinite(v);
             }
-        if (!fin) *bad = 1;
+        if (!fin) {
+            *odd = 1;
+            bad_pt[c.p0 + lane] = 1;
+            bad_cl[f.cl] = 1;
+        }
     }
 }
 
@@ -296,13 +312,25 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
     const T *ty = p.cnodes + (int64_t)b.cc * r;
     for (int e = threadIdx.x; e < r * r; e += WG) {
         int n = e / r, m = e - n * r;
-        p.F[b.foff + e] = kern_exact<T>(p.kid, tx[m], ty[n]);
+        const T v = kern_exact<T>(p.kid, tx[m], ty[n]);
+        p.F[b.foff + e] = v;
+        if (p.kid <= 2 && !formable(v)) p.odd[2] = 1;
     }
 }
 
-// Per workgroup (gridDim.x of them) and array (blockIdx.y, up to four): the
-// non-finite values (low half of the word) and the finite ones within 10^8
-// (10^2 for float) of the largest number (high half, one per thread at most)
+// DevPlanT's odd words and marks, before the factors are formed
+__global__ __launch_bounds__(WG) void k_clear_words(int32_t *w, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG)
+        w[i] = 0;
+}
+template <class T>
+void clear_odd(const DevPlanT<T> &p, hipStream_t s) {
+    if (p.nodd > 0)
+        k_clear_words<<<(int)(p.nodd < 256 * WG ? (p.nodd + WG - 1) / WG : 256), WG, 0, s>>>(p.odd, p.nodd);
+}
+
+// Non-finite values of up to four arrays, one count per workgroup (gridDim.x of
+// them) and array (blockIdx.y)
 template <class T>
 struct CountArgs {
     const T *v[4];
@@ -311,17 +339,12 @@ struct CountArgs {
 template <class T>
 __global__ __launch_bounds__(WG) void k_count_nonfinite(CountArgs<T> a,
                                                         unsigned long long *blockcount) {
-    __shared__ unsigned long long sh[WG];
+    __shared__ unsigned int sh[WG];
     const T *v = a.v[blockIdx.y];
     const int64_t n = a.n[blockIdx.y];
-    const T lim = sizeof(T) == 8 ? (T)1e300 : (T)1e36;
-    unsigned int low = 0, high = 0;
-    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
-        const T q = v[i];
-        low += isfinite(q) ? 0u : 1u;
-        high |= isfinite(q) && fabsT(q) > lim ? 1u : 0u;
-    }
-    const unsigned long long cnt = (unsigned long long)low | ((unsigned long long)high << 32);
+    unsigned int cnt = 0;
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG)
+        cnt += isfinite(v[i]) ? 0u : 1u;
     sh[threadIdx.x] = cnt;
     __syncthreads();
     for (int o = WG / 2; o > 0; o /= 2) {
@@ -1051,17 +1074,14 @@ inline int64_t tr_waves(int64_t ncl, int r, int kb) {
     return (ncl + G - 1) / G;
 }
 
-__global__ void k_clear_word(int32_t *w) { *w = 0; }
-
 template <class T, int RMAX>
 hipError_t gen_basis_r(const DevPlanT<T> &p, hipStream_t s) {
-    k_clear_word<<<1, 1, 0, s>>>(p.uv_bad);
     if (p.ncch > 0 && p.V)
         k_gen_basis<T, RMAX><<<nblk(p.ncch), WG, 0, s>>>(p.cch, p.ncch, p.cfar, p.ccl, p.cnodes, p.lam,
-                                                     p.y, p.V, p.r, p.uv_bad);
+                                                     p.y, p.V, p.r, p.odd, p.bad_y, p.bad_cc);
     if (p.nrch > 0 && p.U)
         k_gen_basis<T, RMAX><<<nblk(p.nrch), WG, 0, s>>>(p.rch, p.nrch, p.rfar, p.rcl, p.rnodes, p.lam,
-                                                     p.x, p.U, p.r, p.uv_bad);
+                                                     p.x, p.U, p.r, p.odd, p.bad_x, p.bad_rc);
     return hipGetLastError();
 }
 

@@ -53,7 +53,12 @@ namespace {
 //             reciprocal (matrix-free products)
 //   N1_EXACT  formed term by term, as the stored entries are rounded, and summed
 //             in the order of N1_READ: a stored or hybrid plan of 1/d^m, whose
-//             values it saves reading
+//             values it saves reading. New points may bring entries that the
+//             refined reciprocal does not give (points that meet, distances out
+//             of range): the plan's word odd[1], written with the entries and
+//             read here, then has every value formed by division. So the route
+//             hangs on nothing that the host would have to wait for, and a
+//             captured product holds for later points too.
 //   N1_READ   the stored entries (the log kernel, a caller's f, entries that
 //             are not all finite)
 
@@ -192,18 +197,20 @@ __device__ __forceinline__ bool near_terms(const T *p, const T *q, const T *v, T
     return odd;
 }
 
-// acc_i + sum_u f(p_i, q_u) v_u over the columns n0 <= u < n1 that col(u, q, v)
-// reads, each term a division (1/d^m) of its own
-template <class T, int KID, bool TR, int NR, class Col>
-__device__ __forceinline__ void near_single(const T *p, int n0, int n1, Col col, T *acc) {
+// acc[i][k] + sum_u f(p_i, q_u) v[u][k] over the columns n0 <= u < n1 that
+// col(u, q, v) reads, each value of 1/d^m a division of its own
+template <class T, int KID, bool TR, int NR, int KB, class Col>
+__device__ __forceinline__ void near_single(const T *p, int n0, int n1, Col col, T (*acc)[KB]) {
 #pragma unroll 1
     for (int u = n0; u < n1; ++u) {
-        T q, v;
+        T q, v[KB];
         col(u, q, v);
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             const T d = TR ? q - p[i] : p[i] - q;
-            acc[i] = fmaT(T(1) / (KID == 0 ? d : KID == 1 ? d * d : d * d * d), v, acc[i]);
+            const T f = T(1) / (KID == 0 ? d : KID == 1 ? d * d : d * d * d);
+#pragma unroll
+            for (int k = 0; k < KB; ++k) acc[i][k] = fmaT(f, v[k], acc[i][k]);
         }
     }
 }
@@ -237,7 +244,7 @@ __device__ __forceinline__ void near_terms_kb(const T *p, const T *q, const T (*
 template <class T, int KID, bool TR, int SRC, int KB>
 __device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, const T *pts_in,
                                           const T *A, const T *x, int64_t incx, int64_t ldx, int nq,
-                                          int row, int b0, int bs, T (&acc)[KB]) {
+                                          int row, int b0, int bs, bool single, T (&acc)[KB]) {
     constexpr int N = KB == 1 ? 8 : 4;
 #pragma unroll
     for (int k = 0; k < KB; ++k) acc[k] = T(0);
@@ -253,9 +260,11 @@ __device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, cons
             return TR ? Ar[(int64_t)(j >> 6) * HM_TILE * R.cols + (j & (HM_TILE - 1))]
                       : Ar[j * HM_TILE];
         };
-        const T acc0 = acc[0];
-        bool odd = false;
-        for (int t = b0; N * t < R.n; t += bs) {
+        T acc0[1][KB];
+#pragma unroll
+        for (int k = 0; k < KB; ++k) acc0[0][k] = acc[k];
+        bool odd = single;
+        for (int t = b0; N * t < R.n && !single; t += bs) {
             T q[N], v[N][KB];
             const int j0 = R.n >= N ? min(N * t, R.n - N) : 0;
             if (KB == 1 && R.n >= N && incx == 1) {
@@ -312,16 +321,19 @@ __device__ __forceinline__ void near_runs(const N1Run *runs, int nrun, T p, cons
                 }
             }
         }
-        if constexpr (KB == 1 && KID <= 2 && SRC == N1_FREE) {
+        if constexpr (KID <= 2 && SRC != N1_READ) {
             if (__builtin_expect(odd, 0)) {
-                acc[0] = acc0;
                 for (int t = b0; N * t < R.n; t += bs)
-                    near_single<T, KID, TR, 1>(&p, N * t, min(N * t + N, R.n),
-                                               [&](int u, T &qu, T &vu) {
-                                                   qu = qs[u];
-                                                   vu = vs[u * incx];
-                                               },
-                                               acc);
+                    near_single<T, KID, TR, 1, KB>(&p, N * t, min(N * t + N, R.n),
+                                                   [&](int u, T &qu, T (&vu)[KB]) {
+                                                       qu = qs[u];
+#pragma unroll
+                                                       for (int k = 0; k < KB; ++k)
+                                                           vu[k] = vs[u * incx + min(k, nq - 1) * ldx];
+                                                   },
+                                                   acc0);
+#pragma unroll
+                for (int k = 0; k < KB; ++k) acc[k] = acc0[0][k];
             }
         }
     }
@@ -340,13 +352,15 @@ struct NearCol {
 // for one or both rows
 template <class T, int KID, bool TR, bool EXACT, int NR, int KB>
 __device__ __forceinline__ void near_tile(const NearCol<T, KB> *t, int n, const T (&p)[NR],
-                                          T (&acc)[NR][KB]) {
+                                          bool single, T (&acc)[NR][KB]) {
     constexpr int N = KID == 3 || KB > 1 ? 2 : 8;
-    T acc0[NR];
-    bool odd = false;
+    T acc0[NR][KB];
+    bool odd = single;
 #pragma unroll
-    for (int i = 0; i < NR; ++i) acc0[i] = acc[i][0];
-    for (int j = 0; j < n; j += N) {
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+        for (int k = 0; k < KB; ++k) acc0[i][k] = acc[i][k];
+    for (int j = 0; j < n && !single; j += N) {
         T q[N], v[N][KB];
 #pragma unroll
         for (int u = 0; u < N; ++u) {
@@ -368,14 +382,17 @@ __device__ __forceinline__ void near_tile(const NearCol<T, KB> *t, int n, const 
             near_terms_kb<T, KID, TR, N, NR, KB>(p, q, v, acc, 0, n - j);
         }
     }
-    if constexpr (KB == 1 && KID <= 2 && !EXACT) {
+    if constexpr (KID <= 2) {
         if (__builtin_expect(odd, 0)) {
-            near_single<T, KID, TR, NR>(p, 0, n, [&](int u, T &qu, T &vu) {
+            near_single<T, KID, TR, NR, KB>(p, 0, n, [&](int u, T &qu, T (&vu)[KB]) {
                 qu = t[u].q;
-                vu = t[u].v[0];
+#pragma unroll
+                for (int k = 0; k < KB; ++k) vu[k] = t[u].v[k];
             }, acc0);
 #pragma unroll
-            for (int i = 0; i < NR; ++i) acc[i][0] = acc0[i];
+            for (int i = 0; i < NR; ++i)
+#pragma unroll
+                for (int k = 0; k < KB; ++k) acc[i][k] = acc0[i][k];
         }
     }
 }
@@ -388,7 +405,7 @@ template <class T, int KID, bool TR, bool EXACT, int KB>
 __device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const T (&p)[2],
                                           const T *pts_in, const T *x, int64_t incx, int64_t ldx,
                                           int nq, NearCol<T, KB> (*tile)[WAVE], int lane,
-                                          T (&acc)[2][KB]) {
+                                          bool single, T (&acc)[2][KB]) {
     if (nrun == 0) return;
     N1UnitRun R = sload_struct(runs);
     int e = 0, j = 0, b = 0;
@@ -416,13 +433,13 @@ __device__ __forceinline__ void near_unit(const N1UnitRun *runs, int nrun, const
         }
         if (e < nrun) load(R, j, c);
         if (mask == 3) {
-            near_tile<T, KID, TR, EXACT, 2, KB>(t, n, p, acc);
+            near_tile<T, KID, TR, EXACT, 2, KB>(t, n, p, single, acc);
         } else {
             const T p1[1] = {mask == 1 ? p[0] : p[1]};
             T a1[1][KB];
 #pragma unroll
             for (int k = 0; k < KB; ++k) a1[0][k] = mask == 1 ? acc[0][k] : acc[1][k];
-            near_tile<T, KID, TR, EXACT, 1, KB>(t, n, p1, a1);
+            near_tile<T, KID, TR, EXACT, 1, KB>(t, n, p1, single, a1);
 #pragma unroll
             for (int k = 0; k < KB; ++k) {
                 if (mask == 1) acc[0][k] = a1[0][k];
@@ -455,16 +472,18 @@ struct NearLds {
 };
 template <class T, int KID, bool TR, int SRC, int KB>
 __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pts_out,
-                                           const T *pts_in, const T *A, const MvArgsT<T> &a, int nq,
-                                           NearLds<T, KB> &s) {
+                                           const T *pts_in, const T *A, const int32_t *odd,
+                                           const MvArgsT<T> &a, int nq, NearLds<T, KB> &s) {
     const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
+    // an entry that the refinement does not give as it is stored: all by division
+    const bool single = SRC == N1_EXACT && odd && odd[1] != 0;
     if (o.nunit == 0) {
         const N1Chunk C = sload_struct(o.ch + blk);
         const int row = min(lane, C.np - 1);
         const T po = SRC == N1_READ ? T(0) : pts_out[C.p0 + row];
         T acc[KB];
         near_runs<T, KID, TR, SRC, KB>(o.run + C.run, C.nrun, po, pts_in, A, a.x, a.incx, a.ldx, nq,
-                                       row, wv, WPB, acc);
+                                       row, wv, WPB, single, acc);
 #pragma unroll
         for (int k = 0; k < KB; ++k) s.red[wv][k][lane] = acc[k];
         __syncthreads();
@@ -490,7 +509,7 @@ __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pt
         for (int k = 0; k < KB; ++k) acc[q][k] = T(0);
     }
     near_unit<T, KID, TR, SRC == N1_EXACT, KB>(o.urun + Un.run, Un.nrun, po, pts_in, a.x, a.incx,
-                                               a.ldx, nq, s.tile[wv], lane, acc);
+                                               a.ldx, nq, s.tile[wv], lane, single, acc);
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -721,6 +740,11 @@ __device__ __forceinline__ void n1_up_block_kb(const N1Side &s, const T *pts, co
     }
 }
 
+template <class T>
+__device__ __forceinline__ T nanT() {
+    return sizeof(T) == 8 ? (T)__builtin_nan("") : (T)__builtin_nanf("");
+}
+
 // Translation: one wavefront per cluster of the output side whose sources all
 // lie in subtrees (a wavefront takes several in turn, the matrix rows kept);
 // the clusters with a source above them ("heavy", first in the target list)
@@ -737,7 +761,7 @@ struct TrLds {
 template <class T, int RMAX, bool TRANS, int SRC, int KID, int KB>
 __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N1Side &o, int nq,
                                                    int blk, int nblk, const T *mats,
-                                                   const T *partial, const T *w, T *z,
+                                                   const T *partial, const T *w, T *z, int basis,
                                                    TrLds<T, RMAX, KB> &L_) {
     using Mt = N1Mat<T, RMAX>;
     constexpr bool FREE = SRC != N1_READ;
@@ -750,6 +774,9 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     const int r = p.r;
     const int mm = m < r ? m : 0;
     const T *oth = TRANS ? p.rnodes : p.cnodes;
+    // a stored product: the source clusters with a basis value that is not finite
+    // (a node meets a point), whose node values it makes NaN
+    const uint8_t *bad = basis && p.odd[0] ? (TRANS ? p.bad_rc : p.bad_cc) : nullptr;
     T At[HALF];
     load_rows(mats + Mt::AT, lane, At);
     T to = T(0), acc[KB];
@@ -767,13 +794,14 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
                     &to, ts + l0 + j, ws[0] + l0 + j, acc, 0, r - l0 - j);
             if constexpr (KID <= 2 && SRC == N1_FREE) {
                 if (__builtin_expect(odd, 0)) {
-                    acc[0] = acc0;
-                    near_single<T, KID, TRANS, 1>(&to, l0, min(l0 + HALF, r),
-                                                  [&](int u, T &qu, T &vu) {
-                                                      qu = ts[u];
-                                                      vu = ws[0][u];
-                                                  },
-                                                  acc);
+                    T sum[1][1] = {{acc0}};
+                    near_single<T, KID, TRANS, 1, 1>(&to, l0, min(l0 + HALF, r),
+                                                     [&](int u, T &qu, T (&vu)[1]) {
+                                                         qu = ts[u];
+                                                         vu[0] = ws[0][u];
+                                                     },
+                                                     sum);
+                    acc[0] = sum[0][0];
                 }
             }
         } else {
@@ -826,7 +854,8 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
                     const int e = i / (KB * RMAX), k = i / RMAX % KB, l = i % RMAX;
                     if (e < ne) {
                         const int64_t src = o.tr[e0 + e].src;
-                        const T wl = w[(src * nq + min(k, nq - 1)) * r + min(l, r - 1)];
+                        T wl = w[(src * nq + min(k, nq - 1)) * r + min(l, r - 1)];
+                        if (bad && bad[src]) wl = nanT<T>();
                         sw[wv][e][k][l] = l < r && k < nq ? wl : T(0);
                         if (FREE && k == 0) st[wv][e][l] = oth[src * r + min(l, r - 1)];
                     }
@@ -879,6 +908,7 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
             } else {
                 wl = w[((int64_t)R.src * nq + kc) * r + mm];
             }
+            if (bad && bad[R.src]) wl = nanT<T>();
             if (h == 0 && m < RMAX) sw[wv][0][k][m] = m < r && k < nq ? wl : T(0);
         }
         wave_sync();
@@ -934,8 +964,9 @@ constexpr int n1_waves(int src, int kid, int rmax, int kb) {
 
 template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID, RMAX, KB))))
-void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *A, const T *mats,
-             MvArgsT<T> a, int r, int nq, int nup, int nb0, int nb) {
+void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *A,
+             const int32_t *odd, const T *mats, MvArgsT<T> a, int r, int nq, int nup, int nb0,
+             int nb) {
     __shared__ union Lds {
         std::conditional_t<KB == 1, UpLds<T, RMAX>, UpLdsKb<T, RMAX>> up;
         NearLds<T, KB> near;
@@ -950,7 +981,7 @@ void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *
             n1_up_block_kb<T, RMAX>(in, in_pts, a.x, a.incx, a.ldx, mats, a.partial, a.w, r, nq, at,
                                     s.up);
     } else if (at < nb) {
-        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, A, a, nq, s.near);
+        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, A, odd, a, nq, s.near);
     }
 }
 
@@ -967,9 +998,10 @@ void k_n1_translate(DevPlanT<T> p, N1Side out, const T *in_pts, const T *out_pts
     if (chain_block(ntr, at)) {
         if (at < ntr)
             n1_translate_block<T, RMAX, TR, SRC, KID, KB>(p, out, nq, at, ntr, p.n1m, a.partial,
-                                                          a.w, a.z, s.tr);
+                                                          a.w, a.z, a.basis, s.tr);
     } else if (at < nb) {
-        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, p.A, a, nq, s.near);
+        near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, p.A, p.odd, a, nq,
+                                        s.near);
     }
 }
 
@@ -1065,21 +1097,31 @@ __device__ __forceinline__ T n1_series(const N1Chunk &C, const T (*cof)[RMAX], T
 // Several right-hand sides: a wavefront forms the coefficients of each.
 template <class T, int RMAX, int KB>
 __global__ __launch_bounds__(WG) void k_n1_down(N1Side o, const T *pts_out, const T *z,
-                                                const T *mats, MvArgsT<T> a, int r, int nq) {
+                                                const T *mats, const int32_t *odd,
+                                                const uint8_t *bad_pt, MvArgsT<T> a, int r,
+                                                int nq) {
     static_assert(KB <= WPB, "a wavefront per right-hand side");
     __shared__ __align__(16) T cof[KB][N1_NODES][RMAX];
     __shared__ __align__(16) T pz[KB][N1_PATH + 1][RMAX];
     const int lane = threadIdx.x % WAVE, wv = uniform((int)(threadIdx.x / WAVE));
     const N1Sub S = sload_struct(o.sub + blockIdx.x);
+    // a stored product: the points with a basis value that is not finite, whose
+    // rows it makes NaN
+    const uint8_t *bad = a.basis && odd[0] ? bad_pt : nullptr;
     if (wv < nq)
         n1_coefficients<T, RMAX>(o, S, mats, z + wv * r, (int64_t)nq * r, r, lane, cof[wv], pz[wv]);
     __syncthreads();
     for (int c = S.ch + wv; c < S.ch + S.nch; c += WPB) {
         const N1Chunk C = sload_struct(o.ch + c);
-        const T po = pts_out[C.p0 + min(lane, C.np - 1)];
+        const int64_t at = C.p0 + min(lane, C.np - 1);
+        const T po = pts_out[at];
+        const bool nan = bad && bad[at];
 #pragma unroll
         for (int k = 0; k < KB; ++k)
-            if (k < nq) n1_write(C, a, k, 1, lane, n1_series<T, RMAX>(C, cof[k], po));
+            if (k < nq) {
+                const T v = n1_series<T, RMAX>(C, cof[k], po);
+                n1_write(C, a, k, 1, lane, nan ? nanT<T>() : v);
+            }
     }
 }
 
@@ -1096,7 +1138,7 @@ void n1_chain(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s) {
     const T *in_pts = TR ? p.x : p.y, *out_pts = TR ? p.y : p.x;
     const int ntr = n1_ntranslate(out);
     k_n1_up<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(in.nsub, 0), WG, 0, s>>>(
-        in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, 1, in.nsub, 0, 0);
+        in, out, in_pts, out_pts, p.A, nullptr, p.n1m, a, p.r, 1, in.nsub, 0, 0);
     k_n1_translate<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(ntr, 0), WG, 0, s>>>(
         p, out, in_pts, out_pts, a, 1, ntr, 0, 0);
 }
@@ -1156,7 +1198,7 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, int nq, hipStr
     mark(0);
     if (nup + nb0 > 0)
         k_n1_up<T, RMAX, SRC, KID, TR, KB><<<n1_grid(nup, nb0), WG, 0, s>>>(
-            in, out, in_pts, out_pts, p.A, p.n1m, a, p.r, nq, nup, 0, nb0);
+            in, out, in_pts, out_pts, p.A, p.odd, p.n1m, a, p.r, nq, nup, 0, nb0);
     mark(1);
     mark(2);
     if (far) {
@@ -1172,7 +1214,8 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, int nq, hipStr
         near_part(s);
     }
     if (far)
-        k_n1_down<T, RMAX, KB><<<out.nsub, WG, 0, s>>>(out, out_pts, a.z, p.n1m, a, p.r, nq);
+        k_n1_down<T, RMAX, KB><<<out.nsub, WG, 0, s>>>(out, out_pts, a.z, p.n1m, p.odd,
+                                                       TR ? p.bad_y : p.bad_x, a, p.r, nq);
     mark(4);
     return hipGetLastError();
 }

@@ -784,7 +784,7 @@ struct PlanBufs {
     // (Staging); A, U, V and F are one allocation (factors) in plans from
     // points, and allocated on their own in plans from blocks
     void *arena = nullptr, *factors = nullptr;
-    unsigned long long *cnt = nullptr;  // the count of non-finite factors
+    unsigned long long *cnt = nullptr;  // the count of non-finite factors, then DevPlanT's odd words
     DevPlanT<T> dp{};
 
     void release() {
@@ -846,14 +846,10 @@ struct hm_plan {
     DTNode *d_xtn = nullptr, *d_ytn = nullptr;
     int32_t *d_xlev = nullptr, *d_ylev = nullptr, *d_chunk_leaf = nullptr;
     DTask *d_yleaf = nullptr;
-    // one right-hand side over the interval trees (nested1.h): both sides'
-    // tables; regen: a stored or hybrid plan's dense entries and F may be
-    // formed from the points and nodes instead of read; refit: the points were
-    // replaced after that was decided; uv_finite: U and V hold finite values
-    // alone, as far as uv_known says (the device's word after a refit);
-    // uv_replayed: a graph holds a refit, whose replays are not seen here
-    bool n1 = false, regen = false, refit = false, uv_finite = true, uv_known = true,
-         uv_replayed = false;
+    // up to N1_KB right-hand sides over the interval trees (nested1.h): both
+    // sides' tables; regen: a stored or hybrid plan's dense entries and F are
+    // formed from the points and nodes instead of read
+    bool n1 = false, regen = false;
     N1Host n1x, n1y;
     N1Side d_n1x{}, d_n1y{};
     void *d_tables = nullptr;  // the one allocation holding d_rcl .. d_yleaf (Staging)
@@ -872,7 +868,6 @@ struct hm_plan {
     std::vector<DSplit> xsplits, ysplits;
     DSplit *d_xsplits = nullptr, *d_ysplits = nullptr;
     int32_t *d_status = nullptr;  // the plan's own status word (in d_tables)
-    int32_t *d_uv_bad = nullptr;  // a value of U or V is not finite (in d_tables)
     int max_kb = HM_MAX_KB;  // right-hand sides per forward launch (1, 2, 4 or 8)
     int tuned_kb = HM_MAX_KB, tuned_mode = -1;  // hm_plan_tune's choice
     std::vector<hipEvent_t> prof_events;  // 5 per product
@@ -1265,6 +1260,10 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     int rc;
 #define HM_TRY_T(expr) do { rc = (expr); if (rc != HM_OK) return rc; } while (0)
     const int64_t nslots = std::max(P->rows.nslots, P->cols.nslots);
+    // DevPlanT's odd words (four) and, with U and V, a mark per point and cluster
+    const bool bases = !(flags & (HM_PLAN_MATRIX_FREE | HM_PLAN_HYBRID));
+    const int64_t nrc = (int64_t)P->rcl.size(), ncc = (int64_t)P->ccl.size();
+    const int64_t odd_bytes = 16 + (bases ? P->nx + P->ny + nrc + ncc : 0);
     const int64_t ncl = std::max(P->rcl.size(), P->ccl.size());
     {
         Staging st;
@@ -1288,7 +1287,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (std::is_same_v<T, double>) st.reserve(&b.xt, P->ny * HM_WS_RHS);
         if ((flags & HM_PLAN_MATRIX_FREE) || (std::is_same_v<T, float> && (flags & HM_PLAN_HYBRID)))
             st.reserve(&b.yt, std::max(P->nx, P->ny));
-        if (!(flags & HM_PLAN_MATRIX_FREE)) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS);
+        if (!(flags & HM_PLAN_MATRIX_FREE)) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS + (odd_bytes + 7) / 8);
         HM_TRY_T(st.commit(&b.arena));
     }
     if (b.my) {  // the moments of empty column nodes are read as zero
@@ -1316,9 +1315,16 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     dp.rmap = b.rmap; dp.cmap = b.cmap; dp.chebA = b.chebA;
     dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx; dp.n1m = b.n1m;
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
-    dp.uv_bad = P->d_uv_bad;
 
     if (stored) {
+        dp.odd = (int32_t *)(b.cnt + 4 * HM_COUNT_BLOCKS);
+        dp.nodd = (odd_bytes + 7) / 8 * 2;
+        if (bases) {
+            dp.bad_x = (uint8_t *)(dp.odd + 4);
+            dp.bad_y = dp.bad_x + P->nx;
+            dp.bad_rc = dp.bad_y + P->ny;
+            dp.bad_cc = dp.bad_rc + nrc;
+        }
         const bool user = P->kid == HM_USER;  // A and F come from hm_plan_set_leaf_data
         if (user) {
             T *arrs[] = {b.A, b.F};
@@ -1334,34 +1340,25 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         // count non-finite factors (coincident points give Inf, as in the reference)
         const T *arrs[] = {user ? nullptr : b.A, b.U, b.V, user ? nullptr : b.F};
         const int64_t lens[] = {nA, nU, nV, nF};
-        std::vector<unsigned long long> h(4 * HM_COUNT_BLOCKS, 0);
+        std::vector<unsigned long long> h(4 * HM_COUNT_BLOCKS + 2, 0);  // 2: the odd words
         e = hmx_launch_count_nonfinite(arrs, lens, b.cnt, s);
         if (e == hipSuccess)
             e = hipMemcpyAsync(h.data(), b.cnt, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
-        int64_t bad[4] = {0, 0, 0, 0}, big[4] = {0, 0, 0, 0};
+        int64_t bad[4] = {0, 0, 0, 0};
         for (int q = 0; q < 4; ++q)
-            for (int k = 0; k < HM_COUNT_BLOCKS; ++k) {
-                bad[q] += (int64_t)(h[q * HM_COUNT_BLOCKS + k] & 0xffffffffull);
-                big[q] += (int64_t)(h[q * HM_COUNT_BLOCKS + k] >> 32);
-            }
+            for (int k = 0; k < HM_COUNT_BLOCKS; ++k) bad[q] += (int64_t)h[q * HM_COUNT_BLOCKS + k];
         P->nonfinite = bad[0] + bad[1] + bad[2] + bad[3];
         P->nonfinite_basis = P->nonfinite;
-        P->uv_finite = bad[1] + bad[2] == 0;
         // A product may form the entries of 1/d^m itself: one reciprocal costs
         // a few vector instructions where an entry costs 8 bytes of HBM (stored
         // n = 2^20, rank 24: 402 M entries, 3.2 GB). The values are the stored
-        // ones while they and d^m stay in the normal range; the log kernel's
-        // and the caller's own entries are read.
-        double span = 0.0;
-        for (size_t t = 0; t + 1 < P->row_off.size(); ++t) {
-            const double xh = x[P->row_off[t]], xl = x[P->row_off[t + 1] - 1];
-            const double yh = y[P->col_off[t]], yl = y[P->col_off[t + 1] - 1];
-            span = std::max({span, std::fabs(xh - yl), std::fabs(yh - xl)});
-        }
+        // ones in the range that the compression checked; the log kernel's and
+        // the caller's own entries are read.
+        int32_t odd[4];
+        std::memcpy(odd, h.data() + 4 * HM_COUNT_BLOCKS, sizeof(odd));
         const bool power = P->kid == HM_CAUCHY || P->kid == HM_COULOMB || P->kid == HM_COULOMB3;
-        const double top = std::is_same_v<T, double> ? 1e100 : 1e12;
-        P->regen = power && span < top && bad[0] + big[0] + bad[3] + big[3] == 0;
+        P->regen = power && odd[1] == 0 && odd[2] == 0;
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression: %s", hipGetErrorString(e));
     }
     hipError_t e = hipStreamSynchronize(s);
@@ -1619,7 +1616,6 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
             add_n1(P->d_n1y, P->n1y);
         }
         st.reserve(&P->d_status, 1);
-        st.reserve(&P->d_uv_bad, 1);
         HM_TRY(st.commit(&P->d_tables));
         // the device holds these now
         const int64_t sx = P->n1x.slots, sy = P->n1y.slots;
@@ -1822,7 +1818,6 @@ static int from_blocks_t(int64_t nrows, int64_t ncols, int64_t nleaves, const in
     DevPlanT<T> &dp = b.dp;
     P->fill_structure(dp);
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
-    dp.uv_bad = P->d_uv_bad;
     (void)stream;
     *out = P;
     return HM_OK;
@@ -1920,15 +1915,6 @@ static int update_points_t(hm_plan_t P, const T *x, const T *y, int32_t *status,
     // the factors that depend on the points (dense blocks; U and V of stored
     // plans) are formed again; F depends on the intervals alone
     if (e == hipSuccess && !(P->flags & HM_PLAN_MATRIX_FREE)) e = hmx_launch_refit(b.dp, s);
-    P->refit = true;  // whether the new factors are finite is not known here
-    if (b.U || b.V) {
-        P->uv_known = false;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            P->uv_replayed = true;
-        }
-    }
     if (e != hipSuccess) return fail(HM_ERR_HIP, "update_points launch: %s", hipGetErrorString(e));
     return HM_OK;
 }
@@ -2154,26 +2140,6 @@ static bool split_near_field(hm_plan_t P, hipStream_t s) {
     return true;
 }
 
-// Whether a stored plan's U and V are finite. After new points the device
-// knows; its word is read back once, except on a stream that is being captured
-// (no: that product then reads U and V, as any plan with such values).
-static bool basis_finite(hm_plan_t P, hipStream_t s) {
-    if (P->uv_replayed) return false;
-    if (!P->uv_known) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        int32_t bad = 1;
-        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
-            hipMemcpyAsync(&bad, P->d_uv_bad, sizeof(bad), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        P->uv_finite = bad == 0;
-        P->uv_known = true;
-    }
-    return P->uv_finite;
-}
-
 template <class T>
 static MvArgsT<T> ws_args(hm_plan_t P) {
     MvArgsT<T> a{};
@@ -2260,9 +2226,11 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
     const bool use_side = mode != 0 && split_near_field(P, s);
     // over the interval trees, up to N1_KB right-hand sides per launch. A
     // stored plan's U and V equal the Chebyshev form's basis up to rounding
-    // unless a node meets a point (non-finite entries then keep the stored form)
-    const bool n1 = P->n1 && (mode != 0 || basis_finite(P, s));
-    const int src = mode == 2 ? N1_FREE : P->regen && !P->refit ? N1_EXACT : N1_READ;
+    // unless a node meets a point: there they are not finite, and the passes
+    // take it from the marks that the compression left (a.basis). The route
+    // does not hang on the points.
+    const bool n1 = P->n1;
+    const int src = mode == 2 ? N1_FREE : P->regen ? N1_EXACT : N1_READ;
     for (int64_t q = 0; q < k;) {
         // per level, forward products take up to HM_MAX_KB right-hand sides
         int kb = 1;
@@ -2277,6 +2245,7 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
         a.ldy = ldy;
         a.ldx = ldx;
         a.beta = beta;
+        a.basis = mode == 0;
         if (use_side) {
             a.side = P->side;
             a.fork = P->fork;
