@@ -103,6 +103,8 @@ struct DevPlanT {
     int n1;
     N1Side n1x, n1y;
     const T *n1m;
+    // a cluster's mapped nodes less the exact ones, in its frame (r per cluster)
+    const T *rdel, *cdel;
 };
 
 template <class T>

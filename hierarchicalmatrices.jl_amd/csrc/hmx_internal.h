@@ -155,10 +155,18 @@ struct N1Node {
     int32_t c[2];  // halves (local), -1: none or empty
 };
 
+// A tree node's frame: the center cx + cl and 1/halfwidth that follow from the
+// root's by halving alone, so that the fixed matrices of a half hold exactly.
+// (The interval ends are rounded at every halving, by up to 7e-12 of a half
+// width at depth 14 of [0, 1].)
+struct N1Frame {
+    double cx, cl, cy;
+};
+
 struct N1Leaf {
     int64_t first;
     int32_t len, loc;  // points, local node
-    double cx, cy;     // (center, 1/halfwidth)
+    N1Frame f;
 };
 
 // A node above a subtree: its cluster (or -1), the half of it that holds the
@@ -172,8 +180,7 @@ struct N1Chunk {
     int64_t p0;         // first point
     int32_t np, leaf;   // points; local node of the leaf holding them
     int32_t run, nrun;  // the near field's column runs
-    int32_t sub, pad;
-    double cx, cy;      // the leaf's (center, 1/halfwidth)
+    N1Frame f;          // the leaf's
 };
 
 // A cluster of the output side and its translation records

@@ -519,13 +519,22 @@ __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pt
 
 // -------------------------------------------------------------- far field
 // A plan's r x r matrices for lanes (m, h) = (lane % 32, lane / 32), padded
-// with zeros to RMAX, one row of 64 values per step (N1Mats): M_h[m][k] and
-// M_h[k][m] for k < RMAX, A[m][16h' + j] and A[h' + j][m] for j < RMAX / 2.
+// with zeros to RMAX, one row of 64 values per step: M_h[m][k] and M_h[k][m] for
+// k < RMAX, A[m][h' + j], A[h' + j][m], D[h' + j][m] and D[m][h' + j] for
+// j < RMAX / 2, h' = h RMAX / 2.
+//
+// F holds f at the mapped nodes as they are rounded, up to 1e-12 of a half width
+// off the exact ones (2^-53 of the point against a deep cluster). The products'
+// polynomials go through the rounded nodes: their offsets d enter w and z to
+// first order, w = w0 - D^T (d w0) for w0 = A mu, and c = A^T (z - d (D z)), D
+// the differentiation matrix of the exact nodes. Without it, stored products at
+// n = 2^20 were 6.4e-15 off, and 1.3e-15 with U and V, which hold the basis at
+// the rounded nodes.
 template <class T, int RMAX>
 struct N1Mat {
     static constexpr int HALF = RMAX / 2;
     static constexpr int MU = 0, MD = RMAX * WAVE, AU = 2 * RMAX * WAVE,
-                         AT = AU + HALF * WAVE, SIZE = AT + HALF * WAVE;
+                         DU = AU + HALF * WAVE, AT = DU + HALF * WAVE, DD = AT + HALF * WAVE;
 };
 template <class T, int N>
 __device__ __forceinline__ void load_rows(const T *m, int lane, T (&row)[N]) {
@@ -544,17 +553,29 @@ __device__ __forceinline__ T dot_row(const T (&row)[N], const T *v) {
     return s0 + s1;
 }
 
+// the same with the lane's column of rows of 64 in LDS
+template <class T, int HALF>
+__device__ __forceinline__ T dot_lds(const T *rows, int lane, const T *v) {
+    T s0 = T(0), s1 = T(0);
+#pragma unroll
+    for (int k = 0; k < HALF; k += 2) {
+        s0 = fmaT(rows[k * WAVE + lane], v[k], s0);
+        s1 = fmaT(rows[(k + 1) * WAVE + lane], v[k + 1], s1);
+    }
+    return s0 + s1;
+}
+
 // The moments sum_j T_m(xh_j) x_j of one leaf's points (one wavefront)
 template <class T, int RMAX>
 __device__ __forceinline__ void leaf_moments(const N1Leaf &L, const T *pts, const T *x, int64_t incx,
                                              int lane, T *out) {
-    const T cx = (T)L.cx, cy = (T)L.cy;
+    const T cx = (T)L.f.cx, cl = (T)L.f.cl, cy = (T)L.f.cy;
     T acc[RMAX];
 #pragma unroll
     for (int k = 0; k < RMAX; ++k) acc[k] = T(0);
     for (int i = lane; i < L.len; i += WAVE) {
         const T xv = x[(L.first + i) * incx];
-        const T xh = (pts[L.first + i] - cx) * cy;
+        const T xh = ((pts[L.first + i] - cx) - cl) * cy;
         const T x2 = xh + xh;
         T t0 = xv, t1 = xh * xv;  // T_m(xh) x by the recurrence
         acc[0] += t0;
@@ -589,6 +610,62 @@ __device__ __forceinline__ void node_moments(const N1Node &N, const T (&Mr)[RMAX
     if (h == 0 && m < RMAX) mom[n][m] = v;
 }
 
+// The w of NB clusters from their moments mom (LDS), d the lane's node offsets,
+// tmp: LDS of this wavefront's; dot_a and dot_d: the lane's row of A and of D^T
+// times a vector in LDS. Together, so that their chains run side by side.
+template <int RMAX, int NB, class T, class DotA, class DotD>
+__device__ __forceinline__ void node_values(DotA dot_a, DotD dot_d, const T *const (&mom)[NB],
+                                            const T (&d)[NB], int m, int h, T (*tmp)[RMAX],
+                                            T (&v)[NB]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        v[b] = dot_a(mom[b] + h * (RMAX / 2));
+        v[b] += __shfl_xor(v[b], 32);
+        if (h == 0 && m < RMAX) tmp[b][m] = d[b] * v[b];
+    }
+    wave_sync();
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        T e = dot_d(tmp[b] + h * (RMAX / 2));
+        e += __shfl_xor(e, 32);
+        v[b] -= e;
+    }
+    wave_sync();
+}
+// The w of a subtree's clusters, N1_WB at a time: of the local nodes next(-1),
+// next(that), ... below nnode, cl(n) their clusters; put(cluster, k, w_k)
+constexpr int N1_WB = 4;
+template <int RMAX, class T, class Next, class Cl, class Put>
+__device__ __forceinline__ void subtree_w(const T *mats, const T *del, const T (*mom)[RMAX],
+                                          T (*tmp)[RMAX], int r, int nnode, int lane, Next next,
+                                          Cl cl, Put put) {
+    using Mt = N1Mat<T, RMAX>;
+    const int m = lane & 31, h = lane >> 5;
+    T Ar[Mt::HALF], Dr[Mt::HALF];
+    load_rows(mats + Mt::AU, lane, Ar);
+    load_rows(mats + Mt::DU, lane, Dr);
+    for (int n = next(-1); n < nnode;) {
+        const int first = n;
+        int id[N1_WB];
+        T d[N1_WB], v[N1_WB];
+        const T *mo[N1_WB];
+#pragma unroll
+        for (int b = 0; b < N1_WB; ++b) {  // past the last: the first again, not written
+            id[b] = n < nnode ? cl(n) : -1;
+            mo[b] = mom[n < nnode ? n : first];
+            d[b] = m < r ? del[(int64_t)(n < nnode ? id[b] : id[0]) * r + m] : T(0);
+            if (n < nnode) n = next(n);
+        }
+        node_values<RMAX, N1_WB>([&](const T *u) { return dot_row(Ar, u); },
+                                 [&](const T *u) { return dot_row(Dr, u); }, mo, d, m, h, tmp, v);
+        if (h == 0 && m < r) {
+#pragma unroll
+            for (int b = 0; b < N1_WB; ++b)
+                if (id[b] >= 0) put(id[b], m, v[b]);
+        }
+    }
+}
+
 // Upward pass, one workgroup per subtree of the input side. The subtree's
 // records and the matrix rows are read before they are needed (the pass is a
 // chain of latencies: a few leaves, the depths, the path).
@@ -596,13 +673,14 @@ template <class T, int RMAX>
 struct UpLds {
     alignas(16) T mom[N1_NODES][RMAX];
     alignas(16) T pv[2][RMAX];
+    alignas(16) T dw[WPB][N1_WB][RMAX];
     N1Node nodes[N1_NODES];
     int32_t lev[N1_NODES + 1];
 };
 template <class T, int RMAX>
 __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const T *x, int64_t incx,
-                                            const T *mats, T *partial, T *w, int r, int blk,
-                                            UpLds<T, RMAX> &L_) {
+                                            const T *mats, const T *del, T *partial, T *w, int r,
+                                            int blk, UpLds<T, RMAX> &L_) {
     using Mt = N1Mat<T, RMAX>;
     auto &mom = L_.mom;
     auto &pv = L_.pv;
@@ -637,16 +715,16 @@ __device__ __forceinline__ void n1_up_block(const N1Side &s, const T *pts, const
     }
     // w of the clusters; the last wavefront walks the path meanwhile
     if (wv < WPB - 1 || S.npath == 0) {
-        T Ar[Mt::HALF];
-        load_rows(mats + Mt::AU, lane, Ar);
         const int step = S.npath == 0 ? WPB : WPB - 1;
-        for (int n = wv; n < S.nnode; n += step) {
-            const int cl = nodes[n].cl;
-            if (cl < 0) continue;
-            T v = dot_row(Ar, &mom[n][h * Mt::HALF]);
-            v += __shfl_xor(v, 32);
-            if (h == 0 && m < r) w[(int64_t)cl * r + m] = v;
-        }
+        subtree_w<RMAX>(
+            mats, del, mom, L_.dw[wv], r, S.nnode, lane,
+            [&](int n) {
+                n = n < 0 ? wv : n + step;
+                while (n < S.nnode && nodes[n].cl < 0) n += step;
+                return n;
+            },
+            [&](int n) { return nodes[n].cl; },
+            [&](int cl, int k, T v) { w[(int64_t)cl * r + k] = v; });
         return;
     }
     const T *cur = mom[0];
@@ -678,11 +756,13 @@ template <class T, int RMAX>
 struct UpLdsKb {
     alignas(16) T mom[N1_KB][N1_NODES][RMAX];
     alignas(16) T pv[N1_KB][2][RMAX];
+    alignas(16) T dw[N1_KB][N1_WB][RMAX];
 };
 template <class T, int RMAX>
 __device__ __forceinline__ void n1_up_block_kb(const N1Side &s, const T *pts, const T *x,
-                                               int64_t incx, int64_t ldx, const T *mats, T *partial,
-                                               T *w, int r, int nq, int blk, UpLdsKb<T, RMAX> &L_) {
+                                               int64_t incx, int64_t ldx, const T *mats,
+                                               const T *del, T *partial, T *w, int r, int nq,
+                                               int blk, UpLdsKb<T, RMAX> &L_) {
     using Mt = N1Mat<T, RMAX>;
     static_assert(N1_KB == WPB, "a wavefront per right-hand side");
     const int lane = threadIdx.x % WAVE, q = uniform((int)(threadIdx.x / WAVE));
@@ -729,15 +809,15 @@ __device__ __forceinline__ void n1_up_block_kb(const N1Side &s, const T *pts, co
         wave_sync();
         cur = nx;
     }
-    T Ar[Mt::HALF];
-    load_rows(mats + Mt::AU, lane, Ar);
-    for (int n = 0; n < S.nnode; ++n) {
-        const int cl = rl_i(nd.cl, n);
-        if (cl < 0) continue;
-        T v = dot_row(Ar, &mom[n][h * Mt::HALF]);
-        v += __shfl_xor(v, 32);
-        if (h == 0 && m < r) w[((int64_t)cl * nq + q) * r + m] = v;
-    }
+    subtree_w<RMAX>(
+        mats, del, mom, L_.dw[q], r, S.nnode, lane,
+        [&](int n) {
+            do ++n;
+            while (n < S.nnode && rl_i(nd.cl, n) < 0);
+            return n;
+        },
+        [&](int n) { return rl_i(nd.cl, n); },
+        [&](int cl, int k, T v) { w[((int64_t)cl * nq + q) * r + k] = v; });
 }
 
 template <class T>
@@ -757,6 +837,9 @@ template <class T, int RMAX, int KB>
 struct TrLds {
     alignas(16) T sw[WPB][4][KB][RMAX], st[WPB][4][RMAX];
     alignas(16) T zr[WPB][KB][RMAX];
+    // A^T and D of the output side (before them A and D^T, for sources above the
+    // subtrees): two matrices' rows in registers spilled
+    T mat[RMAX * WAVE];
 };
 template <class T, int RMAX, bool TRANS, int SRC, int KID, int KB>
 __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N1Side &o, int nq,
@@ -777,8 +860,12 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     // a stored product: the source clusters with a basis value that is not finite
     // (a node meets a point), whose node values it makes NaN
     const uint8_t *bad = basis && p.odd[0] ? (TRANS ? p.bad_rc : p.bad_cc) : nullptr;
-    T At[HALF];
-    load_rows(mats + Mt::AT, lane, At);
+    const T *din = TRANS ? p.rdel : p.cdel, *dout = TRANS ? p.cdel : p.rdel;
+    auto stage = [&](int from) {
+#pragma unroll
+        for (int e = 0; e < RMAX * WAVE; e += WG) L_.mat[e + threadIdx.x] = mats[from + e + threadIdx.x];
+        __syncthreads();
+    };
     T to = T(0), acc[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) acc[k] = T(0);
@@ -832,18 +919,41 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
             acc[k] = T(0);
         }
     };
-    auto finish = [&](int id, const T (*zs)[RMAX]) {  // c = A^T z
-#pragma unroll 1
-        for (int k = 0; k < nq; ++k) {
-            T c = dot_row(At, zs[k] + h * HALF);
-            c += __shfl_xor(c, 32);
-            if (h == 0 && m < r) z[((int64_t)id * nq + k) * r + m] = c;
+    // c = A^T (z - d (D z)), d the lane's node offset; z: zs
+    auto finish = [&](int id, T d, T (*zs)[RMAX]) {
+        T c[KB];
+        auto times = [&](const T *rows) {  // by one of the staged matrices, all z's together
+#pragma unroll
+            for (int k = 0; k < KB; ++k) c[k] = T(0);
+#pragma unroll
+            for (int j = 0; j < HALF; ++j) {
+                const T a = rows[j * WAVE + lane];
+#pragma unroll
+                for (int k = 0; k < KB; ++k) c[k] = fmaT(a, zs[k][h * HALF + j], c[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < KB; ++k) c[k] += __shfl_xor(c[k], 32);
+        };
+        times(L_.mat + HALF * WAVE);
+        wave_sync();
+        if (h == 0 && m < RMAX) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k) zs[k][m] -= d * c[k];
+        }
+        wave_sync();
+        times(L_.mat);
+        if (h == 0 && m < r) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+                if (k < nq) z[((int64_t)id * nq + k) * r + m] = c[k];
         }
     };
     if (blk >= o.nheavy) {
+        stage(Mt::AT);
         const int step = (nblk - o.nheavy) * WPB;
         for (int idx = o.nheavy + (blk - o.nheavy) * WPB + wv; idx < o.ncl; idx += step) {
             const N1Target C = sload_struct(o.target + idx);
+            const T d = m < r ? dout[(int64_t)C.id * r + m] : T(0);
             if constexpr (FREE) to = (TRANS ? p.cnodes : p.rnodes)[(int64_t)C.id * r + mm];
             for (int e0 = C.beg; e0 < C.end; e0 += NB) {
                 const int ne = min(NB, C.end - e0);
@@ -867,15 +977,14 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
             }
             put_z();
             wave_sync();
-            finish(C.id, zr[wv]);
+            finish(C.id, d, zr[wv]);
             wave_sync();
         }
         return;
     }
+    stage(Mt::AU);
     const N1Target C = sload_struct(o.target + blk);
     if constexpr (FREE) to = (TRANS ? p.cnodes : p.rnodes)[(int64_t)C.id * r + mm];
-    T Ar[HALF];
-    load_rows(mats + Mt::AU, lane, Ar);
     for (int e = C.beg + wv; e < C.end; e += WPB) {
         const DTrRec R = o.tr[e];
         if (FREE && h == 0 && m < RMAX) st[wv][0][m] = oth[(int64_t)R.src * r + (m < r ? m : r - 1)];
@@ -902,9 +1011,14 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
                 s += __shfl_xor(s, 32);
                 if (h == 0 && m < RMAX) sw[wv][0][k][m] = m < r ? s : T(0);
                 wave_sync();
-                wl = dot_row(Ar, &sw[wv][0][k][h * HALF]);  // w = A mu
-                wl += __shfl_xor(wl, 32);
-                wave_sync();
+                const T *mu[1] = {sw[wv][0][k]};
+                const T d[1] = {m < r ? din[(int64_t)R.src * r + m] : T(0)};
+                T v[1];
+                node_values<RMAX, 1>(
+                    [&](const T *u) { return dot_lds<T, HALF>(L_.mat, lane, u); },
+                    [&](const T *u) { return dot_lds<T, HALF>(L_.mat + HALF * WAVE, lane, u); }, mu,
+                    d, m, h, &zr[wv][k], v);
+                wl = v[0];
             } else {
                 wl = w[((int64_t)R.src * nq + kc) * r + mm];
             }
@@ -917,6 +1031,7 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
     }
     put_z();
     __syncthreads();
+    stage(Mt::AT);
     if (wv != 0) return;
     for (int k = 0; k < KB; ++k) {
         T s = T(0);
@@ -926,7 +1041,7 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
         if (h == 0 && m < RMAX) zr[0][k][m] = s;
         wave_sync();
     }
-    finish(C.id, zr[0]);
+    finish(C.id, m < r ? dout[(int64_t)C.id * r + m] : T(0), zr[0]);
 }
 
 // The two launches of the far-field chain before the downward pass. Each also
@@ -956,17 +1071,19 @@ __device__ __forceinline__ bool chain_block(int n, int &at) {
 // field is formed: left alone it gives four (upward) and three (translation);
 // six cost the near field's chains their registers (85 us).
 // Several right-hand sides: four, or three where the upward pass's LDS allows
-// no more.
-constexpr int n1_waves(int src, int kid, int rmax, int kb) {
+// no more. Float32 up to rank 16: eight, which its registers allow (left alone,
+// the scalar registers give seven: n = 500009, rank 10: 22.4 -> 24.4 us upward).
+constexpr int n1_waves(int size, int src, int kid, int rmax, int kb) {
+    if (size == 4 && rmax <= 16 && kid <= 2 && src != N1_READ && kb == 1) return 8;
     if (kid == 3 || (src == N1_READ && kb == 1)) return 1;
     return kb == 1 ? 5 : rmax > 24 || src == N1_READ ? 3 : 4;
 }
 
 template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID, RMAX, KB))))
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(sizeof(T), SRC, KID, RMAX, KB))))
 void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *A,
-             const int32_t *odd, const T *mats, MvArgsT<T> a, int r, int nq, int nup, int nb0,
-             int nb) {
+             const int32_t *odd, const T *mats, const T *del, MvArgsT<T> a, int r, int nq, int nup,
+             int nb0, int nb) {
     __shared__ union Lds {
         std::conditional_t<KB == 1, UpLds<T, RMAX>, UpLdsKb<T, RMAX>> up;
         NearLds<T, KB> near;
@@ -976,17 +1093,17 @@ void k_n1_up(N1Side in, N1Side out, const T *in_pts, const T *out_pts, const T *
     if (chain_block(nup, at)) {
         if (at >= nup) return;
         if constexpr (KB == 1)
-            n1_up_block<T, RMAX>(in, in_pts, a.x, a.incx, mats, a.partial, a.w, r, at, s.up);
+            n1_up_block<T, RMAX>(in, in_pts, a.x, a.incx, mats, del, a.partial, a.w, r, at, s.up);
         else
-            n1_up_block_kb<T, RMAX>(in, in_pts, a.x, a.incx, a.ldx, mats, a.partial, a.w, r, nq, at,
-                                    s.up);
+            n1_up_block_kb<T, RMAX>(in, in_pts, a.x, a.incx, a.ldx, mats, del, a.partial, a.w, r, nq,
+                                    at, s.up);
     } else if (at < nb) {
         near_block<T, KID, TR, SRC, KB>(out, at + nb0, out_pts, in_pts, A, odd, a, nq, s.near);
     }
 }
 
 template <class T, int RMAX, int SRC, int KID, bool TR, int KB>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(SRC, KID, RMAX, KB))))
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(n1_waves(sizeof(T), SRC, KID, RMAX, KB))))
 void k_n1_translate(DevPlanT<T> p, N1Side out, const T *in_pts, const T *out_pts, MvArgsT<T> a,
                     int nq, int ntr, int nb0, int nb) {
     __shared__ union Lds {
@@ -1080,7 +1197,7 @@ __device__ __forceinline__ void n1_coefficients(const N1Side &s, const N1Sub &S,
 // past r)
 template <class T, int RMAX>
 __device__ __forceinline__ T n1_series(const N1Chunk &C, const T (*cof)[RMAX], T p) {
-    const T xh = (p - (T)C.cx) * (T)C.cy, x2 = xh + xh;
+    const T xh = ((p - (T)C.f.cx) - (T)C.f.cl) * (T)C.f.cy, x2 = xh + xh;
     const T *ck = cof[C.leaf];
     T b1 = T(0), b2 = T(0);
 #pragma unroll
@@ -1138,7 +1255,7 @@ void n1_chain(const DevPlanT<T> &p, const MvArgsT<T> &a, hipStream_t s) {
     const T *in_pts = TR ? p.x : p.y, *out_pts = TR ? p.y : p.x;
     const int ntr = n1_ntranslate(out);
     k_n1_up<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(in.nsub, 0), WG, 0, s>>>(
-        in, out, in_pts, out_pts, p.A, nullptr, p.n1m, a, p.r, 1, in.nsub, 0, 0);
+        in, out, in_pts, out_pts, p.A, nullptr, p.n1m, TR ? p.rdel : p.cdel, a, p.r, 1, in.nsub, 0, 0);
     k_n1_translate<T, RMAX, N1_FREE, KID, TR, 1><<<n1_grid(ntr, 0), WG, 0, s>>>(
         p, out, in_pts, out_pts, a, 1, ntr, 0, 0);
 }
@@ -1198,7 +1315,7 @@ hipError_t matvec_n1_t(const DevPlanT<T> &p, const MvArgsT<T> &a, int nq, hipStr
     mark(0);
     if (nup + nb0 > 0)
         k_n1_up<T, RMAX, SRC, KID, TR, KB><<<n1_grid(nup, nb0), WG, 0, s>>>(
-            in, out, in_pts, out_pts, p.A, p.odd, p.n1m, a, p.r, nq, nup, 0, nb0);
+            in, out, in_pts, out_pts, p.A, p.odd, p.n1m, TR ? p.rdel : p.cdel, a, p.r, nq, nup, 0, nb0);
     mark(1);
     mark(2);
     if (far) {

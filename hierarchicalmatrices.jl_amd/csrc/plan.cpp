@@ -457,13 +457,14 @@ struct N1Host {
     std::vector<int64_t> sbase;
     std::vector<int32_t> scount;
     int64_t slots = 0;
+    std::vector<N1Frame> frame;  // per cluster
 
     // A subtree has at most N1_NODES nodes and GC chunks (or is one leaf).
     // GC: 4 while a downward workgroup takes one chunk (its wavefronts share
     // the path and the subtree with three others at most), else so that about
     // 1024 to 2048 workgroups share the paths' work among their chunks.
-    bool cut(const std::vector<DTNode> &t, const Side &S, const std::vector<DDense> &dense,
-             bool rows, size_t ncl) {
+    bool cut(const std::vector<DTNode> &t, const std::vector<N1Frame> &fr, const Side &S,
+             const std::vector<DDense> &dense, bool rows, size_t ncl) {
         const std::vector<DChunk> &dc = S.ch;
         const int64_t nch = (int64_t)dc.size();
         int32_t GC = 4;
@@ -501,6 +502,9 @@ struct N1Host {
                 if (!one) return false;
             }
         }
+        frame.resize(ncl);
+        for (size_t k = 0; k < nt; ++k)
+            if (t[k].cl >= 0) frame[t[k].cl] = fr[k];
         sbase.assign(ncl, 0);
         scount.assign(ncl, 0);
         ch.resize(dc.size());
@@ -544,15 +548,13 @@ struct N1Host {
                         const DTNode &q = t[queue[at]];
                         N1Node g{q.cl, {-1, -1}};
                         if (q.child[0] < 0) {
-                            leaf.push_back({q.first, q.len, (int32_t)at, q.cx, q.cy});
+                            leaf.push_back({q.first, q.len, (int32_t)at, fr[queue[at]]});
                             for (int32_t c = cb[queue[at]]; c < cb[queue[at]] + cn[queue[at]]; ++c) {
                                 N1Chunk &w = ch[c];
                                 w.p0 = dc[c].p0;
                                 w.np = dc[c].np;
                                 w.leaf = (int32_t)at;
-                                w.sub = (int32_t)sub.size();
-                                w.cx = q.cx;
-                                w.cy = q.cy;
+                                w.f = fr[queue[at]];
                                 ++covered;
                             }
                         } else {
@@ -779,7 +781,8 @@ struct PlanBufs {
     // nested far field of the MFMA passes (Float64 plans): the re-expansion
     // matrices, moments per column node, coefficients per row node
     T *nestM = nullptr, *my = nullptr, *mx = nullptr;
-    T *n1m = nullptr;  // padded matrices of the single-right-hand-side tree passes
+    // padded matrices of the single-right-hand-side tree passes, node offsets
+    T *n1m = nullptr, *rdel = nullptr, *cdel = nullptr;
     // x .. chebA and the workspace partial .. xt live in this one allocation
     // (Staging); A, U, V and F are one allocation (factors) in plans from
     // points, and allocated on their own in plans from blocks
@@ -962,6 +965,40 @@ struct hm_plan {
         return true;
     }
 
+    // The frames of one side's tree nodes: the root's center and halfwidth to
+    // twice the precision (near an end of the interval at zero a node may be
+    // 2^-50 of it), the others by halving. Float32: the center as two floats.
+    template <class TN>
+    std::vector<N1Frame> frames(const std::vector<TN> &t) const {
+        struct Two {
+            double hi, lo;
+        };
+        auto sum = [](double a, double b) {  // a + b = hi + lo exactly
+            const double s = a + b, v = s - a;
+            return Two{s, (a - (s - v)) + (b - v)};
+        };
+        std::vector<N1Frame> o(t.size());
+        std::vector<Two> c(t.size()), h(t.size());
+        for (size_t k = 0; k < t.size(); ++k) {  // every node comes after its parent
+            if (t[k].parent < 0) {
+                c[k] = sum(0.5 * t[k].lo, 0.5 * t[k].hi);
+                h[k] = sum(0.5 * t[k].hi, -0.5 * t[k].lo);
+            } else {
+                const Two pc = c[t[k].parent], ph = h[t[k].parent];
+                const double q = t[k].half ? 0.5 : -0.5;
+                const Two s = sum(pc.hi, q * ph.hi);
+                c[k] = sum(s.hi, s.lo + (pc.lo + q * ph.lo));
+                h[k] = {0.5 * ph.hi, 0.5 * ph.lo};
+            }
+            o[k] = {c[k].hi, c[k].lo, 1.0 / h[k].hi};
+            if (f32) {
+                o[k].cx = (double)(float)c[k].hi;
+                o[k].cl = (c[k].hi - o[k].cx) + c[k].lo;
+            }
+        }
+        return o;
+    }
+
     // Tables of the single-right-hand-side tree passes; n1 stays false (the
     // per-level passes are used) where the trees do not nest, a chunk lies in
     // several leaves, or the rank exceeds 32 (a wavefront's two halves hold a
@@ -974,8 +1011,8 @@ struct hm_plan {
         std::vector<DTNode> xs, ys;
         if (!nest && (!tree_nodes(xt, xs) || !tree_nodes(yt, ys))) return;
         bool okx = false, oky = false;
-        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, rows, dense, true, rcl.size()); },
-                   [&] { oky = n1y.cut(nest ? ytn : ys, cols, dense, false, ccl.size()); });
+        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, frames(xt), rows, dense, true, rcl.size()); },
+                   [&] { oky = n1y.cut(nest ? ytn : ys, frames(yt), cols, dense, false, ccl.size()); });
         if (!okx || !oky) return;
         n1x.targets(rcl, by_rc, far, true, n1y);
         n1y.targets(ccl, by_cc, far, false, n1x);
@@ -1185,15 +1222,28 @@ std::vector<T> nest_matrices(int r) {
 
 // The matrices of the single-right-hand-side tree passes, laid out for lanes
 // (m, h) = (lane % 32, lane / 32) and padded with zeros to the rank bucket
-// (N1Mat): M_h[m][k], M_h[k][m], A[m][h R/2 + j], A[h R/2 + j][m].
+// (N1Mat): M_h[m][k], M_h[k][m], A[m][h R/2 + j], A[h R/2 + j][m], and of the
+// nodes' differentiation matrix D (values at the nodes -> the polynomial's
+// derivatives there; the barycentric formula) D[h R/2 + j][m], D[m][h R/2 + j].
 extern "C++" {
 template <class T>
 std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> &A) {
     const int R = r <= 8 ? 8 : r <= 16 ? 16 : (r <= 24 && std::is_same_v<T, double>) ? 24 : 32;
     const int HALF = R / 2;
-    std::vector<T> out((size_t)(2 * R + 2 * HALF) * 64, T(0));
+    std::vector<T> out((size_t)(2 * R + 4 * HALF) * 64, T(0));
     T *MU = out.data(), *MD = MU + (size_t)R * 64, *AU = MD + (size_t)R * 64,
-      *AT = AU + (size_t)HALF * 64;
+      *DU = AU + (size_t)HALF * 64, *AT = DU + (size_t)HALF * 64, *DD = AT + (size_t)HALF * 64;
+    std::vector<double> D((size_t)r * r, 0.0);
+    for (int k = 0; k < r; ++k)
+        for (int j = 0; j < r; ++j) {
+            if (j == k) continue;
+            // t_k - t_j = -2 sin((a + b)/2) sin((a - b)/2), weights (-1)^k sin
+            const double a = (2 * k + 1) * M_PI / (2 * r), c = (2 * j + 1) * M_PI / (2 * r);
+            const double q = std::sin(c) / std::sin(a) /
+                             (-2.0 * std::sin(0.5 * (a + c)) * std::sin(0.5 * (a - c)));
+            D[(size_t)k * r + j] = ((k + j) & 1) ? -q : q;
+            D[(size_t)k * r + k] -= D[(size_t)k * r + j];
+        }
     for (int lane = 0; lane < 64; ++lane) {
         const int m = lane % 32, h = lane / 32;
         if (m >= r) continue;
@@ -1204,6 +1254,8 @@ std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> 
         for (int j = 0; j < HALF && h * HALF + j < r; ++j) {
             AU[j * 64 + lane] = A[(size_t)m * r + h * HALF + j];
             AT[j * 64 + lane] = A[(size_t)(h * HALF + j) * r + m];
+            DU[j * 64 + lane] = (T)D[(size_t)(h * HALF + j) * r + m];
+            DD[j * 64 + lane] = (T)D[(size_t)m * r + h * HALF + j];
         }
     }
     return out;
@@ -1244,6 +1296,23 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     std::vector<V2> rmap, cmap;
     nodes(hr, rn, rmap);
     nodes(hc, cn, cmap);
+    // the mapped nodes are rounded: by how much, in the frames of the trees
+    // (both differences below are exact or nearly so)
+    std::vector<T> rdel, cdel;
+    auto offsets = [&](const std::vector<N1Frame> &f, const std::vector<T> &t, std::vector<T> &o) {
+        std::vector<double> c(r);
+        for (int q = 0; q < r; ++q) c[q] = std::cos((2 * q + 1) * M_PI / (2 * r));
+        o.resize(t.size());
+        for (size_t k = 0; k < f.size(); ++k)
+            for (int q = 0; q < r; ++q)
+                o[k * r + q] = (T)(((double)t[k * r + q] - f[k].cx - f[k].cl) * f[k].cy - c[q]);
+    };
+    if (P->n1) {
+        offsets(P->n1x.frame, rn, rdel);
+        offsets(P->n1y.frame, cn, cdel);
+        P->n1x.frame.clear();
+        P->n1y.frame.clear();
+    }
     // A[k][m] = (m ? 2 : 1) T_m(xhat_k) / r, T_m(cos t) = cos(m t), t_k = (2k-1) pi / (2r)
     std::vector<T> chebA((size_t)r * r);
     {
@@ -1280,7 +1349,11 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
             st.reserve(&b.my, (int64_t)P->ytn.size() * r * HM_WS_RHS);
             st.reserve(&b.mx, (int64_t)P->xtn.size() * r * HM_WS_RHS);
         }
-        if (P->n1) st.add(&b.n1m, n1m);
+        if (P->n1) {
+            st.add(&b.n1m, n1m);
+            st.add(&b.rdel, rdel);
+            st.add(&b.cdel, cdel);
+        }
         st.reserve(&b.partial, std::max(nslots * HM_WS_RHS, std::max(P->n1x.slots, P->n1y.slots) * N1_KB) * r);
         st.reserve(&b.w, ncl * r * HM_WS_RHS);
         st.reserve(&b.z, ncl * r * HM_WS_RHS);
@@ -1313,7 +1386,8 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     dp.x = b.x; dp.y = b.y; dp.lam = b.lam;
     dp.rnodes = b.rnodes; dp.cnodes = b.cnodes;
     dp.rmap = b.rmap; dp.cmap = b.cmap; dp.chebA = b.chebA;
-    dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx; dp.n1m = b.n1m;
+    dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx;
+    dp.n1m = b.n1m; dp.rdel = b.rdel; dp.cdel = b.cdel;
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
 
     if (stored) {
@@ -1619,10 +1693,13 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
         HM_TRY(st.commit(&P->d_tables));
         // the device holds these now
         const int64_t sx = P->n1x.slots, sy = P->n1y.slots;
+        std::vector<N1Frame> fx = std::move(P->n1x.frame), fy = std::move(P->n1y.frame);
         P->n1x = N1Host{};
         P->n1y = N1Host{};
         P->n1x.slots = sx;
         P->n1y.slots = sy;
+        P->n1x.frame = std::move(fx);
+        P->n1y.frame = std::move(fy);
     }
     P->far_by_rc_h = std::move(by_rc);
     if (f32) HM_TRY(setup_typed<float>(P, x, y, B.rcl, B.ccl, flags, nA, nU, nV, nF, (hipStream_t)stream));
