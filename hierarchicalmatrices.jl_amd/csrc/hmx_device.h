@@ -104,7 +104,7 @@ struct DevPlanT {
     N1Side n1x, n1y;
     const T *n1m;
     // a cluster's mapped nodes less the exact ones, in its frame (r per cluster)
-    const T *rdel, *cdel;
+    T *rdel, *cdel;
 };
 
 template <class T>
@@ -136,6 +136,10 @@ using DevPlan = DevPlanT<double>;
 using DevPlanF = DevPlanT<float>;
 using MvArgs = MvArgsT<double>;
 using MvArgsF = MvArgsT<float>;
+
+// rdel and cdel of a plan with n1, from the clusters' frames
+hipError_t hmx_launch_node_offsets(const DevPlan &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
+hipError_t hmx_launch_node_offsets(const DevPlanF &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
 
 // compression: dense blocks, U, V, F (bit-exact operation order)
 hipError_t hmx_launch_compress(const DevPlan &p, hipStream_t s);

@@ -4,10 +4,17 @@
 #include "hmx.h"
 #include "kernels_impl.h"
 
+hipError_t hmx_launch_node_offsets(const DevPlan &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
+    return hmxk::node_offsets(p, rf, cf, s);
+}
+hipError_t hmx_launch_node_offsets(const DevPlanF &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
+    return hmxk::node_offsets(p, rf, cf, s);
+}
+
 hipError_t hmx_launch_compress(const DevPlan &p, hipStream_t s) {
     // HM_USER plans take A and F from the caller (hm_plan_set_leaf_data)
     const bool gen = p.kid != HM_USER;
-    hmxk::clear_odd(p, s);
+    if (p.bad_x) hmxk::clear_odd(p, s);  // without marks the words come cleared
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<double><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<double><<<p.nfar, hmxk::WG, 0, s>>>(p);
     if (p.U && p.V && p.nrc + p.ncc > 0)
@@ -83,7 +90,7 @@ hipError_t hmx_launch_matvec_m(const DevPlan &p, const MvArgs &a, int mode, int 
 
 hipError_t hmx_launch_compress(const DevPlanF &p, hipStream_t s) {
     const bool gen = p.kid != HM_USER;
-    hmxk::clear_odd(p, s);
+    if (p.bad_x) hmxk::clear_odd(p, s);  // without marks the words come cleared
     if (gen && p.ndense > 0 && p.A) hmxk::k_gen_dense<float><<<p.ndense, hmxk::WG, 0, s>>>(p);
     if (gen && p.nfar > 0 && p.F) hmxk::k_gen_F<float><<<p.nfar, hmxk::WG, 0, s>>>(p);
     if (p.U && p.V && p.nrc + p.ncc > 0)

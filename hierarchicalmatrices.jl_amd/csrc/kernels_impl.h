@@ -42,6 +42,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace hmxk {
@@ -318,6 +319,30 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
     }
 }
 
+// DevPlanT's rdel and cdel: how far the mapped nodes are off the exact ones in
+// their cluster's frame, by rounding (the differences from the center are exact
+// or nearly so)
+template <class T>
+__global__ __launch_bounds__(WG) void k_node_offsets(DevPlanT<T> p, const N1Frame *rf,
+                                                     const N1Frame *cf) {
+    const int64_t nr = (int64_t)p.nrc * p.r, n = nr + (int64_t)p.ncc * p.r;
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
+        const bool row = i < nr;
+        const int64_t at = row ? i : i - nr, c = at / p.r;
+        const N1Frame f = row ? rf[c] : cf[c];
+        const double t = (double)(row ? p.rnodes : p.cnodes)[at];
+        (row ? p.rdel : p.cdel)[at] =
+            (T)(((t - f.cx) - f.cl) * f.cy - cospi((2 * (int)(at - c * p.r) + 1) / (2.0 * p.r)));
+    }
+}
+template <class T>
+hipError_t node_offsets(const DevPlanT<T> &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
+    const int64_t n = ((int64_t)p.nrc + p.ncc) * p.r;
+    if (n > 0)
+        k_node_offsets<T><<<(int)std::min<int64_t>((n + WG - 1) / WG, 1024), WG, 0, s>>>(p, rf, cf);
+    return hipGetLastError();
+}
+
 // DevPlanT's odd words and marks, before the factors are formed
 __global__ __launch_bounds__(WG) void k_clear_words(int32_t *w, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG)
@@ -326,7 +351,7 @@ __global__ __launch_bounds__(WG) void k_clear_words(int32_t *w, int64_t n) {
 template <class T>
 void clear_odd(const DevPlanT<T> &p, hipStream_t s) {
     if (p.nodd > 0)
-        k_clear_words<<<(int)(p.nodd < 256 * WG ? (p.nodd + WG - 1) / WG : 256), WG, 0, s>>>(p.odd, p.nodd);
+        k_clear_words<<<(int)std::min<int64_t>((p.nodd + WG - 1) / WG, 256), WG, 0, s>>>(p.odd, p.nodd);
 }
 
 // Non-finite values of up to four arrays, one count per workgroup (gridDim.x of

@@ -42,8 +42,6 @@
 #pragma once
 #include "kernels_impl.h"
 
-#include <algorithm>
-
 namespace hmxk {
 namespace {
 

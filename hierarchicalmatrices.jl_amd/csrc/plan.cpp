@@ -723,6 +723,11 @@ struct Staging {
         if (!src.empty()) items.push_back({(void **)dst, src.data(), sizeof(T) * src.size()});
     }
     template <class T>
+    void add(T **dst, const T *src, int64_t n) {
+        *dst = nullptr;
+        if (n > 0) items.push_back({(void **)dst, src, sizeof(T) * (size_t)n});
+    }
+    template <class T>
     void reserve(T **dst, int64_t n) {
         *dst = nullptr;
         if (n > 0) items.push_back({(void **)dst, nullptr, sizeof(T) * (size_t)n});
@@ -738,14 +743,14 @@ struct Staging {
         for (const Item &I : items)
             if (!I.src) total += up(I.bytes);
         if (!total) return HM_OK;
-        std::vector<unsigned char> host(copied);
+        std::unique_ptr<unsigned char[]> host(new unsigned char[copied]);  // (not cleared first)
         std::vector<size_t> off(items.size());
         size_t c = 0, w = copied;
         for (size_t q = 0; q < items.size(); ++q) {
             const Item &I = items[q];
             if (I.src) {
                 off[q] = c;
-                std::memcpy(host.data() + c, I.src, I.bytes);
+                std::memcpy(host.get() + c, I.src, I.bytes);
                 c += up(I.bytes);
             } else {
                 off[q] = w;
@@ -760,7 +765,7 @@ struct Staging {
                         hipGetErrorString(e));
         }
         *arena = d;
-        if (copied) HM_HIP(hipMemcpy(d, host.data(), copied, hipMemcpyHostToDevice));
+        if (copied) HM_HIP(hipMemcpy(d, host.get(), copied, hipMemcpyHostToDevice));
         for (size_t q = 0; q < items.size(); ++q) *items[q].dst = (unsigned char *)d + off[q];
         return HM_OK;
     }
@@ -783,6 +788,7 @@ struct PlanBufs {
     T *nestM = nullptr, *my = nullptr, *mx = nullptr;
     // padded matrices of the single-right-hand-side tree passes, node offsets
     T *n1m = nullptr, *rdel = nullptr, *cdel = nullptr;
+    N1Frame *rframe = nullptr, *cframe = nullptr;  // per cluster
     // x .. chebA and the workspace partial .. xt live in this one allocation
     // (Staging); A, U, V and F are one allocation (factors) in plans from
     // points, and allocated on their own in plans from blocks
@@ -1233,14 +1239,15 @@ std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> 
     std::vector<T> out((size_t)(2 * R + 4 * HALF) * 64, T(0));
     T *MU = out.data(), *MD = MU + (size_t)R * 64, *AU = MD + (size_t)R * 64,
       *DU = AU + (size_t)HALF * 64, *AT = DU + (size_t)HALF * 64, *DD = AT + (size_t)HALF * 64;
-    std::vector<double> D((size_t)r * r, 0.0);
+    std::vector<double> D((size_t)r * r, 0.0), sn(2 * r);  // sn[i] = sin(i pi / (2r))
+    for (int i = 0; i < 2 * r; ++i) sn[i] = std::sin(i * M_PI / (2 * r));
     for (int k = 0; k < r; ++k)
         for (int j = 0; j < r; ++j) {
             if (j == k) continue;
-            // t_k - t_j = -2 sin((a + b)/2) sin((a - b)/2), weights (-1)^k sin
-            const double a = (2 * k + 1) * M_PI / (2 * r), c = (2 * j + 1) * M_PI / (2 * r);
-            const double q = std::sin(c) / std::sin(a) /
-                             (-2.0 * std::sin(0.5 * (a + c)) * std::sin(0.5 * (a - c)));
+            // t_k = cos((2k + 1) pi / (2r)), weights (-1)^k sin; t_k - t_j =
+            // -2 sin((k + j + 1) pi / (2r)) sin((k - j) pi / (2r))
+            const double q = sn[2 * j + 1] / sn[2 * k + 1] /
+                             (-2.0 * sn[k + j + 1] * (k > j ? sn[k - j] : -sn[j - k]));
             D[(size_t)k * r + j] = ((k + j) & 1) ? -q : q;
             D[(size_t)k * r + k] -= D[(size_t)k * r + j];
         }
@@ -1296,23 +1303,6 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     std::vector<V2> rmap, cmap;
     nodes(hr, rn, rmap);
     nodes(hc, cn, cmap);
-    // the mapped nodes are rounded: by how much, in the frames of the trees
-    // (both differences below are exact or nearly so)
-    std::vector<T> rdel, cdel;
-    auto offsets = [&](const std::vector<N1Frame> &f, const std::vector<T> &t, std::vector<T> &o) {
-        std::vector<double> c(r);
-        for (int q = 0; q < r; ++q) c[q] = std::cos((2 * q + 1) * M_PI / (2 * r));
-        o.resize(t.size());
-        for (size_t k = 0; k < f.size(); ++k)
-            for (int q = 0; q < r; ++q)
-                o[k * r + q] = (T)(((double)t[k * r + q] - f[k].cx - f[k].cl) * f[k].cy - c[q]);
-    };
-    if (P->n1) {
-        offsets(P->n1x.frame, rn, rdel);
-        offsets(P->n1y.frame, cn, cdel);
-        P->n1x.frame.clear();
-        P->n1y.frame.clear();
-    }
     // A[k][m] = (m ? 2 : 1) T_m(xhat_k) / r, T_m(cos t) = cos(m t), t_k = (2k-1) pi / (2r)
     std::vector<T> chebA((size_t)r * r);
     {
@@ -1322,7 +1312,17 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
                 chebA[(size_t)(k - 1) * r + m] =
                     (T)((m ? 2.0L : 1.0L) * cosl((long double)m * (2 * k - 1) * PI_L / (2.0L * r)) / r);
     }
-    const std::vector<T> xv(x, x + P->nx), yv(y, y + P->ny);
+    std::vector<T> xv, yv;  // Float32: the points as floats
+    const T *xp, *yp;
+    if constexpr (std::is_same_v<T, double>) {
+        xp = x;
+        yp = y;
+    } else {
+        xv.assign(x, x + P->nx);
+        yv.assign(y, y + P->ny);
+        xp = xv.data();
+        yp = yv.data();
+    }
     std::vector<T> nestM, n1m;
     if ((std::is_same_v<T, double> && P->nest) || P->n1) nestM = nest_matrices<T>(r);
     if (P->n1) n1m = n1_matrices<T>(r, nestM, chebA);
@@ -1332,12 +1332,13 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     // DevPlanT's odd words (four) and, with U and V, a mark per point and cluster
     const bool bases = !(flags & (HM_PLAN_MATRIX_FREE | HM_PLAN_HYBRID));
     const int64_t nrc = (int64_t)P->rcl.size(), ncc = (int64_t)P->ccl.size();
+    const std::vector<unsigned long long> cnt0(4 * HM_COUNT_BLOCKS + 2, 0);
     const int64_t odd_bytes = 16 + (bases ? P->nx + P->ny + nrc + ncc : 0);
     const int64_t ncl = std::max(P->rcl.size(), P->ccl.size());
     {
         Staging st;
-        st.add(&b.x, xv);
-        st.add(&b.y, yv);
+        st.add(&b.x, xp, P->nx);
+        st.add(&b.y, yp, P->ny);
         st.add(&b.lam, lam);
         st.add(&b.rnodes, rn);
         st.add(&b.cnodes, cn);
@@ -1351,8 +1352,10 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         }
         if (P->n1) {
             st.add(&b.n1m, n1m);
-            st.add(&b.rdel, rdel);
-            st.add(&b.cdel, cdel);
+            st.add(&b.rframe, P->n1x.frame);
+            st.add(&b.cframe, P->n1y.frame);
+            st.reserve(&b.rdel, (int64_t)rn.size());
+            st.reserve(&b.cdel, (int64_t)cn.size());
         }
         st.reserve(&b.partial, std::max(nslots * HM_WS_RHS, std::max(P->n1x.slots, P->n1y.slots) * N1_KB) * r);
         st.reserve(&b.w, ncl * r * HM_WS_RHS);
@@ -1360,8 +1363,12 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (std::is_same_v<T, double>) st.reserve(&b.xt, P->ny * HM_WS_RHS);
         if ((flags & HM_PLAN_MATRIX_FREE) || (std::is_same_v<T, float> && (flags & HM_PLAN_HYBRID)))
             st.reserve(&b.yt, std::max(P->nx, P->ny));
-        if (!(flags & HM_PLAN_MATRIX_FREE)) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS + (odd_bytes + 7) / 8);
+        // with the marks the words are cleared on the device, else they come cleared
+        if (bases) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS + (odd_bytes + 7) / 8);
+        else if (!(flags & HM_PLAN_MATRIX_FREE)) st.add(&b.cnt, cnt0);
         HM_TRY_T(st.commit(&b.arena));
+        P->n1x.frame.clear();
+        P->n1y.frame.clear();
     }
     if (b.my) {  // the moments of empty column nodes are read as zero
         const hipError_t e0 =
@@ -1435,7 +1442,10 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         P->regen = power && odd[1] == 0 && odd[2] == 0;
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression: %s", hipGetErrorString(e));
     }
-    hipError_t e = hipStreamSynchronize(s);
+    hipError_t e = hipSuccess;
+    // (behind the wait above: before it, it took that wait past the host's polling)
+    if (P->n1) e = hmx_launch_node_offsets(dp, b.rframe, b.cframe, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return fail(HM_ERR_HIP, "compression sync: %s", hipGetErrorString(e));
     return HM_OK;
 }
