@@ -139,7 +139,6 @@ struct DSplit {
 #define N1_NODES 47          // nodes per subtree (LDS: a rank vector each, N1_KB of them)
 #define N1_PATH 16           // path nodes staged together
 #define N1_KB 4              // right-hand sides per launch
-#define N1_SPLIT_CHUNKS 4096 // a downward workgroup per chunk up to this many chunks
 
 struct N1Sub {
     int32_t node, nnode;  // first node record, nodes

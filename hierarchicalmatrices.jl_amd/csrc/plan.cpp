@@ -464,12 +464,11 @@ struct N1Host {
     // the path and the subtree with three others at most), else so that about
     // 1024 to 2048 workgroups share the paths' work among their chunks.
     bool cut(const std::vector<DTNode> &t, const std::vector<N1Frame> &fr, const Side &S,
-             const std::vector<DDense> &dense, bool rows, size_t ncl) {
+             const std::vector<DDense> &dense, bool rows, size_t ncl, bool units) {
         const std::vector<DChunk> &dc = S.ch;
         const int64_t nch = (int64_t)dc.size();
         int32_t GC = 4;
-        if (nch > N1_SPLIT_CHUNKS)
-            while (GC < 32 && (int64_t)GC * 1024 < nch) GC *= 2;
+        while (GC < 32 && (int64_t)GC * 1024 < nch) GC *= 2;
         const size_t nt = t.size();
         std::vector<int32_t> nn(nt, 0), cb(nt, 0), cn(nt, 0);
         for (size_t k = nt; k-- > 0;) {  // halves come after their parent
@@ -595,7 +594,7 @@ struct N1Host {
             }
             pos += (size_t)u.npath + 1;
         }
-        if (nch <= N1_SPLIT_CHUNKS) {
+        if (!units) {
             for (int64_t c = 0; c < nch; ++c) {
                 ch[c].run = (int32_t)run.size();
                 ch[c].nrun = dc[c].near_end - dc[c].near_beg;
@@ -1016,9 +1015,24 @@ struct hm_plan {
         if (r > 32 || xt.empty() || yt.empty()) return;
         std::vector<DTNode> xs, ys;
         if (!nest && (!tree_nodes(xt, xs) || !tree_nodes(yt, ys))) return;
+        // Where the near field takes its columns through LDS for two chunks a
+        // wavefront (units), not by scalar loads for one a workgroup: above 1024
+        // chunks, where the units fill the chip (n = 131071, 1, 2 and 4 right-hand
+        // sides: Float32 Cauchy 36, 69, 72 -> 29, 48, 59 us; Float64 38, 79, 83 ->
+        // 34, 63, 70; n = 65536: 26, 44, 45 -> 24, 34, 38). Float64 entries that
+        // are read stream through k_down then: above 4096 (n = 131071, log kernel,
+        // 1 and 4: 64, 152 -> 71, 156; n = 200003: 109, 175 -> 106, 165). A Float64
+        // logarithm formed costs more than its column's load, and its workgroups
+        // are the better balanced the smaller they are: never (n = 131071: 119 us,
+        // 156 with units; n = 600000: 950, 1102).
+        auto units = [&](const Side &S) {
+            const bool power = kid == HM_CAUCHY || kid == HM_COULOMB || kid == HM_COULOMB3;
+            if (power || f32) return S.ch.size() > 1024;
+            return !(flags & HM_PLAN_MATRIX_FREE) && S.ch.size() > 4096;
+        };
         bool okx = false, oky = false;
-        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, frames(xt), rows, dense, true, rcl.size()); },
-                   [&] { oky = n1y.cut(nest ? ytn : ys, frames(yt), cols, dense, false, ccl.size()); });
+        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, frames(xt), rows, dense, true, rcl.size(), units(rows)); },
+                   [&] { oky = n1y.cut(nest ? ytn : ys, frames(yt), cols, dense, false, ccl.size(), units(cols)); });
         if (!okx || !oky) return;
         n1x.targets(rcl, by_rc, far, true, n1y);
         n1y.targets(ccl, by_cc, far, false, n1x);
@@ -2316,10 +2330,15 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
     // unless a node meets a point: there they are not finite, and the passes
     // take it from the marks that the compression left (a.basis). The route
     // does not hang on the points.
-    const bool n1 = P->n1;
     const int src = mode == 2 ? N1_FREE : P->regen ? N1_EXACT : N1_READ;
     for (int64_t q = 0; q < k;) {
-        // per level, forward products take up to HM_MAX_KB right-hand sides
+        // per level, forward products take up to HM_MAX_KB right-hand sides: eight
+        // of a small stored Float32 plan in one set of launches, where the trees
+        // take two (n = 4096, 128 chunks: 43 us, 53 over the trees; n = 1000: 33,
+        // 46; n = 10000: 78, 57). Eight of a Float64 plan go to the MFMA passes.
+        const bool eight = std::is_same_v<T, float> && mode == 0 && !tr && max_kb >= 8 &&
+                           k - q >= 8 && P->rows.ch.size() <= 128;
+        const bool n1 = P->n1 && !eight;
         int kb = 1;
         if (n1) kb = (int)std::min<int64_t>(std::min(max_kb, N1_KB), k - q);
         else if (!tr && max_kb > 1)
