@@ -2321,16 +2321,18 @@ static int matvec_common(hm_plan_t P, T *y, const T *x, int64_t ioff, int64_t jo
         if (prec >= 0) return fail(HM_ERR_UNSUPPORTED, "reduced-precision far field: Float64 plans only");
         if (flags & HM_MV_MFMA) return fail(HM_ERR_UNSUPPORTED, "MFMA passes: Float64 plans only");
     }
-    // a streamed near field (stored form) competes with the upward pass for
-    // HBM and gains nothing on a side stream; the computed ones (hybrid's
-    // Clenshaw far field, matrix-free kernel values) overlap the chain
-    const bool use_side = mode != 0 && split_near_field(P, s);
     // over the interval trees, up to N1_KB right-hand sides per launch. A
     // stored plan's U and V equal the Chebyshev form's basis up to rounding
     // unless a node meets a point: there they are not finite, and the passes
     // take it from the marks that the compression left (a.basis). The route
     // does not hang on the points.
     const int src = mode == 2 ? N1_FREE : P->regen ? N1_EXACT : N1_READ;
+    // A near field with launches of its own (per level, or entries streamed past
+    // the trees) may run on the plan's side stream. The stored form's competes
+    // with the upward pass for HBM and gains nothing there; the others overlap the
+    // chain.
+    const bool apart = !P->n1 || (src == N1_READ && (tr ? P->d_n1y : P->d_n1x).nunit > 0);
+    const bool use_side = mode != 0 && apart && split_near_field(P, s);
     for (int64_t q = 0; q < k;) {
         // per level, forward products take up to HM_MAX_KB right-hand sides: eight
         // of a small stored Float32 plan in one set of launches, where the trees
