@@ -146,7 +146,6 @@ struct N1Sub {
     int32_t leaf, nleaf;  // first leaf record, non-empty leaves
     int32_t path, npath;  // the nodes above the root, the tree's root first
     int32_t ch, nch;      // the chunks of its points
-    int32_t unit, nunit;  // their units (none where a workgroup takes a chunk)
 };
 
 struct N1Node {

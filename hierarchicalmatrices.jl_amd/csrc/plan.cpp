@@ -624,7 +624,6 @@ struct N1Host {
         };
         std::vector<N1UnitRun> ra, rb;
         for (N1Sub &u : sub) {
-            u.unit = (int32_t)unit.size();
             for (int32_t c = u.ch; c < u.ch + u.nch; c += 2) {
                 N1Unit w{c, std::min(2, u.ch + u.nch - c), (int32_t)urun.size(), 0};
                 rb.clear();
@@ -650,7 +649,6 @@ struct N1Host {
                 }
                 unit.push_back(w);
             }
-            u.nunit = (int32_t)unit.size() - u.unit;
         }
         return true;
     }
