@@ -96,14 +96,16 @@ struct DevPlanT {
     const int32_t *chunk_leaf;
     const DTask *yleaf;
     int32_t nyleaf;
-    const T *nestM;
+    const T *nestM, *nestD;  // the re-expansion matrices; the differentiation matrix,
+                             // where the node offsets enter the MFMA passes (else null)
     T *my, *mx;
     // one right-hand side over the interval trees (n1 is 0 when the trees or
     // the rank do not allow it), and its padded r x r matrices (N1Mat)
     int n1;
     N1Side n1x, n1y;
     const T *n1m;
-    // a cluster's mapped nodes less the exact ones, in its frame (r per cluster)
+    // a cluster's mapped nodes less the exact ones, in its frame (r per cluster),
+    // where the trees nest
     T *rdel, *cdel;
 };
 
@@ -137,7 +139,7 @@ using DevPlanF = DevPlanT<float>;
 using MvArgs = MvArgsT<double>;
 using MvArgsF = MvArgsT<float>;
 
-// rdel and cdel of a plan with n1, from the clusters' frames
+// rdel and cdel, from the clusters' frames
 hipError_t hmx_launch_node_offsets(const DevPlan &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
 hipError_t hmx_launch_node_offsets(const DevPlanF &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
 

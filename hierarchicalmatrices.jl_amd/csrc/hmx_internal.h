@@ -71,6 +71,7 @@ struct DTask {
     int64_t slot;    // partial-sum slot
     int64_t first;   // first point of the task (cluster first + off)
     double cx, cy;   // the cluster's (center, 1/halfwidth), Float64 plans
+    double clo;      // tree leaves: the second part of their frame's center (N1Frame)
 };
 
 struct DDense {
@@ -118,7 +119,8 @@ struct DTNode {
     int32_t child[2];  // -1 at a leaf
     int32_t cl;        // the row / column cluster with this range, or -1
     int32_t half;      // which half of its parent (0: the half holding the upper interval end)
-    double cx, cy;     // (center, 1/halfwidth) of its interval, as the cluster maps form them
+    double cx, cy;     // (center, 1/halfwidth) of its interval; the plan's nested trees: of its
+    double clo;        // frame, the center's second part (N1Frame; else 0)
 };
 
 // One indsplit of the tree: the range [first, first + len) of one side split

@@ -1436,15 +1436,60 @@ __device__ __forceinline__ void store_ranks(const md4_t (&Mo)[G][RP / 16], S *ds
     }
 }
 
+// The rounding of the mapped nodes, by their offsets d (DevPlanT's rdel, cdel),
+// to first order (nested1.h says why), W in the result layout, which is the
+// B operand of the K-steps as it stands: W -= D^T (d W) (node values of the
+// input side) or W -= d (D W) (of the output side, before A^T).
+template <int RP, int G, bool IN>
+__device__ __forceinline__ void node_offset_terms(const double *D, const double *del, int r,
+                                                  int j16, int g, md4_t (&W)[G][RP / 16]) {
+    constexpr int MT = RP / 16;
+    double d[MT][4];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = t * 16 + 4 * v + g;
+            d[t][v] = k < r ? del[k] : 0.0;
+        }
+    md4_t E[G][MT];
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi)
+#pragma unroll
+        for (int tt = 0; tt < MT; ++tt) E[gi][tt] = md4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = t * 16 + 4 * v + g;
+#pragma unroll
+            for (int tt = 0; tt < MT; ++tt) {
+                const int m = tt * 16 + j16;
+                const double av = (m < r && k < r) ? D[IN ? k * r + m : m * r + k] : 0.0;
+#pragma unroll
+                for (int gi = 0; gi < G; ++gi)
+                    E[gi][tt] = mfma64(av, IN ? d[t][v] * W[gi][t][v] : W[gi][t][v], E[gi][tt]);
+            }
+        }
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) W[gi][t][v] -= IN ? E[gi][t][v] : d[t][v] * E[gi][t][v];
+}
+
 // Node values w = A mu of one cluster from its moments held as in
 // store_ranks: Mo[gi][t][v] is B[k0 + g][j16] of the K-step k0 = 16t + 4v, so
 // the product takes mu from registers; A's rows are loaded once for the
 // groups. Stored as dst[q r + m], or (KQ, the nested far field's) as
-// dst[m 16G + q] (FP64, or rounded to FP32 once).
+// dst[m 16G + q] (FP64, or rounded to FP32 once), there with the node offsets'
+// terms.
 template <int RP, int G, class S, bool KQ = false>
 __device__ __forceinline__ void nodes_from_moments(const md4_t (&Mo)[G][RP / 16],
                                                    const double *chebA, S *dst, int r,
-                                                   int j16, int g) {
+                                                   int j16, int g, const double *D = nullptr,
+                                                   const double *del = nullptr) {
     constexpr int MT = RP / 16;
     double av[MT][MT][4];
 #pragma unroll
@@ -1467,6 +1512,9 @@ __device__ __forceinline__ void nodes_from_moments(const md4_t (&Mo)[G][RP / 16]
 #pragma unroll
                 for (int v = 0; v < 4; ++v) W[gi][tt] = mfma64(av[tt][t][v], Mo[gi][t][v], W[gi][tt]);
         }
+    if constexpr (KQ) {
+        if (D) node_offset_terms<RP, G, true>(D, del, r, j16, g, W);
+    }
     store_ranks<RP, G, KQ>(W, dst, r, j16, g);
 }
 
@@ -1498,7 +1546,8 @@ template <int RP, int PREC, int G, bool NEST, class WS>
 __global__ __launch_bounds__(WAVE) void k_up_m(const DTask *tasks, const double *pts,
                                               const double *xt, int64_t ldxt, int nq,
                                               const double *chebA, double *partial, WS *w,
-                                              int r, double *mom) {
+                                              int r, double *mom, const double *D,
+                                              const double *del) {
     static_assert(NEST || std::is_same<WS, double>::value, "per-level w is FP64");
     using TL = typename std::conditional<PREC == 2, double, float>::type;
     constexpr bool BF = PREC == 1 || PREC == 3;  // split-BF16 operands (K = 32 shape)
@@ -1537,7 +1586,8 @@ __global__ __launch_bounds__(WAVE) void k_up_m(const DTask *tasks, const double 
         if (lane < PTS) {
             const int i = base + lane;
             const bool ok = i < Tk.len;
-            const double xh = ok ? (pts[first + i] - cm.x) * cm.y : 0.0;
+            const double off = pts[first + i * (int)ok] - cm.x;
+            const double xh = ok ? (NEST ? off - Tk.clo : off) * cm.y : 0.0;
             double t0 = 1.0, t1 = xh;
 #pragma unroll
             for (int m = 0; m < RP; ++m) {
@@ -1609,7 +1659,8 @@ __global__ __launch_bounds__(WAVE) void k_up_m(const DTask *tasks, const double 
     if constexpr (NEST) {
         store_ranks<RP, G, true>(D64, mom + (int64_t)Tk.cl * MQT * r, r, j16, g);
         if (Tk.slot >= 0)
-            nodes_from_moments<RP, G, WS, true>(D64, chebA, w + Tk.slot * MQT * r, r, j16, g);
+            nodes_from_moments<RP, G, WS, true>(D64, chebA, w + Tk.slot * MQT * r, r, j16, g, D,
+                                                del + Tk.slot * r);
     } else if (Tk.single) {
         nodes_from_moments<RP, G>(D64, chebA, w + (int64_t)Tk.cl * MQT * r, r, j16, g);
     } else {  // a multi-task cluster's slot gets mu itself
@@ -1693,7 +1744,7 @@ __device__ __forceinline__ void m2m_node(const DTNode &N, const double *M, const
 template <int RP, int G, class WS, bool TWO>
 __global__ __launch_bounds__(WG) void k_m2m(const DTNode *tn, const int32_t *ids, int n,
                                            const double *M, double *mom, const double *chebA,
-                                           WS *w, int r) {
+                                           WS *w, int r, const double *D, const double *del) {
     constexpr int MT = RP / 16;
     constexpr int MQT = MQ * G;
     const int wid = wave_id();
@@ -1743,10 +1794,12 @@ __global__ __launch_bounds__(WG) void k_m2m(const DTNode *tn, const int32_t *ids
         for (int h = 0; h < 2; ++h)
             if (in[h] && Cn[h].cl >= 0)
                 nodes_from_moments<RP, G, WS, true>(mu[h], chebA, w + (int64_t)Cn[h].cl * MQT * r, r,
-                                                    j16, g);
+                                                    j16, g, D, del + (int64_t)Cn[h].cl * r);
     }
     store_ranks<RP, G, true>(W, mom + (int64_t)P * MQT * r, r, j16, g);
-    if (N.cl >= 0) nodes_from_moments<RP, G, WS, true>(W, chebA, w + (int64_t)N.cl * MQT * r, r, j16, g);
+    if (N.cl >= 0)
+        nodes_from_moments<RP, G, WS, true>(W, chebA, w + (int64_t)N.cl * MQT * r, r, j16, g, D,
+                                            del + (int64_t)N.cl * r);
 }
 
 // z[N's row cluster] (zero if it is none) in the result layout (the FP64
@@ -1918,6 +1971,10 @@ __global__ __launch_bounds__(WG) void k_translate_m(DevPlan p, const DCluster *c
                         for (int gi = 0; gi < G; ++gi) Z[gi][t] = mfma64(av[h][t], bv[gi][h], Z[gi][t]);
             }
         }
+    }
+    if constexpr (KQ) {
+        if (p.nestD)
+            node_offset_terms<RP, G, false>(p.nestD, p.rdel + (int64_t)wid * r, r, j16, g, Z);
     }
     // C[m][q] = sum_k A[k][m] Z[k][q]; this lane holds Z[16t + g + 4v][j16] in
     // Z[t][v], which is B[k0 + g][j16] of the K-step k0 = 16t + 4v
@@ -2237,7 +2294,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(down_m_waves
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             if (t >= nt) break;
-            const double xh = (pf[t] - L.cx) * L.cy;
+            const double xh = ((pf[t] - L.cx) - L.clo) * L.cy;
             const double x2 = xh + xh;
             const double c2 = __builtin_fma(x2, xh, -1.0), c3 = __builtin_fma(x2, c2, -xh);
             const double c4 = __builtin_fma(x2, c3, -c2), c5 = __builtin_fma(x2, c4, -c3);
@@ -2445,7 +2502,7 @@ hipError_t matvec_m_t(const DevPlan &p, const MvArgs &a, int nq, hipStream_t s) 
     if (p.nfar > 0 && nest) {
         if (p.nyleaf > 0)
             k_up_m<RP, PREC, G, true, WS><<<p.nyleaf, WAVE, 0, s>>>(
-                p.yleaf, p.y, xr, ldxr, nq, p.chebA, a.partial, wn, p.r, p.my);
+                p.yleaf, p.y, xr, ldxr, nq, p.chebA, a.partial, wn, p.r, p.my, p.nestD, p.cdel);
         // moments: two depths per launch (the even depths, each with the one
         // below it) where the second node's registers fit, else one
         constexpr bool TWO = RP <= 32;
@@ -2453,7 +2510,8 @@ hipError_t matvec_m_t(const DevPlan &p, const MvArgs &a, int nq, hipStream_t s) 
             const int off = p.ylev_off_h[d], cnt = p.ylev_off_h[d + 1] - off;
             if (cnt > 0)
                 k_m2m<RP, G, WS, TWO><<<nblk(cnt), WG, 0, s>>>(p.ytn, p.ylev + off, cnt, p.nestM,
-                                                                p.my, p.chebA, wn, p.r);
+                                                                p.my, p.chebA, wn, p.r, p.nestD,
+                                                                p.cdel);
         }
         k_translate_m<RP, FREE, KID, G, WS, true><<<nblk(p.nrc), WG, 0, s>>>(p, p.rcl, p.nrc, wn, zn);
         for (int d = 0; d < p.nxlev; ++d) {
@@ -2464,7 +2522,7 @@ hipError_t matvec_m_t(const DevPlan &p, const MvArgs &a, int nq, hipStream_t s) 
         }
     } else if (p.nfar > 0 && p.nctask > 0) {
         k_up_m<RP, PREC, G, false, double><<<p.nctask, WAVE, 0, s>>>(
-            p.ctask, p.y, xr, ldxr, nq, p.chebA, a.partial, a.w, p.r, nullptr);
+            p.ctask, p.y, xr, ldxr, nq, p.chebA, a.partial, a.w, p.r, nullptr, nullptr, nullptr);
         if (p.nmulti_c > 0)
             k_reduce<double, true, MQT><<<nblk(p.nmulti_c), WG, 0, s>>>(
                 p.ccl, p.multi_c, p.nmulti_c, a.partial, p.chebA, a.w, p.r);

@@ -457,7 +457,6 @@ struct N1Host {
     std::vector<int64_t> sbase;
     std::vector<int32_t> scount;
     int64_t slots = 0;
-    std::vector<N1Frame> frame;  // per cluster
 
     // A subtree has at most N1_NODES nodes and GC chunks (or is one leaf).
     // GC: 4 while a downward workgroup takes one chunk (its wavefronts share
@@ -501,9 +500,6 @@ struct N1Host {
                 if (!one) return false;
             }
         }
-        frame.resize(ncl);
-        for (size_t k = 0; k < nt; ++k)
-            if (t[k].cl >= 0) frame[t[k].cl] = fr[k];
         sbase.assign(ncl, 0);
         scount.assign(ncl, 0);
         ch.resize(dc.size());
@@ -782,7 +778,7 @@ struct PlanBufs {
     T *yt = nullptr;  // a split product's far field (hybrid and matrix-free plans)
     // nested far field of the MFMA passes (Float64 plans): the re-expansion
     // matrices, moments per column node, coefficients per row node
-    T *nestM = nullptr, *my = nullptr, *mx = nullptr;
+    T *nestM = nullptr, *nestD = nullptr, *my = nullptr, *mx = nullptr;
     // padded matrices of the single-right-hand-side tree passes, node offsets
     T *n1m = nullptr, *rdel = nullptr, *cdel = nullptr;
     N1Frame *rframe = nullptr, *cframe = nullptr;  // per cluster
@@ -856,7 +852,9 @@ struct hm_plan {
     // sides' tables; regen: a stored or hybrid plan's dense entries and F are
     // formed from the points and nodes instead of read
     bool n1 = false, regen = false;
+    bool nest_offsets = false;  // the MFMA passes take the node offsets in
     N1Host n1x, n1y;
+    std::vector<N1Frame> rframe, cframe;  // per cluster, where the trees nest (until uploaded)
     N1Side d_n1x{}, d_n1y{};
     void *d_tables = nullptr;  // the one allocation holding d_rcl .. d_yleaf (Staging)
     // side stream and fork / join events of products whose near field runs
@@ -935,9 +933,10 @@ struct hm_plan {
     // its parent's interval to the rounding of the interval ends. Float64
     // ends are rounded to eps |end|, which is eps |end| / halfwidth in the
     // node's variable (7e-12 at depth 14 of [0, 1]; the mapped nodes behind F
-    // carry the same). Float32 trees nest where the midpoints are exact.
+    // carry the same). Float32 trees nest where the midpoints are exact. worst:
+    // grows to the largest deviation from a half.
     template <class TN>
-    bool tree_nodes(const std::vector<TN> &t, std::vector<DTNode> &o) const {
+    bool tree_nodes(const std::vector<TN> &t, std::vector<DTNode> &o, double &worst) const {
         o.resize(t.size());
         for (size_t k = 0; k < t.size(); ++k) {
             const TN &q = t[k];
@@ -961,9 +960,9 @@ struct hm_plan {
             const double alpha = P.cy / d.cy, beta = (d.cx - P.cx) * P.cy;
             const double end = std::max(std::fabs(t[k].lo), std::fabs(t[k].hi));
             const double tol = std::max(1e-12, std::min(1e-10, 4.0 * 0x1p-52 * end * std::fabs(d.cy)));
-            if (!(std::fabs(alpha - 0.5) <= tol) ||
-                !(std::fabs(beta - (d.half ? 0.5 : -0.5)) <= tol))
-                return false;
+            const double da = std::fabs(alpha - 0.5), db = std::fabs(beta - (d.half ? 0.5 : -0.5));
+            if (!(da <= tol) || !(db <= tol)) return false;
+            worst = std::max({worst, da, db});
         }
         return true;
     }
@@ -1002,17 +1001,27 @@ struct hm_plan {
         return o;
     }
 
+    template <class TN>
+    static void cluster_frames(const std::vector<TN> &t, const std::vector<N1Frame> &f, size_t ncl,
+                               std::vector<N1Frame> &o) {
+        o.resize(ncl);
+        for (size_t k = 0; k < t.size(); ++k)
+            if (t[k].cl >= 0) o[t[k].cl] = f[k];
+    }
+
     // Tables of the single-right-hand-side tree passes; n1 stays false (the
     // per-level passes are used) where the trees do not nest, a chunk lies in
     // several leaves, or the rank exceeds 32 (a wavefront's two halves hold a
     // matrix row per lane).
     template <class TN>
     void build_n1(const std::vector<TN> &xt, const std::vector<TN> &yt,
+                  const std::vector<N1Frame> &fx, const std::vector<N1Frame> &fy,
                   const std::vector<int32_t> &by_rc, const std::vector<int32_t> &by_cc) {
         n1 = false;
         if (r > 32 || xt.empty() || yt.empty()) return;
         std::vector<DTNode> xs, ys;
-        if (!nest && (!tree_nodes(xt, xs) || !tree_nodes(yt, ys))) return;
+        double worst = 0.0;
+        if (!nest && (!tree_nodes(xt, xs, worst) || !tree_nodes(yt, ys, worst))) return;
         // Where the near field takes its columns through LDS for two chunks a
         // wavefront (units), not by scalar loads for one a workgroup: above 1024
         // chunks, where the units fill the chip (n = 131071, 1, 2 and 4 right-hand
@@ -1029,8 +1038,8 @@ struct hm_plan {
             return !(flags & HM_PLAN_MATRIX_FREE) && S.ch.size() > 4096;
         };
         bool okx = false, oky = false;
-        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, frames(xt), rows, dense, true, rcl.size(), units(rows)); },
-                   [&] { oky = n1y.cut(nest ? ytn : ys, frames(yt), cols, dense, false, ccl.size(), units(cols)); });
+        both_sides(nx + ny, [&] { okx = n1x.cut(nest ? xtn : xs, fx, rows, dense, true, rcl.size(), units(rows)); },
+                   [&] { oky = n1y.cut(nest ? ytn : ys, fy, cols, dense, false, ccl.size(), units(cols)); });
         if (!okx || !oky) return;
         n1x.targets(rcl, by_rc, far, true, n1y);
         n1y.targets(ccl, by_cc, far, false, n1x);
@@ -1043,10 +1052,29 @@ struct hm_plan {
     // back by their deepest intervals' rounding), every column leaf fits one
     // upward task and every row chunk lies in one row leaf.
     template <class TN>
-    void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt) {
+    void build_nest(const std::vector<TN> &xt, const std::vector<TN> &yt,
+                    const std::vector<N1Frame> &fx, const std::vector<N1Frame> &fy) {
         nest = false;
         if (f32 || xt.empty() || yt.empty()) return;
-        if (!tree_nodes(xt, xtn) || !tree_nodes(yt, ytn)) return;
+        double worst = 0.0;
+        if (!tree_nodes(xt, xtn, worst) || !tree_nodes(yt, ytn, worst)) return;
+        // Halves off by more than 1e-12 (deep trees over rounded ends) would show in
+        // the products: there the leaves take the exact frames and the clusters their
+        // nodes' offsets, else the leaves' own intervals do. (n = 400000, leaf 40,
+        // log kernel: 4.4e-15 per level, 5.6e-15 without the offsets, 7.9e-16 with
+        // them. They cost 32 x 256 batched instances 4 %, n = 2^22 2 %.)
+        nest_offsets = worst > 1e-12;
+        if (nest_offsets) {
+            auto into = [](const std::vector<N1Frame> &f, std::vector<DTNode> &t) {
+                for (size_t k = 0; k < t.size(); ++k) {
+                    t[k].cx = f[k].cx;
+                    t[k].clo = f[k].cl;
+                    t[k].cy = f[k].cy;
+                }
+            };
+            into(fx, xtn);
+            into(fy, ytn);
+        }
         auto by_depth = [](const std::vector<TN> &t, bool internal_only, std::vector<int32_t> &ids,
                            std::vector<int32_t> &off) {
             int maxd = 0;
@@ -1078,6 +1106,7 @@ struct hm_plan {
             T.slot = d.cl;
             T.first = d.first;
             T.cx = d.cx;
+            T.clo = d.clo;
             T.cy = d.cy;
             yleaf.push_back(T);
         }
@@ -1238,19 +1267,9 @@ std::vector<T> nest_matrices(int r) {
 }
 }  // extern "C++"
 
-// The matrices of the single-right-hand-side tree passes, laid out for lanes
-// (m, h) = (lane % 32, lane / 32) and padded with zeros to the rank bucket
-// (N1Mat): M_h[m][k], M_h[k][m], A[m][h R/2 + j], A[h R/2 + j][m], and of the
-// nodes' differentiation matrix D (values at the nodes -> the polynomial's
-// derivatives there; the barycentric formula) D[h R/2 + j][m], D[m][h R/2 + j].
-extern "C++" {
-template <class T>
-std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> &A) {
-    const int R = r <= 8 ? 8 : r <= 16 ? 16 : (r <= 24 && std::is_same_v<T, double>) ? 24 : 32;
-    const int HALF = R / 2;
-    std::vector<T> out((size_t)(2 * R + 4 * HALF) * 64, T(0));
-    T *MU = out.data(), *MD = MU + (size_t)R * 64, *AU = MD + (size_t)R * 64,
-      *DU = AU + (size_t)HALF * 64, *AT = DU + (size_t)HALF * 64, *DD = AT + (size_t)HALF * 64;
+// The differentiation matrix of the nodes t_k = cos((2k + 1) pi / (2r)): values
+// there -> the polynomial's derivatives there, D[k r + j] (the barycentric formula)
+static std::vector<double> node_derivative(int r) {
     std::vector<double> D((size_t)r * r, 0.0), sn(2 * r);  // sn[i] = sin(i pi / (2r))
     for (int i = 0; i < 2 * r; ++i) sn[i] = std::sin(i * M_PI / (2 * r));
     for (int k = 0; k < r; ++k)
@@ -1263,6 +1282,22 @@ std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> 
             D[(size_t)k * r + j] = ((k + j) & 1) ? -q : q;
             D[(size_t)k * r + k] -= D[(size_t)k * r + j];
         }
+    return D;
+}
+
+// The matrices of the single-right-hand-side tree passes, laid out for lanes
+// (m, h) = (lane % 32, lane / 32) and padded with zeros to the rank bucket
+// (N1Mat): M_h[m][k], M_h[k][m], A[m][h R/2 + j], A[h R/2 + j][m], and of the
+// nodes' differentiation matrix D[h R/2 + j][m], D[m][h R/2 + j].
+extern "C++" {
+template <class T>
+std::vector<T> n1_matrices(int r, const std::vector<T> &M, const std::vector<T> &A,
+                           const std::vector<double> &D) {
+    const int R = r <= 8 ? 8 : r <= 16 ? 16 : (r <= 24 && std::is_same_v<T, double>) ? 24 : 32;
+    const int HALF = R / 2;
+    std::vector<T> out((size_t)(2 * R + 4 * HALF) * 64, T(0));
+    T *MU = out.data(), *MD = MU + (size_t)R * 64, *AU = MD + (size_t)R * 64,
+      *DU = AU + (size_t)HALF * 64, *AT = DU + (size_t)HALF * 64, *DD = AT + (size_t)HALF * 64;
     for (int lane = 0; lane < 64; ++lane) {
         const int m = lane % 32, h = lane / 32;
         if (m >= r) continue;
@@ -1337,7 +1372,10 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     }
     std::vector<T> nestM, n1m;
     if ((std::is_same_v<T, double> && P->nest) || P->n1) nestM = nest_matrices<T>(r);
-    if (P->n1) n1m = n1_matrices<T>(r, nestM, chebA);
+    std::vector<double> D;
+    if (P->nest || P->n1) D = node_derivative(r);
+    const std::vector<T> nestD(D.begin(), D.end());
+    if (P->n1) n1m = n1_matrices<T>(r, nestM, chebA, D);
     int rc;
 #define HM_TRY_T(expr) do { rc = (expr); if (rc != HM_OK) return rc; } while (0)
     const int64_t nslots = std::max(P->rows.nslots, P->cols.nslots);
@@ -1359,13 +1397,14 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         st.add(&b.chebA, chebA);
         if (std::is_same_v<T, double> && P->nest) {
             st.add(&b.nestM, nestM);
+            if (P->nest_offsets) st.add(&b.nestD, nestD);
             st.reserve(&b.my, (int64_t)P->ytn.size() * r * HM_WS_RHS);
             st.reserve(&b.mx, (int64_t)P->xtn.size() * r * HM_WS_RHS);
         }
-        if (P->n1) {
-            st.add(&b.n1m, n1m);
-            st.add(&b.rframe, P->n1x.frame);
-            st.add(&b.cframe, P->n1y.frame);
+        if (P->n1) st.add(&b.n1m, n1m);
+        if (!P->rframe.empty() || !P->cframe.empty()) {
+            st.add(&b.rframe, P->rframe);
+            st.add(&b.cframe, P->cframe);
             st.reserve(&b.rdel, (int64_t)rn.size());
             st.reserve(&b.cdel, (int64_t)cn.size());
         }
@@ -1379,8 +1418,6 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (bases) st.reserve(&b.cnt, 4 * HM_COUNT_BLOCKS + (odd_bytes + 7) / 8);
         else if (!(flags & HM_PLAN_MATRIX_FREE)) st.add(&b.cnt, cnt0);
         HM_TRY_T(st.commit(&b.arena));
-        P->n1x.frame.clear();
-        P->n1y.frame.clear();
     }
     if (b.my) {  // the moments of empty column nodes are read as zero
         const hipError_t e0 =
@@ -1405,7 +1442,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     dp.x = b.x; dp.y = b.y; dp.lam = b.lam;
     dp.rnodes = b.rnodes; dp.cnodes = b.cnodes;
     dp.rmap = b.rmap; dp.cmap = b.cmap; dp.chebA = b.chebA;
-    dp.nestM = b.nestM; dp.my = b.my; dp.mx = b.mx;
+    dp.nestM = b.nestM; dp.nestD = b.nestD; dp.my = b.my; dp.mx = b.mx;
     dp.n1m = b.n1m; dp.rdel = b.rdel; dp.cdel = b.cdel;
     dp.A = b.A; dp.U = b.U; dp.V = b.V; dp.F = b.F;
 
@@ -1456,7 +1493,9 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
     }
     hipError_t e = hipSuccess;
     // (behind the wait above: before it, it took that wait past the host's polling)
-    if (P->n1) e = hmx_launch_node_offsets(dp, b.rframe, b.cframe, s);
+    if (b.rdel || b.cdel) e = hmx_launch_node_offsets(dp, b.rframe, b.cframe, s);
+    P->rframe.clear();
+    P->cframe.clear();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return fail(HM_ERR_HIP, "compression sync: %s", hipGetErrorString(e));
     return HM_OK;
@@ -1633,8 +1672,15 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
     both_sides(nx + ny, [&] { build_side(nx, P->dense, true, P->rcl, P->rows); },
                [&] { build_side(ny, P->dense, false, P->ccl, P->cols); });
     P->list_multi();
-    P->build_nest(B.xt, B.yt);
-    P->build_n1(B.xt, B.yt, by_rc, by_cc);
+    {
+        const std::vector<N1Frame> fx = P->frames(B.xt), fy = P->frames(B.yt);
+        P->build_nest(B.xt, B.yt, fx, fy);
+        P->build_n1(B.xt, B.yt, fx, fy, by_rc, by_cc);
+        if (P->n1 || (P->nest && P->nest_offsets)) {
+            hm_plan::cluster_frames(B.xt, fx, P->rcl.size(), P->rframe);
+            hm_plan::cluster_frames(B.yt, fy, P->ccl.size(), P->cframe);
+        }
+    }
     // the cluster maps the Float64 MFMA upward pass reads from its task
     // record: (a+b)/2 and 1/((b-a)/2) as the Float64 cluster maps form them
     if (!f32) {
@@ -1715,13 +1761,10 @@ static int make_plan(int kernel_id, const Inst *inst, int64_t count, int blocksi
         HM_TRY(st.commit(&P->d_tables));
         // the device holds these now
         const int64_t sx = P->n1x.slots, sy = P->n1y.slots;
-        std::vector<N1Frame> fx = std::move(P->n1x.frame), fy = std::move(P->n1y.frame);
         P->n1x = N1Host{};
         P->n1y = N1Host{};
         P->n1x.slots = sx;
         P->n1y.slots = sy;
-        P->n1x.frame = std::move(fx);
-        P->n1y.frame = std::move(fy);
     }
     P->far_by_rc_h = std::move(by_rc);
     if (f32) HM_TRY(setup_typed<float>(P, x, y, B.rcl, B.ccl, flags, nA, nU, nV, nF, (hipStream_t)stream));

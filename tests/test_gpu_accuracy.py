@@ -55,3 +55,21 @@ def test_float32(cuda, form):
     assert len(rows) > 16 and (form == "stored" or np.isfinite(u).all())
     K = 1 / (x[rows].astype(np.float64)[:, None] - y.astype(np.float64)[None, :])
     assert error(u[rows], K, b.astype(np.float64)) <= 1e-6
+
+
+@pytest.mark.parametrize("form", ["hybrid", "free"])
+@pytest.mark.parametrize("seed", [2, 3])
+def test_deep_nested(cuda, form, seed):
+    # eight right-hand sides over trees whose halves are rounded by more than 1e-12: no further off
+    # than the products that apply every covering cluster (4.4e-15)
+    n, k = 400000, 8
+    x = np.sort(np.random.default_rng(seed).random(n))[::-1].copy()
+    y = x + 0.5 / n
+    H = hmx.KernelMatrix("logkernel", x, y, x[0], x[-1], y[0], y[-1], blocksize=40, rank=24,
+                         hybrid=form == "hybrid", matrix_free=form == "free")
+    assert H.info["nested"] == 1
+    b = np.random.default_rng(100 + seed).standard_normal((n, k))
+    rows = np.arange(0, n, n // 48)
+    u = H.matvec(torch.from_numpy(b).to(cuda), mfma=True).cpu().numpy()[rows]
+    K = np.log(abs(x[rows].astype(np.longdouble)[:, None] - y.astype(np.longdouble)[None, :]))
+    assert error(u, K, b.astype(np.longdouble)) <= 4.4e-15
