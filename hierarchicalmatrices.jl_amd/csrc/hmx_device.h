@@ -139,7 +139,8 @@ using DevPlanF = DevPlanT<float>;
 using MvArgs = MvArgsT<double>;
 using MvArgsF = MvArgsT<float>;
 
-// rdel and cdel, from the clusters' frames
+// rdel and cdel, from the clusters' frames (matrix-free plans; the others' come
+// with the count below)
 hipError_t hmx_launch_node_offsets(const DevPlan &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
 hipError_t hmx_launch_node_offsets(const DevPlanF &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s);
 
@@ -175,10 +176,12 @@ hipError_t hmx_launch_grad(const DevPlan &p, const MvArgs &a, bool transpose, do
 hipError_t hmx_launch_entries(const DevPlan &p, int64_t n, const int64_t *i, const int64_t *j,
                               const int32_t *kind, const int32_t *id, double *out, hipStream_t s);
 // non-finite values of the generated factors (after compression): the arrays
-// v[q] of n[q] values, HM_COUNT_BLOCKS partial counts each
+// v[q] of n[q] values, HM_COUNT_BLOCKS partial counts each; and the node offsets
+// of a plan that has them
 #define HM_COUNT_BLOCKS 256
 hipError_t hmx_launch_count_nonfinite(const double *const v[4], const int64_t n[4],
-                                      unsigned long long *count, hipStream_t s);
+                                      unsigned long long *count, const DevPlan &p, const N1Frame *rf,
+                                      const N1Frame *cf, hipStream_t s);
 
 // in-place diagonal scaling of stored dense blocks and bases (plans built
 // from blocks): side 0 scales columns (A and V rows), 1 rows (A and U rows);
@@ -222,4 +225,5 @@ hipError_t hmx_launch_grad(const DevPlanF &p, const MvArgsF &a, bool transpose, 
 hipError_t hmx_launch_entries(const DevPlanF &p, int64_t n, const int64_t *i, const int64_t *j,
                               const int32_t *kind, const int32_t *id, float *out, hipStream_t s);
 hipError_t hmx_launch_count_nonfinite(const float *const v[4], const int64_t n[4],
-                                      unsigned long long *count, hipStream_t s);
+                                      unsigned long long *count, const DevPlanF &p, const N1Frame *rf,
+                                      const N1Frame *cf, hipStream_t s);

@@ -66,13 +66,15 @@ hipError_t hmx_launch_entries(const DevPlan &p, int64_t n, const int64_t *i, con
 }
 
 hipError_t hmx_launch_count_nonfinite(const double *const v[4], const int64_t n[4],
-                                      unsigned long long *blockcount, hipStream_t s) {
+                                      unsigned long long *blockcount, const DevPlan &p,
+                                      const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
     hmxk::CountArgs<double> a;
     for (int q = 0; q < 4; ++q) {
         a.v[q] = v[q];
         a.n[q] = v[q] ? n[q] : 0;
     }
-    hmxk::k_count_nonfinite<double><<<dim3(HM_COUNT_BLOCKS, 4), hmxk::WG, 0, s>>>(a, blockcount);
+    hmxk::k_count_nonfinite<double><<<dim3(HM_COUNT_BLOCKS, p.rdel ? 5 : 4), hmxk::WG, 0, s>>>(
+        a, blockcount, p, rf, cf);
     return hipGetLastError();
 }
 
@@ -134,13 +136,15 @@ hipError_t hmx_launch_entries(const DevPlanF &p, int64_t n, const int64_t *i, co
 }
 
 hipError_t hmx_launch_count_nonfinite(const float *const v[4], const int64_t n[4],
-                                      unsigned long long *blockcount, hipStream_t s) {
+                                      unsigned long long *blockcount, const DevPlanF &p,
+                                      const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
     hmxk::CountArgs<float> a;
     for (int q = 0; q < 4; ++q) {
         a.v[q] = v[q];
         a.n[q] = v[q] ? n[q] : 0;
     }
-    hmxk::k_count_nonfinite<float><<<dim3(HM_COUNT_BLOCKS, 4), hmxk::WG, 0, s>>>(a, blockcount);
+    hmxk::k_count_nonfinite<float><<<dim3(HM_COUNT_BLOCKS, p.rdel ? 5 : 4), hmxk::WG, 0, s>>>(
+        a, blockcount, p, rf, cf);
     return hipGetLastError();
 }
 

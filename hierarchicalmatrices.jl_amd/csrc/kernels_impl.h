@@ -323,8 +323,8 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
 // their cluster's frame, by rounding (the differences from the center are exact
 // or nearly so)
 template <class T>
-__global__ __launch_bounds__(WG) void k_node_offsets(DevPlanT<T> p, const N1Frame *rf,
-                                                     const N1Frame *cf) {
+__device__ __forceinline__ void node_offset_block(const DevPlanT<T> &p, const N1Frame *rf,
+                                                  const N1Frame *cf) {
     const int64_t nr = (int64_t)p.nrc * p.r, n = nr + (int64_t)p.ncc * p.r;
     for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
         const bool row = i < nr;
@@ -334,6 +334,11 @@ __global__ __launch_bounds__(WG) void k_node_offsets(DevPlanT<T> p, const N1Fram
         (row ? p.rdel : p.cdel)[at] =
             (T)(((t - f.cx) - f.cl) * f.cy - cospi((2 * (int)(at - c * p.r) + 1) / (2.0 * p.r)));
     }
+}
+template <class T>
+__global__ __launch_bounds__(WG) void k_node_offsets(DevPlanT<T> p, const N1Frame *rf,
+                                                     const N1Frame *cf) {
+    node_offset_block(p, rf, cf);
 }
 template <class T>
 hipError_t node_offsets(const DevPlanT<T> &p, const N1Frame *rf, const N1Frame *cf, hipStream_t s) {
@@ -355,7 +360,8 @@ void clear_odd(const DevPlanT<T> &p, hipStream_t s) {
 }
 
 // Non-finite values of up to four arrays, one count per workgroup (gridDim.x of
-// them) and array (blockIdx.y)
+// them) and array (blockIdx.y); the fifth row of workgroups forms the node
+// offsets meanwhile (a launch of their own cost small plans 15 to 50 us)
 template <class T>
 struct CountArgs {
     const T *v[4];
@@ -363,7 +369,13 @@ struct CountArgs {
 };
 template <class T>
 __global__ __launch_bounds__(WG) void k_count_nonfinite(CountArgs<T> a,
-                                                        unsigned long long *blockcount) {
+                                                        unsigned long long *blockcount,
+                                                        DevPlanT<T> p, const N1Frame *rf,
+                                                        const N1Frame *cf) {
+    if (blockIdx.y == 4) {
+        node_offset_block(p, rf, cf);
+        return;
+    }
     __shared__ unsigned int sh[WG];
     const T *v = a.v[blockIdx.y];
     const int64_t n = a.n[blockIdx.y];

@@ -1471,7 +1471,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         const T *arrs[] = {user ? nullptr : b.A, b.U, b.V, user ? nullptr : b.F};
         const int64_t lens[] = {nA, nU, nV, nF};
         std::vector<unsigned long long> h(4 * HM_COUNT_BLOCKS + 2, 0);  // 2: the odd words
-        e = hmx_launch_count_nonfinite(arrs, lens, b.cnt, s);
+        e = hmx_launch_count_nonfinite(arrs, lens, b.cnt, dp, b.rframe, b.cframe, s);
         if (e == hipSuccess)
             e = hipMemcpyAsync(h.data(), b.cnt, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1492,8 +1492,7 @@ int setup_typed(hm_plan *P, const double *x, const double *y, const std::vector<
         if (e != hipSuccess) return fail(HM_ERR_HIP, "compression: %s", hipGetErrorString(e));
     }
     hipError_t e = hipSuccess;
-    // (behind the wait above: before it, it took that wait past the host's polling)
-    if (b.rdel || b.cdel) e = hmx_launch_node_offsets(dp, b.rframe, b.cframe, s);
+    if (!stored && b.rdel) e = hmx_launch_node_offsets(dp, b.rframe, b.cframe, s);
     P->rframe.clear();
     P->cframe.clear();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
