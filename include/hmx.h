@@ -240,7 +240,9 @@ enum hm_info {
     HM_INFO_N_D, HM_INFO_N_K1, HM_INFO_N_K2, HM_INFO_N_DENSE, HM_INFO_N_FAR,
     HM_INFO_N_ROWCLUSTERS, HM_INFO_N_COLCLUSTERS, HM_INFO_DEPTH,
     HM_INFO_DENSE_ENTRIES, HM_INFO_BASIS_ROWS_U, HM_INFO_BASIS_ROWS_V,
-    HM_INFO_BYTES_STORED,      /* bytes of every stored array read by one product */
+    HM_INFO_BYTES_STORED,      /* bytes of the stored arrays that a product per covering cluster
+                                  reads; one over the interval trees (hm_matvec) reads no U
+                                  and V, and no A and F of the kernels 1/d^m */
     HM_INFO_BYTES_REF_LAYOUT,  /* same arrays in the reference's per-block layout */
     HM_INFO_FLAGS, HM_INFO_N_ROWCHUNKS, HM_INFO_N_COLCHUNKS, HM_INFO_NONFINITE,
     HM_INFO_N_INSTANCES, HM_INFO_FROM_BLOCKS,
@@ -262,10 +264,21 @@ int hm_plan_blocks(hm_plan_t plan, int64_t *ints, double *dbls, int64_t cap, int
  * for q < k right-hand sides, beta in {0, 1}. beta = 1 is the reference's
  * accumulating mul!(u, H, v, istart, jstart) (src/KernelMatrix.jl:14-45, the
  * leaf loops src/algebra.jl:34-48 and :243-277); beta = 0 is H*v
- * (src/KernelMatrix.jl:5-8). Hybrid and matrix-free products with at least
- * 2^24 near-field entries run the near field on a stream the plan owns,
- * forked from and joined back to `stream` by events; a product stays on
- * `stream` while it is being captured or pass profiling is on. */
+ * (src/KernelMatrix.jl:5-8).
+ * Where the intervals halve to rounding and the rank is at most 32, one to
+ * four right-hand sides per launch go over the interval trees: three launches,
+ * each with a part of the near field. Stored and hybrid plans of the kernels
+ * 1/d^m then form the entries that they hold, with the same values; a row is
+ * not finite where U, V or an entry is not, as if they were read. Otherwise
+ * every covering cluster is applied, level by level. The route is fixed when
+ * the plan is made: new points (hm_plan_update_points) do not change it, the
+ * host waits for nothing, and a captured product holds for them.
+ * A near field with launches of its own (level by level, or entries that are
+ * read of plans with more than 4096 chunks of 64 rows, Float32 1024) of a hybrid
+ * or matrix-free product with at least 2^24 near-field entries runs on a
+ * stream the plan owns, forked from and joined back to `stream` by events; a
+ * product stays on `stream` while it is being captured or pass profiling is
+ * on. */
 int hm_matvec(hm_plan_t plan, double *y, const double *x, int64_t ioff, int64_t joff,
               int64_t incy, int64_t incx, int64_t k, int64_t ldy, int64_t ldx, int beta,
               unsigned flags, void *stream);
@@ -332,7 +345,10 @@ int hm_plan_tune(hm_plan_t plan, void *y, const void *x, int64_t k, void *stream
 
 /* Per-pass timing of the products of this plan (bench support, no counterpart
  * in the reference). enable=1 starts recording HIP events around the four
- * passes of every later product (up, reduce, translate, down) on its stream;
+ * passes of every later product (up, reduce, translate, down) on its stream
+ * (over the interval trees: the upward launch with five ninths of the near
+ * field, nothing, the translation with the rest of it, and the downward
+ * launch, before it a near field with launches of its own);
  * enable=0 stops and discards. hm_plan_profile_read synchronises, returns the
  * summed milliseconds per pass in ms[0..3] and the number of products. */
 int hm_plan_profile(hm_plan_t plan, int enable);
