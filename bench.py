@@ -8,12 +8,13 @@ Workload (one "step" = one product y = H b over the whole matrix):
 
 Prints one JSON line. `value` is matvecs/s of the stored-factor plan's product;
 the matrix-free variant is reported beside it. The single right-hand side's
-product forms the entries of A and F from the points and nodes (as they are
-stored, bit for bit) and never reads U and V, so it is bound by FP64 vector
-issue: `roofline` describes the dominant kernel (the upward launch, which
+product forms the entries of A and F from the points and nodes (equal to the
+stored ones but for rare half-way cases of a reciprocal) and never reads U and
+V, so it is bound by FP64 vector issue: `roofline` describes the dominant kernel (the upward launch, which
 carries five ninths of the near field) from HIP events recorded around each
-pass. `bytes_per_matvec` is the counted HBM traffic of a product (see
-`hbm_source`); `bytes_stored` is what the plan holds.
+pass. `bytes_per_matvec` is the HBM traffic of a product as counted once, in the
+committed profile (see `hbm_source`), not by this run; `bytes_stored` is what
+the plan holds.
 `cpu_baseline` times the oracle's restatement of the reference mul! on the
 host (bounded sample, see its `sample` field).
 """

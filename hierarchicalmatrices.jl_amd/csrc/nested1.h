@@ -14,7 +14,7 @@
 //              moments re-expanded up the path, one slot per cluster met
 //   translate  per cluster of the output side: z = sum_b F_b w_b; a source above
 //              the subtrees is summed from its slots (in slot order);
-//              coefficients c = A^T z
+//              coefficients c = A^T z (w and z with the node offsets, N1Mat)
 //   down       per subtree: coefficients down the path and the subtree by one
 //              wavefront, then one series per row, added onto y
 // The near field, y = beta*y + near, needs nothing of the chain and fills the
@@ -32,13 +32,13 @@
 // the tree. Single products four times over would form the entries four times;
 // the per-level passes read every level's U, V and F once for four.
 //
-// Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1235 -> 179 us
-// a product, matrix-free 233 -> 126 us, where the vector instructions alone
+// Measured (FP64, n = 2^20, leaf 256, rank 24, Cauchy): stored 1237 -> 178 us
+// a product, matrix-free 236 -> 128 us, where the vector instructions alone
 // take 62 us (near) and 17 us (far); transposed stored, n = 200003, leaf 80,
-// rank 20: 427 -> 59 us; Float32 hybrid, n = 500009, rank 10: 179 -> 59 us;
-// n = 1000: 27.0 -> 22.7 us. Four right-hand sides, stored log kernel, n = 2^17,
-// leaf 80, rank 20: 349 -> 141 us (the translation, whose log entries of F and
-// of the near field are read, takes 58 of them, the upward pass 50).
+// rank 20: 432 -> 62 us; Float32 hybrid, n = 500009, rank 10: 180 -> 63 us;
+// n = 1000: 25.9 -> 22.2 us. Four right-hand sides, stored log kernel, n = 2^17,
+// leaf 80, rank 20: 349 -> 151 us (the translation, whose log entries of F and
+// of the near field are read, takes 66 of them, the upward pass 57).
 #pragma once
 #include "kernels_impl.h"
 
@@ -131,7 +131,7 @@ __device__ __forceinline__ float rcp_refine(float d, float r) {
 // returns true, and the caller forms its sum again from where it began, term by
 // term (near_single). No branch between the columns, whose chains then run side
 // by side: a branch for each four took 45 us more at n = 2^20, one for each
-// eight 4. n = 2^20, leaf 256, rank 24: Cauchy 126 us, Coulomb 147 (common
+// eight 4. n = 2^20, leaf 256, rank 24: Cauchy 125 us, Coulomb 138 (common
 // denominator 126 and 140); Float32, leaf 64, rank 16: 96 us (90).
 // EXACT: term by term. The reciprocal's last step starts within 2^-48 (FP32
 // 2^-22) of it, so the result is a division's but for rare half-way cases
