@@ -321,7 +321,7 @@ __global__ __launch_bounds__(WG) void k_gen_F(DevPlanT<T> p) {
 
 // DevPlanT's rdel and cdel: how far the mapped nodes are off the exact ones in
 // their cluster's frame, by rounding (the differences from the center are exact
-// or nearly so)
+// or nearly so), times 2^12 (N1Mat)
 template <class T>
 __device__ __forceinline__ void node_offset_block(const DevPlanT<T> &p, const N1Frame *rf,
                                                   const N1Frame *cf) {
@@ -332,7 +332,8 @@ __device__ __forceinline__ void node_offset_block(const DevPlanT<T> &p, const N1
         const N1Frame f = row ? rf[c] : cf[c];
         const double t = (double)(row ? p.rnodes : p.cnodes)[at];
         (row ? p.rdel : p.cdel)[at] =
-            (T)(((t - f.cx) - f.cl) * f.cy - cospi((2 * (int)(at - c * p.r) + 1) / (2.0 * p.r)));
+            (T)(4096.0 * (((t - f.cx) - f.cl) * f.cy -
+                          cospi((2 * (int)(at - c * p.r) + 1) / (2.0 * p.r))));
     }
 }
 template <class T>

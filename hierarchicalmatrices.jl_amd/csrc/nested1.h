@@ -525,7 +525,9 @@ __device__ __forceinline__ void near_block(const N1Side &o, int blk, const T *pt
 // off the exact ones (2^-53 of the point against a deep cluster). The products'
 // polynomials go through the rounded nodes: their offsets d enter w and z to
 // first order, w = w0 - D^T (d w0) for w0 = A mu, and c = A^T (z - d (D z)), D
-// the differentiation matrix of the exact nodes. Without it, stored products at
+// the differentiation matrix of the exact nodes (held at 2^-12 and d at 2^12
+// times itself: D's entries reach r^2, and D z would leave the range before c
+// does). Without it, stored products at
 // n = 2^20 were 6.4e-15 off, and 1.3e-15 with U and V, which hold the basis at
 // the rounded nodes.
 template <class T, int RMAX>

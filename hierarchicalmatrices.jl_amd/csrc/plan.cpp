@@ -1268,7 +1268,8 @@ std::vector<T> nest_matrices(int r) {
 }  // extern "C++"
 
 // The differentiation matrix of the nodes t_k = cos((2k + 1) pi / (2r)): values
-// there -> the polynomial's derivatives there, D[k r + j] (the barycentric formula)
+// there -> the polynomial's derivatives there, D[k r + j] (the barycentric formula),
+// times 2^-12, as the node offsets are times 2^12
 static std::vector<double> node_derivative(int r) {
     std::vector<double> D((size_t)r * r, 0.0), sn(2 * r);  // sn[i] = sin(i pi / (2r))
     for (int i = 0; i < 2 * r; ++i) sn[i] = std::sin(i * M_PI / (2 * r));
@@ -1282,6 +1283,7 @@ static std::vector<double> node_derivative(int r) {
             D[(size_t)k * r + j] = ((k + j) & 1) ? -q : q;
             D[(size_t)k * r + k] -= D[(size_t)k * r + j];
         }
+    for (double &v : D) v *= 0x1p-12;
     return D;
 }
 

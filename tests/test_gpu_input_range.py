@@ -63,3 +63,25 @@ def test_scaled_inputs_units(cuda, transpose):
     for e in (-93, 70):
         got = (op @ (b * 2.0 ** e)).cpu().numpy()
         assert rel(got.astype(np.float64) * 2.0 ** -e, want) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("form", ["hybrid", "free"])
+@pytest.mark.parametrize("k", [1, 3, 8])
+@pytest.mark.parametrize("rank", [20, 32])
+def test_top_of_the_range(cuda, dtype, form, k, rank):
+    # results in the last binary order below the largest number, and nothing on the way beyond it:
+    # a power of two times the product at order one
+    n = 700
+    dt = np.float32 if dtype == "f32" else np.float64
+    i = np.arange(n, 0, -1, dtype=np.float64)
+    x, y = ((i - 0.25) / n).astype(dt), ((i - 0.75) / n).astype(dt)
+    H = hmx.KernelMatrix("cauchykernel", x, y, 1.0, 0.0, 1.0, 0.0, blocksize=40, rank=rank,
+                         hybrid=form == "hybrid", matrix_free=form == "free")
+    b = torch.from_numpy(np.abs(np.random.default_rng(3).standard_normal((n, k))).astype(dt)).to(cuda)
+    b = b[:, 0].contiguous() if k == 1 else b
+    for op in (H, H.T):
+        want = (op @ b).cpu().numpy().astype(np.float64)
+        e = int(np.floor(np.log2(float(np.finfo(dt).max)) - np.log2(np.abs(want).max())))
+        got = (op @ (b * 2.0 ** e)).cpu().numpy().astype(np.float64)
+        assert rel(got * 2.0 ** -e, want) <= (1e-5 if dtype == "f32" else 1e-12)
