@@ -826,7 +826,7 @@ __device__ __forceinline__ T nanT() {
 }
 
 // Translation: one wavefront per cluster of the output side whose sources all
-// lie in subtrees (a wavefront takes several in turn, the matrix rows kept);
+// lie in subtrees (a wavefront takes several in turn, the matrices in LDS);
 // the clusters with a source above them ("heavy", first in the target list)
 // take a workgroup, a source per wavefront. Lane (m, h) sums its row's half h
 // of the columns l. A cluster has at most about four sources; their node
@@ -838,7 +838,7 @@ struct TrLds {
     alignas(16) T sw[WPB][4][KB][RMAX], st[WPB][4][RMAX];
     alignas(16) T zr[WPB][KB][RMAX];
     // A^T and D of the output side (before them A and D^T, for sources above the
-    // subtrees): two matrices' rows in registers spilled
+    // subtrees); two matrices' rows in registers spilled
     T mat[RMAX * WAVE];
 };
 template <class T, int RMAX, bool TRANS, int SRC, int KID, int KB>
@@ -994,7 +994,7 @@ __device__ __forceinline__ void n1_translate_block(const DevPlanT<T> &p, const N
             T wl;
             if (R.nslots > 0) {
                 // lane half h sums the slots h, h + 2, ..., eight loads in flight
-                // at 32-bit offsets (sixteen at 64-bit ones spilled the matrix rows)
+                // at 32-bit offsets (sixteen at 64-bit ones spilled)
                 const T *ps = partial + (R.pbase * nq + kc) * r;
                 const unsigned ld = 2u * nq * r;
                 unsigned at = (unsigned)h * nq * r + mm;
